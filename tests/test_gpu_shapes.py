@@ -1,0 +1,71 @@
+"""The launch shapes the fused kernels choose for default tiles (frequency
+chunks, directions per wave, split advection) against the same substeps under
+an explicit tile, at the sizes where the choice changes; and the directional
+moments formed after a spectrum is set against those the advection leaves."""
+import numpy as np
+import pytest
+
+from umwm_amd import configs, hip
+
+pytestmark = pytest.mark.gpu
+
+# (mm, nm, om, pm): two directions a wave and the most chunks; one point block
+# with idle lanes; pm = 28 (no divisor 9 or 6); pm = 44 and 68 (one direction
+# segment, prime pm / 4); pm = 48; chunks that do not divide om; one chunk;
+# a spectrum wider than the split takes
+GRIDS = [(12, 11, 37, 36), (5, 4, 25, 24), (30, 21, 31, 28), (30, 20, 26, 44), (16, 14, 33, 68),
+         (60, 45, 41, 48), (105, 101, 29, 36), (190, 170, 25, 24), (14, 12, 25, 76)]
+
+
+def fresh(grid, precision):
+    mm, nm, om, pm = grid
+    wl = configs.regional_random(7, mm, nm, om, pm, dx=1e4, land_frac=0.1, shelf=True, wspd=11.0,
+                                 wdir=0.4)
+    d = hip.Domain(wl.params, wl.grid_input(), wl.forcing_input(0), precision=precision)
+    d.init_jonswap(wl.jonswap)
+    d.stokes_drift(True)
+    return d
+
+
+@pytest.mark.parametrize("precision", [8, 4])
+@pytest.mark.parametrize("grid", GRIDS)
+def test_default_shape_equals_explicit_tile(grid, precision):
+    # the same operations in the same order per bin; the rates of an explicit
+    # tile with an even D are paired, which regroups one sum: a few ulp
+    tol = 1e-13 if precision == 8 else 1e-5
+    pm = grid[3]
+    a, b = fresh(grid, precision), fresh(grid, precision)
+    try:
+        D = 9 if pm <= 72 else 18
+        b.set_tile(D, -(-pm // D), D, -(-pm // D), 2)
+        for n in (1, 3):
+            ra, rb = a.substeps(n), b.substeps(n)
+            assert ra[2] == rb[2] and abs(ra[1] - rb[1]) <= tol * abs(rb[1])
+        for name in ("e", "ustar", "physics_time_step"):
+            x, y = a.get(name), b.get(name)
+            assert np.linalg.norm(x - y) <= tol * np.linalg.norm(y), name
+        dts = min(float(a.get("physics_time_step").min()), a.scalar("dtamin"))
+        assert a.scalar("dts") == dts
+    finally:
+        a.close()
+        b.close()
+
+
+@pytest.mark.parametrize("precision", [8, 4])
+@pytest.mark.parametrize("grid", [(12, 11, 37, 36), (30, 21, 31, 28), (105, 101, 29, 24)])
+def test_moments_after_set_equal_advection(grid, precision):
+    """Setting the spectrum to itself makes the next substep form the moments
+    anew: bit for bit what the advection had left."""
+    a, b = fresh(grid, precision), fresh(grid, precision)
+    try:
+        for d in (a, b):
+            d.substeps(3)
+        e = b.get("e")
+        b.set("e", e)
+        a.substeps(2)
+        b.substeps(2)
+        for name in ("e", "ustar"):
+            assert np.array_equal(a.get(name), b.get(name)), name
+    finally:
+        a.close()
+        b.close()

@@ -16,9 +16,9 @@
 #include "rawio.hpp"
 #include "surrogate.hpp"
 
-// Scratch of umwm_hip_substeps_noalloc: the fused kernels' prefix moments
-// and stress partials ([om][ldi][4] each in the working precision), which
-// the other entry points keep in buffers allocated with the domain.  Every
+// Scratch of umwm_hip_substeps_noalloc: the fused kernels' FP64 prefix
+// moments ([om][ldi][4]) and y stress partials ([om][ldi]), which the other
+// entry points keep in buffers allocated with the domain.  Every
 // GPU the library runs on holds one copy until the process ends; in host
 // code the name is only a stand-in, and the device address comes from
 // hipGetSymbolAddress (umwm::noalloc_scratch).
@@ -269,7 +269,8 @@ int create_impl(const umwm_params& P, const umwm_grid_input* g, const umwm_forci
   // the fused kernels address one frequency of a spectrum (pm rows), of the
   // table block (FT_N rows) or of a per-point array with one buffer
   // descriptor each, and drop predicated stores with an offset of 2^31
-  const size_t maxrows = std::max<size_t>({(size_t)pm, (size_t)FT_N, 4});
+  const size_t maxrows = std::max<size_t>((size_t)pm, 12);
+  static_assert(FT_N <= 12, "rows of the table block");
   if (maxrows * ldi * std::max(sizeof(T), sizeof(double)) >= (size_t(1) << 31) ||
       (size_t)ldq * sizeof(double) >= (size_t(1) << 31)) {
     delete D;
@@ -343,11 +344,11 @@ int create_impl(const umwm_params& P, const umwm_grid_input* g, const umwm_forci
   // per-(frequency, point) table records for the fused FP64 kernels,
   // [o][ldi][FT_N] (the FP32 kernels derive them from k)
   if (sizeof(T) == 8) {
-    const std::vector<double>* ft[FT_PAD] = {&S.cp0, &S.logl2overz, &S.cothkd, &S.sbf, &S.k,
-                                             &S.cg0, &S.bf1r, &S.bf2r, &S.kdk};
+    const std::vector<double>* ft[FT_N] = {&S.cp0, &S.logl2overz, &S.cothkd, &S.sbf, &S.k,
+                                           &S.lsds, &S.bf1r, &S.bf2r};
     std::vector<double> blk((size_t)FT_N * nt, 0.0);
     for (size_t q = 0; q < nt; ++q)
-      for (int t = 0; t < FT_PAD; ++t) blk[q * FT_N + t] = (*ft[t])[q];
+      for (int t = 0; t < FT_N; ++t) blk[q * FT_N + t] = (*ft[t])[q];
     h.ftab = A.template alloc<T>((size_t)FT_N * nt);
     if (!h.ftab) {
       delete D;
@@ -438,14 +439,18 @@ int create_impl(const umwm_params& P, const umwm_grid_input* g, const umwm_forci
   // reduction scratch and scalars
   h.nblocks = (S.im + kLanes - 1) / kLanes;
   h.block0 = 0;
-  h.pfx = A.template alloc<T>(4 * nt);
-  h.spart = A.template alloc<T>(4 * nt);
+  h.mom = A.template alloc<T>(4 * nt);
+  h.sty = A.template alloc<T>(nt);
+  h.rkey = A.template alloc<unsigned long long>(ldi);
+  h.pfx = sizeof(T) == 8 ? A.template alloc<T>(4 * nt) : nullptr;
   h.sc = A.template alloc<Scalars>(1);
-  if (!h.sc || !h.pfx || !h.spart) {
+  if (!h.sc || !h.mom || !h.sty || !h.rkey || (sizeof(T) == 8 && !h.pfx)) {
     delete D;
     return fail(UMWM_ERR_NOMEM, "device allocation failed");
   }
-  if ((rc = dfill<T>(h.pfx, 4 * nt, T(0), s)) || (rc = dfill<T>(h.spart, 4 * nt, T(0), s))) {
+  if (h.pfx && (rc = dfill<T>(h.pfx, 4 * nt, T(0), s))) { delete D; return rc; }
+  if ((rc = dfill<T>(h.mom, 4 * nt, T(0), s)) || (rc = dfill<T>(h.sty, nt, T(0), s)) ||
+      (rc = dfill<unsigned long long>(h.rkey, ldi, 0ull, s))) {
     delete D;
     return rc;
   }
@@ -630,9 +635,20 @@ int surrogate_rates(DomainImpl<T>& D, hipStream_t s, bool& on) {
   return 0;
 }
 
+// The directional moments the sweeps read, after anything but a fused
+// substep wrote the spectrum.
+template <typename T>
+int ensure_moments(DomainImpl<T>& D, hipStream_t s) {
+  if (D.mom_valid) return 0;
+  if (int rc = launch_moments<T>(D.d, D.tasks, D.ntasks, D.h.om, s)) return rc;
+  D.mom_valid = true;
+  return 0;
+}
+
 template <typename T>
 int fused_substep(DomainImpl<T>& D, const DomainDev<T>* dd = nullptr) {
   int rc;
+  if ((rc = ensure_moments(D, D.stream))) return rc;
   if (any_forcing(D) && (rc = launch_forcinginterpolate(D, true))) return rc;
   bool sur = false;
   if (D.timing) UMWM_HIP_TRY(hipEventRecord(D.ev[5], D.stream));
@@ -674,7 +690,7 @@ uint64_t graph_signature(const DomainImpl<T>& D) {
   uint64_t h = 1469598103934665603ull;
   auto mix = [&](uint64_t v) { h = (h ^ v) * 1099511628211ull; };
   const Tile& t = D.tile;
-  for (int v : {t.D1, t.W1, t.D2, t.W2, t.NB, t.pmax}) mix((uint64_t)v);
+  for (int v : {t.D1, t.W1, t.D2, t.W2, t.NB, t.pmax, (int)t.chosen}) mix((uint64_t)v);
   mix(D.h.e_keep != nullptr);
   mix((uint64_t)(uintptr_t)D.sur);
   mix((uint64_t)(uintptr_t)D.h.sur_r);
@@ -691,6 +707,7 @@ uint64_t graph_signature(const DomainImpl<T>& D) {
 // the fused kernels, the same launches fused_substep makes.
 template <typename T>
 int graph_substep(DomainImpl<T>& D) {
+  if (int rc = ensure_moments(D, D.stream)) return rc;
   const uint64_t sig = graph_signature(D);
   if (!D.gexec || D.gsig != sig) {
     if (D.gexec) (void)hipGraphExecDestroy(D.gexec);
@@ -725,10 +742,11 @@ int substeps_impl(DomainImpl<T>& D, int n) {
   return read_scalars(D);
 }
 
-// umwm_hip_substeps_noalloc: the same substeps with the prefix moments and
-// stress partials in the device's shared scratch array.  Calls no
-// allocating routine: the record copy and the scratch address were set up
-// when the domain was created.
+// umwm_hip_substeps_noalloc: the same substeps with the prefix moments and y
+// stress partials in the device's shared scratch array (room for two records
+// of four values per frequency and point).
+// Calls no allocating routine: the record copy and the scratch address were
+// set up when the domain was created.
 template <typename T>
 int substeps_noalloc_impl(DomainImpl<T>& D, int n) {
   const size_t part = (size_t)4 * D.h.om * D.h.ldi * sizeof(T);
@@ -741,8 +759,8 @@ int substeps_noalloc_impl(DomainImpl<T>& D, int n) {
                                    " bytes of the shared array; use umwm_hip_substeps");
   if (!D.scr || !D.d_scr) return fail(UMWM_ERR_STATE, "substeps_noalloc: no scratch set up");
   D.h_scr = D.h;
-  D.h_scr.pfx = reinterpret_cast<T*>(D.scr);
-  D.h_scr.spart = reinterpret_cast<T*>(D.scr + off);
+  if (D.h.pfx) D.h_scr.pfx = reinterpret_cast<T*>(D.scr);
+  D.h_scr.sty = reinterpret_cast<T*>(D.scr + off);
   UMWM_HIP_TRY(hipMemcpyAsync(D.d_scr, &D.h_scr, sizeof(DomainDev<T>), hipMemcpyHostToDevice,
                               D.stream));
   // the array keeps the previous call's contents: start from zeros, as the
@@ -1001,6 +1019,7 @@ int set_field_impl(DomainImpl<T>& D, const std::string& name, const double* buf,
       return fail(UMWM_ERR_ARGUMENT, "field " + name + " is read-only");
   }
   if (name == "e") {
+    D.mom_valid = false;
     int rc = launch_hs_ice(D);
     if (rc) return rc;
     UMWM_HIP_TRY(hipStreamSynchronize(D.stream));
@@ -1179,6 +1198,7 @@ int umwm_hip_init_jonswap(umwm_domain* dom, const umwm_jonswap* js) {
   if (!js) return fail(UMWM_ERR_ARGUMENT, "null jonswap");
   return dispatch(dom, [&](auto& D) {
     if (js->fp <= 0 && !js->fp_from_wind) return fail(UMWM_ERR_ARGUMENT, "fp must be > 0");
+    D.mom_valid = false;
     int rc = launch_jonswap(D, *js);
     if (!rc) rc = launch_hs_ice(D);
     if (!rc) rc = sync_and_check(D);
@@ -1286,12 +1306,22 @@ OP_ENTRY(umwm_hip_sds_d12, launch_op_sds)
 OP_ENTRY(umwm_hip_snl_d12, launch_op_snl)
 OP_ENTRY(umwm_hip_s_ice, launch_op_sice)
 OP_ENTRY(umwm_hip_propagation, launch_op_propagation)
-OP_ENTRY(umwm_hip_update, launch_op_update)
+
+int umwm_hip_update(umwm_domain* dom) {
+  return dispatch(dom, [&](auto& D) {
+    int rc = ensure_ops(D);
+    D.mom_valid = false;
+    if (!rc) rc = launch_op_update(D);
+    if (!rc) rc = sync_and_check(D);
+    return rc;
+  });
+}
 
 int umwm_hip_source(umwm_domain* dom) {
   return dispatch(dom, [&](auto& D) {
     int rc = ensure_ops(D);
     D.ef_mirrors_e = false;
+    D.mom_valid = false;
     if (!rc) rc = launch_op_source(D);
     if (!rc) rc = sync_and_check(D);
     return rc;
@@ -1714,6 +1744,7 @@ int umwm_hip_set_tile(umwm_domain* dom, const int32_t tile[5]) {
     if (!tile_ok(t, D.S.pm))
       return fail(UMWM_ERR_ARGUMENT, "tile needs D1 in {6,9,18,36}, D2 in {3,6,9,12,18}, "
                                      "W in 1..8, D*W >= pm, NB in {2,4}");
+    t.chosen = true;
     D.tile = t;
     return 0;
   });
@@ -1884,6 +1915,8 @@ int batch_launch_substep(BatchImpl<T>& B, int first) {
 template <typename T>
 int batch_prepare(BatchImpl<T>& B, int use_graph) {
   int rc;
+  for (auto* D : B.doms)
+    if ((rc = ensure_moments(*D, B.stream))) return rc;
   bool any_first = false;
   for (auto* D : B.doms) any_first |= D->first;
   if (any_first) {
@@ -2041,6 +2074,7 @@ int umwm_hip_batch_set_tile(umwm_batch* b, const int32_t tile[5]) {
     for (auto* D : B->doms) pmmax = std::max(pmmax, D->S.pm);
     Tile t = tile_from(tile, pmmax);
     if (!tile_ok(t, pmmax)) return fail(UMWM_ERR_ARGUMENT, "tile does not cover pm");
+    t.chosen = true;
     B->tile = t;
     for (auto& g : B->groups) {
       Tile gt = t;  // same D and NB, waves for this class's pm

@@ -108,14 +108,17 @@ struct DomainDev {
   double *us1, *vs1;  // surface Stokes drift used by stress('atm')
   // fused-path copy of the (o, j) tables, [om][ldi][FT_N]: the FT_N values
   // of one (frequency, point) are contiguous, so a lane fetches them with a
-  // few 16-byte loads and a wave reads one contiguous span; the exclusive
-  // frequency prefix of the cos^2 directional convolution times dth/2,
-  // [om][ldi][4] (3 used, written by k_rates); the per-frequency stress /
-  // wave-height partial sums, [om][ldi][4] (3 used; summed over frequency
-  // in FP64 by k_stress)
+  // few 16-byte loads and a wave reads one contiguous span; the directional
+  // moments of e and the x stress partial, [om][ldi][4] (m0, mc, ms, x), and
+  // the y stress partial, [om][ldi], all written by k_advect; per point the
+  // bits of the largest rate while k_rates' workgroups of it collect it;
+  // FP64 only, dth/2 times the exclusive frequency prefix of the moments,
+  // [om][ldi][4] (3 used), from k_rates to k_integrate
   T* ftab;
   T* pfx;
-  T* spart;
+  T* mom;
+  T* sty;
+  unsigned long long* rkey;
   Scalars* sc;
   // learned surrogate of the FP32 path (null sur_r: none attached): the
   // network's spreading factor per bin as dm^2 - 1 in bfloat16 bits,
@@ -134,14 +137,15 @@ struct DomainDev {
 };
 
 // Slots of one (frequency, point) record of DomainDev::ftab: the tables the
-// sweep kernels cannot rebuild from k cheaply (k^4, 1/k^4, sdv, f k/g,
-// snl_arg and k^3 dk are formed from k, kdk, bf1r and bf2r on the fly).
-// The integrate kernel reads the first eight, the rates kernel all nine.
+// sweep kernels cannot rebuild from k cheaply (k^4, 1/k^4, sdv, f k/g and
+// snl_arg are formed on the fly).  FT_L is the natural logarithm of
+// 2 pi sds_fac f cothkd k^(4 sds_power), the factor of (e)^sds_power in sds:
+// with it the FP64 sweeps take no logarithm per frequency.
 enum FusedTable {
-  FT_CP0, FT_LOGL2, FT_COTH, FT_SBF, FT_K, FT_CG0, FT_B1, FT_B2, FT_KDK, FT_PAD, FT_N = 12
+  FT_CP0, FT_LOGL2, FT_COTH, FT_SBF, FT_K, FT_L, FT_B1, FT_B2, FT_N,
+  FT_KDK = FT_N, FT_CG0  // FP32 only (TabGen)
 };
-constexpr int kRatesSlots = 12;
-constexpr int kIntegrateSlots = 8;
+constexpr int kSweepSlots = 8;
 
 // Zero records after the pm records of DomainDev::dir4.  A sweep wave w of
 // W <= 8 reads slots w*ceil(pm/W) + q, q < DMAX <= 36, which stay below

@@ -22,6 +22,9 @@ struct Tile {
   // pm of the domains launched together (a batch launches each pm class
   // on its own); W D = pmax selects the sweeps' mask-free variants
   int pmax = 36;
+  // set by the caller: the sweeps run as set (else choose_shape in fused.hip
+  // may split them further where the grid is small)
+  bool chosen = false;
 };
 
 bool tile_supported(int D);
@@ -63,6 +66,9 @@ struct DomainBase {
   // the fused substep does not store E_s: after it, ef equals e (as after
   // the reference's e = ef) and reads of "ef" are served from e
   bool ef_mirrors_e = false;
+  // DomainDev::mom holds the moments of the current spectrum (the fused
+  // substep leaves them so; everything else that writes e clears this)
+  bool mom_valid = false;
   // rates, integrate, advect, stress, surrogate inference
   double ms[5] = {0, 0, 0, 0, 0};
   int64_t launches[5] = {0, 0, 0, 0, 0};
@@ -80,7 +86,7 @@ struct DomainImpl : DomainBase {
   int32_t* list0 = nullptr;
   // umwm_hip_substeps_noalloc: the device's shared scratch array (from
   // hipGetSymbolAddress at creation) and a second device copy of the domain
-  // record whose pfx and spart point into it, with its host image
+  // record whose pfx and sty point into it, with its host image
   unsigned char* scr = nullptr;
   DomainDev<T>* d_scr = nullptr;
   DomainDev<T> h_scr{};
@@ -145,6 +151,11 @@ template <typename T>
 int launch_fused(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, int omax,
                  int first, int rotation, Tile tile, bool keep, hipStream_t s, hipEvent_t* ev,
                  bool sur = false);
+
+// Directional moments of the current spectra (DomainDev::mom).
+template <typename T>
+int launch_moments(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, int omax,
+                   hipStream_t s);
 
 // The attached surrogate's spreading factors for the domain's current
 // spectrum and forcing (dm^2 - 1 into DomainDev::sur_r), on stream s.

@@ -5,9 +5,9 @@
 //                then a grid-wide min (atomic max on order-preserving keys,
 //                finished by the last block) -> dts, dta, sumt, dtr
 //                (src/umwm_physics.F90:22-58, src/umwm_advection.F90:329-365).
-//                Reads E^n once and writes the exclusive frequency prefix of
-//                the directional cos^2 convolution (3 values per frequency
-//                and point).
+//                Reads E^n up to each point block's last prognostic bin,
+//                and its directional moments, whose running sum over
+//                frequency is the sds prefix.
 //   k_integrate  sin + sds + snl + exponential integration + diagnostic
 //                tail (src/umwm_physics.F90:60-84); writes only
 //                E* = (E^n + E_s)/2 (es).
@@ -16,24 +16,25 @@
 //                (frequency, 64 sea points), with E_s recovered in place as
 //                2 E* - E^n from the e it overwrites (one spectrum stream
 //                fewer than storing E_s; the round-off is |E^n + E_s| ulp);
-//                also the per-frequency partial sums of
-//                stress_vector_integral (src/umwm_stress.F90:313-331).
+//                also the directional moments of the new spectrum and the
+//                per-frequency partial sums of stress_vector_integral
+//                (src/umwm_stress.F90:313-331).
 //   k_stress     per point: frequency sums, tail and the FP64 form/skin
 //                drag chain of stress('atm') (src/umwm_stress.F90:216-264).
 //
 // k_rates and k_integrate sweep frequencies in order inside the kernel: a
-// workgroup owns 64 consecutive sea points (one per lane, so every
-// spectrum/table access is a coalesced 64-wide stream of the
-// i-contiguous layout) and W waves, wave w owning directions
-// p = w*D .. w*D+D-1.  The prefix over frequency of
-// sum_pp e(o,pp) cos^2(th_pp - th_p) (src/umwm_source_functions.F90:92-97)
-// uses cos^2(a-b) = (1 + cos2a cos2b + sin2a sin2b)/2: three directional
-// moments per frequency, exchanged between waves through LDS when W > 1,
-// which turns the O(pm^2) convolution into O(pm).  Each sweep prefetches
-// the next frequency's spectrum (and, in FP32, its tables) while computing
-// the current one.  Launches whose waves all hold exactly DMAX directions
-// take a variant without per-slot masks, in which k_rates also pairs each
-// direction with its opposite.
+// wave owns 64 consecutive sea points (one per lane, so every spectrum and
+// table access is a coalesced 64-wide stream of the i-contiguous layout), D
+// directions and a chunk of consecutive frequencies (all of them on large
+// grids).  The prefix over frequency of sum_pp e(o,pp) cos^2(th_pp - th_p)
+// (src/umwm_source_functions.F90:92-97) uses cos^2(a-b) = (1 + cos2a cos2b +
+// sin2a sin2b)/2: three directional moments per frequency, which turns the
+// O(pm^2) convolution into O(pm).  k_advect leaves the moments of the
+// spectrum it writes, so the waves of a point need no exchange.  Each sweep
+// prefetches the next frequency's spectrum (and, in FP32, its tables) while
+// computing the current one.  Launches whose waves all hold exactly DMAX
+// directions take a variant without per-slot masks, and k_rates one that
+// pairs each direction with its opposite (caller-chosen tiles).
 //
 // snl(o) = bf1r(o) X(o+1) + bf2r(o) X(o+2) - snl_fac X(o), X = sds e
 // (src/umwm_source_functions.F90:165-171) is folded into the integration
@@ -51,10 +52,11 @@
 // one descriptor per frequency in scalar registers, 32-bit lane offsets
 // computed once per thread, directions reached with a scalar offset.  The
 // FP32 sweeps derive their (frequency, point) tables from k and the depth
-// (TabGen); FP64 reads a 12-value record per lane (three 16-byte loads).
-// The prefix moments and stress partial sums are 4-value records.
+// (TabGen); FP64 reads an 8-value record per lane (four 16-byte loads).
+// The directional moments with the x stress partial are a 4-value record.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "bufio.hpp"
@@ -200,9 +202,16 @@ __device__ __forceinline__ T rot_dir(T dcx, T dcy, T sth, T cth, T dvc, T duc, T
 // DomainDev::ftab.
 template <typename T>
 struct FreqTab {
-  T v[FT_N];
+  T v[FT_N + 2];  // the record, FT_KDK and FT_CG0
   __device__ __forceinline__ T operator[](int i) const { return v[i]; }
 };
+
+// Quotient of wave-uniform integers in a scalar register: the division runs
+// on the vector unit, and what is derived from its result (descriptors, loop
+// bounds) would stay there.
+__device__ __forceinline__ int uniform_div(int a, int b) {
+  return __builtin_amdgcn_readfirstlane(a / b);
+}
 
 // Descriptor of frequency o's slice of a [om][rows][ldi] spectrum (rows =
 // pm; a direction is then the scalar offset p * ldi * sizeof(T)) or of a
@@ -225,8 +234,7 @@ __device__ __forceinline__ void load_tab(const T* ftab, size_t ldi, int o, uint3
   bldn<T, N>(freq_rsrc(ftab, o, FT_N, ldi), vr, tmp);
 #pragma unroll
   for (int i = 0; i < N; ++i) r.v[i] = tmp[i];
-#pragma unroll
-  for (int i = N; i < FT_N; ++i) r.v[i] = T(0);
+  r.v[FT_KDK] = r.v[FT_CG0] = T(0);
 }
 
 // FP32 sweeps derive the (frequency, point) tables from k and the depth
@@ -247,7 +255,7 @@ struct TabGen {
   size_t ldi;
   uint32_t vj;
   int om;
-  float dep, sgr, sbf, sbp, s1, s2, l2z, lz;
+  float dep, sgr, sbf, sbp, s1, s2, l2z, lz, sp4, tpsf;
   float k0, k1, k2, kn;   // k(o), k(o+1), k(o+2), k(o+3) (loaded ahead)
   float kdk0, kdk1, kdk2;
 
@@ -266,7 +274,7 @@ struct TabGen {
     return k * cld(domr, o) * __builtin_amdgcn_rcpf(fabsf(cg));
   }
   template <typename D>
-  __device__ void init(const D& d, int j, uint32_t vj_) {
+  __device__ void init(const D& d, int j, uint32_t vj_, int o0) {
     kb = d.k;
     fr = d.f;
     domr = d.dom;
@@ -283,13 +291,15 @@ struct TabGen {
     s2 = float(d.snl_fac * d.bf2);
     lz = float(log(d.z));
     l2z = float(log(20.0 / d.z));
-    k0 = load_k(0);
-    k1 = load_k(1);
-    k2 = load_k(2);
-    kn = load_k(3);
-    kdk0 = kdk_of(k0, 0);
-    kdk1 = kdk_of(k1, 1);
-    kdk2 = kdk_of(k2, 2);
+    sp4 = float(4 * d.sds_power);
+    tpsf = float(d.twopisds_fac);
+    k0 = load_k(o0);
+    k1 = load_k(o0 + 1);
+    k2 = load_k(o0 + 2);
+    kn = load_k(o0 + 3);
+    kdk0 = kdk_of(k0, o0);
+    kdk1 = kdk_of(k1, o0 + 1);
+    kdk2 = kdk_of(k2, o0 + 2);
   }
   // slots of frequency o (the FreqTab layout of the record tables)
   __device__ void table(int o, FreqTab<float>& r) const {
@@ -306,7 +316,9 @@ struct TabGen {
     const float l2 = 0.5f * cp * __builtin_amdgcn_rcpf(fo);
     r.v[FT_CP0] = cp;
     r.v[FT_LOGL2] = l2 > 20.f ? l2z : 0.6931471805599453f * __builtin_amdgcn_logf(l2) - lz;
-    r.v[FT_COTH] = (1.f + w) * __builtin_amdgcn_rcpf(1.f - w);
+    const float coth = (1.f + w) * __builtin_amdgcn_rcpf(1.f - w);
+    r.v[FT_COTH] = coth;
+    r.v[FT_L] = sp4 * __builtin_amdgcn_logf(k) + __builtin_amdgcn_logf(tpsf * fo * coth);
     r.v[FT_SBF] = sbf * k * isinh2 + sbp * k * __builtin_amdgcn_rcpf(ch * ch);
     r.v[FT_K] = k;
     r.v[FT_CG0] = cp * (0.5f + k * dep * isinh2 + sk2 * __builtin_amdgcn_rcpf(1.f + sk2));
@@ -315,7 +327,6 @@ struct TabGen {
     r.v[FT_B1] = bo ? s1 * kdk1 * ik : 0.f;
     r.v[FT_B2] = bo ? s2 * kdk2 * ik : 0.f;
     r.v[FT_KDK] = kdk0;
-    for (int q = FT_PAD; q < FT_N; ++q) r.v[q] = 0.f;
   }
   // moves to frequency o+1; `next` is k(o+4), loaded during iteration o
   __device__ void advance(int o, float next) {
@@ -402,12 +413,87 @@ __device__ __forceinline__ T sin_m(const SinFreq<T>& q, T y, T m) {
 }
 
 // ---------------------------------------------------------------------
+// Directional moments of E^n, the raw material of the sds prefix: per
+// (frequency, point) the sums over the directions of e, e cos 2th and
+// e sin 2th, [om][ldi][4] (the fourth value is the x stress partial).
+// k_advect forms them from the spectrum it writes, so the sweeps need no
+// exchange between the waves of a point and may be split over directions
+// and frequencies freely; k_moments forms them after anything else wrote
+// the spectrum.  The order of the sums does not depend on the launch: four
+// consecutive directions in the working precision, these quads in FP64 over
+// the pm / kSegs directions of a segment, the segments in FP64.
+// ---------------------------------------------------------------------
+// Segments of the directional sums: the largest divisor of pm / 4 up to 8.
+__host__ __device__ inline int dir_segments(int pm) {
+  int n = 8;
+  while ((pm / 4) % n) --n;
+  return n;
+}
+
+template <typename T>
+struct Mom {
+  T m0, mc, ms;
+};
+
+template <typename T>
+__device__ __forceinline__ Mom<T> load_mom(const T* mom, size_t ldi, int o, int j) {
+  const rsrc_t pf = freq_rsrc(mom, o, 4, ldi);
+  Mom<T> r;
+  if constexpr (sizeof(T) == 4) {
+    const auto v = bld16<T>(pf, (uint32_t)j * 16u);
+    r.m0 = v[0];
+    r.mc = v[1];
+    r.ms = v[2];
+  } else {
+    const auto v = bld16<T>(pf, (uint32_t)j * 32u);
+    r.m0 = v[0];
+    r.mc = v[1];
+    r.ms = bld<T>(pf, (uint32_t)j * 32u + 16u);
+  }
+  return r;
+}
+
+// Running prefix of the moments over frequency, sum_{o' < o} k^3 dk m(o'),
+// in FP64 (src/umwm_source_functions.F90:92-97).
+struct Prefix {
+  double a0 = 0, ac = 0, as = 0;
+  template <typename T>
+  __device__ __forceinline__ void add(T k3dk, const Mom<T>& m) {
+    const double k3 = k3dk;
+    a0 += k3 * (double)m.m0;
+    ac += k3 * (double)m.mc;
+    as += k3 * (double)m.ms;
+  }
+};
+
+// In FP64 k_rates stores dth/2 times the prefix ([om][ldi][4], 3 used) for
+// k_integrate, which has no registers left for the running sums (keeping
+// them there spilled: 155 -> 350 us on 2,852 points); in FP32 k_integrate
+// forms its own and the 8 values of traffic per (frequency, point) are saved.
+template <typename T>
+constexpr bool kStoredPrefix = sizeof(T) == 8;
+
+// The prefix at frequency o0 of a sweep that starts there.
+template <typename T>
+__device__ __forceinline__ Prefix prefix_at(const DomainDev<T>& d, int o0, int j, uint32_t vj) {
+  Prefix P;
+#pragma unroll 4
+  for (int o = 0; o < o0; ++o)
+    P.add(bld<T>(row_rsrc(d.k3dk, o, (size_t)d.ldi), vj), load_mom(d.mom, d.ldi, o, j));
+  return P;
+}
+
+// ---------------------------------------------------------------------
 // k_rates
 // ---------------------------------------------------------------------
-template <typename T, int DMAX, bool FULL, bool SUR>
+// Wave `slot` of a point block (blockIdx.y W + w) takes directions p0 ..
+// p0 + DMAX - 1 of direction group slot % ng and the frequencies of chunk
+// slot / ng; slots past ng * chunks are idle.  SUR launches keep all of a
+// point's waves in one workgroup (one chunk, gridDim.y = 1).
+template <typename T, int DMAX, bool FULL, bool PAIR, bool SUR>
 __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ doms,
                                                const BlockTask* __restrict__ tasks, int first,
-                                               int rot_all) {
+                                               int rot_all, int ng, int chunks) {
   extern __shared__ double smem[];
   stage_fm64<T>();
   const BlockTask tk = tasks[blockIdx.x];
@@ -427,9 +513,12 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
   [[maybe_unused]] const int nsub0 = sc->nsub;
   const int pm = d.pm, om = d.om;
   const size_t ldi = d.ldi, ldq = d.ldq;
-  const int D = FULL ? DMAX : (pm + W - 1) / W, p0 = w * D;
-  // directions of this wave (uniform); FULL launches have W * DMAX = pm
+  const int slot = (int)blockIdx.y * W + w, chunk = uniform_div(slot, ng), grp = slot - chunk * ng;
+  const int D = FULL ? DMAX : uniform_div(pm + ng - 1, ng), p0 = grp * D;
+  // directions of this wave (uniform); FULL launches have ng * DMAX = pm
   const int nd = FULL ? DMAX : max(0, min(D, pm - p0));
+  const int oper = uniform_div(om + chunks - 1, chunks);
+  const int o0 = chunk * oper, o1 = min(om, o0 + oper);  // empty for an idle slot
   const uint32_t vj = (uint32_t)j * (uint32_t)sizeof(T);
   const uint32_t vr = (uint32_t)j * (uint32_t)(FT_N * sizeof(T));
   const uint32_t rb = (uint32_t)ldi * (uint32_t)sizeof(T);  // bytes of one direction row
@@ -439,16 +528,22 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
   // opaque to the compiler, which would otherwise reload these pointers
   // from the domain record after every store.
   const T* const eb = d.e;
-  T* const pfxb = d.pfx;
+  const T* const momb = d.mom;
+  const T* const k3b = d.k3dk;
+  [[maybe_unused]] T* const pfxb = d.pfx;
   const T* const ftab = d.ftab;
   const T* const fr = d.f;
   const T* const dir4 = d.dir4;
   double pts = INFINITY, rotmax = -INFINITY;
 
   if (active) {
-    const PointState<T> s = point_fresh(d, j, valid && w == 0);
+    const PointState<T> s = point_fresh(d, j, valid && slot == 0);
     const int oc = s.oc;
-    if (rotation && valid && w == 0) pstore(d.oc_rot, ldi, j, (int32_t)oc);
+    const int ocmax = wave_max_i32(valid ? oc : -1);
+    const bool anyice = __any(valid && s.ice != T(0));
+    // cg0, which the FP64 record leaves out: only ice attenuation needs it
+    auto ice_cg0 = [&](int o) { return bld<T>(row_rsrc(d.cg0, o, ldi), vj); };
+    if (rotation && valid && slot == 0) pstore(d.oc_rot, ldi, j, (int32_t)oc);
     uint32_t vie = 0, viw = 0, vin = 0, vis = 0;
     T dvc = 0, duc = 0, odx = 0, ody = 0;
     if (rotation) {
@@ -462,7 +557,7 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
       ody = pload(d.oneovdy, ldi, j);
     }
     const T sin_diss1 = T(d.sin_fac * d.fieldscale1), fs2 = T(d.fieldscale2);
-    const T tpsf = T(d.twopisds_fac), spow = T(d.sds_power), mssf = T(d.mss_fac);
+    const T spow = T(d.sds_power), mssf = T(d.mss_fac);
     const T nu4 = T(4 * d.nu_water), ig = T(1 / d.g);
     const double hdth = 0.5 * d.dth;
     // Slots q >= nd are computed but never used: their spectrum loads go
@@ -471,15 +566,15 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
     // maximum.  With no per-slot branch the compiler can interleave the
     // directions.
     const rsrc_t rz = make_rsrc(eb, 0u);
-    // FULL launches with an even DMAX pair each direction p with p + pm/2
+    // PAIR launches (FULL with an even DMAX) pair each direction p with p + pm/2
     // (theta + pi): cos and sin change sign while cos 2theta and sin 2theta
     // do not, so a pair shares its direction record, the mss factor and one
     // update of the moments.  Wave w then holds pairs w DMAX/2 + h in slots
     // h and h + DMAX/2, which also halves the direction records the loop
     // keeps in scalar registers.
-    constexpr bool PAIR = FULL && DMAX % 2 == 0;
+    static_assert(!PAIR || (FULL && DMAX % 2 == 0), "paired sweeps are mask-free and even");
     constexpr int H = DMAX / 2;
-    const int ph = w * H, half = pm / 2;
+    const int ph = grp * H, half = pm / 2;
     auto dirp = [&](int q) { return PAIR ? (q < H ? ph + q : ph + q - H + half) : p0 + q; };
     // overrun factor of slot q: fieldscale2 where the wind overruns the
     // direction, else 1; the paired loop reads it as bit q of mb (one
@@ -526,24 +621,29 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
     }
     T rmax = 0;
     [[maybe_unused]] T rmax_s = 0, neg = 0, tot = 0, anum = 0, aden = 0;
-    // One sweep over frequencies: `ds` also evaluates the network's
-    // dissipation; `pass0` stores the prefix moments and the rotation
-    // maximum.
-    auto sweep = [&](bool ds, bool pass0) {
-    double A0 = 0, AC = 0, AS = 0;
+    // One sweep over this wave's frequencies: `ds` also evaluates the
+    // network's dissipation.
+    auto sweep = [&](bool ds) {
+    // the rates count up to the cut-off: past the last prognostic bin of the
+    // wave's points there is nothing to evaluate (16 of 37 frequencies at
+    // 15 m/s) unless the network's share of the energy is being measured
+    const int omain = ds ? o1 : min(o1, ocmax + 1);
+    Prefix P = prefix_at(d, o0, j, vj);
     T ec[DMAX];
     // the network's dm^2 - 1 of this and the next frequency as raw bf16
     // bits; the direction's row offset joins the lane offset (a vector add)
     // rather than holding DMAX more scalar registers
     [[maybe_unused]] uint32_t rc[DMAX];
     FreqTab<T> tc;
+    Mom<T> mo = load_mom(momb, ldi, o0, j);
+    T k3 = bld<T>(row_rsrc(k3b, o0, ldi), vj);
     {
-      const rsrc_t ep = freq_rsrc(eb, 0, pm, ldi);
+      const rsrc_t ep = freq_rsrc(eb, o0, pm, ldi);
 #pragma unroll
       for (int q = 0; q < DMAX; ++q) ec[q] = bld<T>(FULL || q < nd ? ep : rz, vj, dirp(q) * rb);
       if constexpr (SUR) {
         if (ds) {
-          const rsrc_t rp = sur_rsrc(rsur, 0, pm, ldi);
+          const rsrc_t rp = sur_rsrc(rsur, o0, pm, ldi);
 #pragma unroll
           for (int q = 0; q < DMAX; ++q) rc[q] = bld_u16(FULL || q < nd ? rp : rz, vj2 + dirp(q) * rb2);
         }
@@ -552,10 +652,19 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
     // FP32 derives the tables from k (TabGen); FP64 loads the record
     constexpr bool kDerive = sizeof(T) == 4;
     TabGen tg;
-    if constexpr (kDerive) tg.init(d, j, vj);
-    for (int o = 0; o < om; ++o) {
+    if constexpr (kDerive) tg.init(d, j, vj, o0);
+    auto store_prefix = [&](int o, T pa0, T pac, T pas) {
+      if constexpr (kStoredPrefix<T>) {
+        if (valid && grp == 0) {
+          const rsrc_t pf = freq_rsrc(pfxb, o, 4, ldi);
+          bst16(pf, (uint32_t)j * 32u, typename Vec16<T>::type{pa0, pac});
+          bst(pf, (uint32_t)j * 32u + 16u, pas);
+        }
+      }
+    };
+    for (int o = o0; o < omain; ++o) {
       // issue the next frequency's loads before computing this one
-      const int on = o + 1 < om ? o + 1 : o;
+      const int on = o + 1 < omain ? o + 1 : o;
       T en[DMAX];
       const rsrc_t epn = freq_rsrc(eb, on, pm, ldi);
 #pragma unroll
@@ -568,37 +677,28 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
           for (int q = 0; q < DMAX; ++q) rn[q] = bld_u16(FULL || q < nd ? rp : rz, vj2 + dirp(q) * rb2);
         }
       }
+      const Mom<T> mn = load_mom(momb, ldi, on, j);
+      const T k3n = bld<T>(row_rsrc(k3b, on, ldi), vj);
       float knext = 0.f;
       if constexpr (kDerive) {
         knext = tg.load_k(o + 4);
         tg.table(o, tc);
       } else {
-        load_tab<kRatesSlots>(ftab, ldi, o, vr, tc);
+        load_tab<kSweepSlots>(ftab, ldi, o, vr, tc);
       }
 
-      const T k = tc[FT_K], k2 = k * k, fo = cld(fr, o);
-      const T sdt = s.csdt * k;
-      const T sice = T(2) * tc[FT_CG0] * s.ice;
-      const T crest = tc[FT_SBF] + sdt + nu4 * k2 - sice;  // sbf + sdt + sdv - sice
+      const T k = tc[FT_K], fo = cld(fr, o);
+      T crest = tc[FT_SBF] + s.csdt * k + nu4 * (k * k);  // sbf + sdt + sdv - sice
+      if (anyice) crest -= T(2) * s.ice * ice_cg0(o);
       const SinFreq<T> sf = sin_freq(s, tc[FT_LOGL2], tc[FT_CP0], fo * k * ig, sin_diss1, fs2);
-      const T pa0 = T(hdth * A0), pac = T(hdth * AC), pas = T(hdth * AS);
-      if (pass0 && valid && w == 0) {
-        if constexpr (sizeof(T) == 4) {
-          bst16(freq_rsrc(pfxb, o, 4, ldi), (uint32_t)j * 16u,
-                typename Vec16<T>::type{pa0, pac, pas, T(0)});
-        } else {
-          const rsrc_t pf = freq_rsrc(pfxb, o, 4, ldi);
-          bst16(pf, (uint32_t)j * 32u, typename Vec16<T>::type{pa0, pac});
-          bst16(pf, (uint32_t)j * 32u + 16u, typename Vec16<T>::type{pas, T(0)});
-        }
-      }
+      const T pa0 = T(hdth * P.a0), pac = T(hdth * P.ac), pas = T(hdth * P.as);
+      store_prefix(o, pa0, pac, pas);
       // sds (after cothkd) = cf coth dm^2 (e k4)^p = dm^2 ex(p lg e + Lk)
-      const T cfo = tpsf * fo * tc[FT_COTH];
-      const T Lk = T(4) * spow * Tr<T>::lg_nn(k) + Tr<T>::lg_nn(cfo);  // lg(k^4) = 4 lg k
+      const T Lk = tc[FT_L];  // lg(cf coth k^(4 p))
       const T cs = T(1) - (tc[FT_B1] + tc[FT_B2]);                // snl_arg
       const T q0 = T(1) + mssf * pa0, qc = mssf * pac, qs = mssf * pas;
-      [[maybe_unused]] const T sbfv = tc[FT_SBF], kdkv = tc[FT_KDK];
-      T m0 = 0, mc = 0, ms = 0, rq = 0;
+      [[maybe_unused]] const T kdkv = tc[FT_KDK];
+      T rq = 0;
       [[maybe_unused]] T rqs = 0;
       // sds = dm^2 sat with sat = ex(p lg |e| + Lk) = cf coth (e k4)^p: of
       // |e|, so that a bin emptied by round-off to about -1e-30 gives a
@@ -653,10 +753,6 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
               sur_bin(ssb, bf16_bits_to_f(rc[h + H]), eb2, satb, spb, true);
             }
           }
-          const T ep2 = ea + eb2;
-          m0 += ep2;
-          mc = fma(ep2, c2, mc);
-          ms = fma(ep2, s2, ms);
         }
       } else {
 #pragma unroll
@@ -674,49 +770,28 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
           if constexpr (SUR) {
             if (ds) sur_bin(ss, bf16_bits_to_f(rc[q]), e, sat, sp, FULL || q < nd);
           }
-          m0 += e;
-          mc = fma(e, c2, mc);
-          ms = fma(e, s2, ms);
         }
       }
       if (o <= oc) {  // rates of prognostic bins only
         rmax = fmax(rmax, rq);
         if constexpr (SUR) rmax_s = fmax(rmax_s, rqs);
       }
-      if (rotation && pass0) {
+      if (rotation) {
         // rotation tendency of the first substep (src/umwm_advection.F90:329-349)
         const rsrc_t cpr = row_rsrc(d.cp0, o, ldi);
         const T dcx = bld<T>(cpr, vie) - bld<T>(cpr, viw);
         const T dcy = bld<T>(cpr, vin) - bld<T>(cpr, vis);
-        double rm = 0;  // bins above oc hold 0 and join the signed max
         if (o <= oc) {
-          rm = -INFINITY;
           for (int q = 0; q < nd; ++q) {
             const int p = dirp(q);
-            rm = fmax(rm, (double)rot_dir(dcx, dcy, cld(d.sth, p), cld(d.cth, p), dvc, duc, odx,
-                                          ody));
+            rotmax = fmax(rotmax, (double)rot_dir(dcx, dcy, cld(d.sth, p), cld(d.cth, p), dvc, duc,
+                                                  odx, ody));
           }
         }
-        if (nd > 0) rotmax = fmax(rotmax, rm);
       }
-      double s0 = m0, s2c = mc, s2s = ms;
-      if (W > 1) {
-        double* b = smem + (size_t)(o & 1) * 3 * W * 64;
-        b[(0 * W + w) * 64 + lane] = s0;
-        b[(1 * W + w) * 64 + lane] = s2c;
-        b[(2 * W + w) * 64 + lane] = s2s;
-        __syncthreads();
-        s0 = s2c = s2s = 0;
-        for (int q = 0; q < W; ++q) {
-          s0 += b[(0 * W + q) * 64 + lane];
-          s2c += b[(1 * W + q) * 64 + lane];
-          s2s += b[(2 * W + q) * 64 + lane];
-        }
-      }
-      const double k3 = k2 * tc[FT_KDK];  // k^3 dk
-      A0 += k3 * s0;
-      AC += k3 * s2c;
-      AS += k3 * s2s;
+      P.add(k3, mo);
+      mo = mn;
+      k3 = k3n;
 #pragma unroll
       for (int q = 0; q < DMAX; ++q) ec[q] = en[q];
       if constexpr (SUR) {
@@ -727,8 +802,19 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
       }
       if constexpr (kDerive) tg.advance(o, knext);
     }
+    if constexpr (kStoredPrefix<T>) {
+      // the prefix of the diagnostic tail's bins, for k_integrate
+      if (grp == 0) {
+        for (int o = max(o0, omain); o < o1; ++o) {
+          store_prefix(o, T(hdth * P.a0), T(hdth * P.ac), T(hdth * P.as));
+          P.add(bld<T>(row_rsrc(k3b, o, ldi), vj), load_mom(momb, ldi, o, j));
+        }
+      }
+    }
     };
-    sweep(do_sur, true);
+    if (o0 < o1) sweep(do_sur);
+    // bins above the cut-off hold a rotation of 0 and join the signed max
+    if (rotation && nd > 0) rotmax = fmax(rotmax, 0.0);
     // the surrogate's verdict per lane (the same in every wave)
     [[maybe_unused]] bool use = false;
     if constexpr (SUR) {
@@ -795,7 +881,14 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
       double mx = 0;
       for (int q = 0; q < W; ++q) mx = fmax(mx, smem[q * 64 + lane]);
       pts = d.explim / mx;
-      if (valid) pstore(d.pts, ldi, j, pts);
+      if (valid) {
+        // a point whose waves span several workgroups collects its maximum
+        // (rates are >= 0, so their bits order as they do); k_stress divides
+        if (gridDim.y > 1)
+          atomicMax(d.rkey + j, (unsigned long long)__double_as_longlong(mx));
+        else
+          pstore(d.pts, ldi, j, pts);
+      }
       if (!valid) pts = INFINITY;
     }
     if (!valid) rotmax = -INFINITY;
@@ -829,7 +922,7 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
     // both atomics complete (s_waitcnt 0) before the arrival count
     __builtin_amdgcn_s_waitcnt(0);
     const unsigned tkt = atomicAdd(&sc->counter, 1u);
-    is_last = (tkt == (unsigned)d.nblocks - 1);
+    is_last = (tkt == (unsigned)d.nblocks * gridDim.y - 1);
   }
   __syncthreads();
   if (!is_last) return;
@@ -873,44 +966,29 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
 // ---------------------------------------------------------------------
 // k_integrate
 // ---------------------------------------------------------------------
-template <typename T>
-struct Prefix {
-  T a0, ac, as;
-};
-
-template <typename T>
-__device__ __forceinline__ Prefix<T> load_prefix(const T* pfx, size_t ldi, int o, int j) {
-  const rsrc_t pf = freq_rsrc(pfx, o, 4, ldi);
-  Prefix<T> r;
-  if constexpr (sizeof(T) == 4) {
-    const auto v = bld16<T>(pf, (uint32_t)j * 16u);
-    r.a0 = v[0];
-    r.ac = v[1];
-    r.as = v[2];
-  } else {
-    const auto v = bld16<T>(pf, (uint32_t)j * 32u);
-    r.a0 = v[0];
-    r.ac = v[1];
-    r.as = bld<T>(pf, (uint32_t)j * 32u + 16u);
-  }
-  return r;
-}
-
 template <typename T, int DMAX, bool FULL, bool SUR>
 __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restrict__ doms,
-                                                   const BlockTask* __restrict__ tasks) {
+                                                   const BlockTask* __restrict__ tasks, int ng,
+                                                   int chunks) {
   const BlockTask tk = tasks[blockIdx.x];
   const DomainDev<T>& d = doms[tk.dom];
   const Scalars* sc = d.sc;
   if (!sc->active) return;  // uniform over the block
   stage_fm64<T>();
-  const int W = blockDim.x >> 6, w = wave_id();
   const int j = tk.i0 + (threadIdx.x & 63);
   const bool valid = j < d.im;
   const int pm = d.pm, om = d.om;
   const size_t ldi = d.ldi;
-  const int D = FULL ? DMAX : (pm + W - 1) / W, p0 = w * D;
+  const int slot = (int)blockIdx.y * (int)(blockDim.x >> 6) + wave_id();
+  const int chunk = uniform_div(slot, ng), grp = slot - chunk * ng;
+  const int D = FULL ? DMAX : uniform_div(pm + ng - 1, ng), p0 = grp * D;
   const int nd = FULL ? DMAX : max(0, min(D, pm - p0));
+  // This wave completes bins o0 .. o1 - 1.  It sweeps two frequencies past
+  // them for the snl gains their energy feeds down, of which it takes only
+  // X; the wave of the next chunk integrates those bins.
+  const int oper = uniform_div(om + chunks - 1, chunks);
+  const int o0 = chunk * oper, o1 = min(om, o0 + oper);
+  if (o0 >= o1) return;  // an idle slot; no barrier follows
   const T dts = T(sc->dts);
   const T dtx = dts * Tr<T>::kExpScale;  // dts in the exponential's base
   const uint32_t vj = (uint32_t)j * (uint32_t)sizeof(T);
@@ -920,13 +998,16 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
   const T* const eb = d.e;
   T* const esb = d.es;
   const T* const ftab = d.ftab;
-  const T* const pfxb = d.pfx;
+  [[maybe_unused]] const T* const momb = d.mom;
+  [[maybe_unused]] const T* const k3b = d.k3dk;
+  [[maybe_unused]] const T* const pfxb = d.pfx;
   const T* const fr = d.f;
 
   const PointState<T> s = point_stored(d, j);
   const int oc = s.oc;
+  const bool anyice = __any(valid && s.ice != T(0));
   const T sin_diss1 = T(d.sin_fac * d.fieldscale1), fs2 = T(d.fieldscale2);
-  const T tpsf = T(d.twopisds_fac), spow = T(d.sds_power), ipow = T(d.inv_sds_power);
+  const T spow = T(d.sds_power), ipow = T(d.inv_sds_power);
   const T mssf = T(d.mss_fac), dsnl = dts * T(d.snl_fac);
   const T nu4 = T(4 * d.nu_water), ig = T(1 / d.g);
   // direction constants of this wave, loaded once.  Slots q >= nd are
@@ -935,15 +1016,17 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
   // direction loop has no per-slot branch and the compiler can interleave
   // the directions.
   const rsrc_t rz = make_rsrc(eb, 0u);
-  T mq[DMAX], ctq[DMAX], stq[DMAX];
+  // wind overrunning a direction (fieldscale2, see sin_m) as bits of mb, and
+  // the direction records re-read per frequency: both in registers cost
+  // k_integrate a wave per SIMD in FP64
+  uint32_t mb = 0;
 #pragma unroll
   for (int q = 0; q < DMAX; ++q) {
     T ct, st, c2, s2;
     cld4(d.dir4, p0 + q, ct, st, c2, s2);
-    mq[q] = s.cw * ct + s.sw * st > T(0) ? fs2 : T(1);
-    ctq[q] = ct;
-    stq[q] = st;
+    if (s.cw * ct + s.sw * st > T(0)) mb |= 1u << q;
   }
+  const T* const dir4 = d.dir4;
   // per direction, the partial E* = (E^n + partial E_s) / 2 of the two
   // previous frequencies, still waiting for their snl gains
   T H1[DMAX], H2[DMAX];
@@ -967,28 +1050,33 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
   T ec[DMAX];
   [[maybe_unused]] uint32_t rc[DMAX];  // raw bf16 bits of dm^2 - 1 (see k_rates)
   {
-    const rsrc_t ep = freq_rsrc(eb, 0, pm, ldi);
+    const rsrc_t ep = freq_rsrc(eb, o0, pm, ldi);
 #pragma unroll
     for (int q = 0; q < DMAX; ++q) ec[q] = bld<T>(FULL || q < nd ? ep : rz, vj, (p0 + q) * rb);
     if constexpr (SUR) {
       if (do_sur) {
-        const rsrc_t rp = sur_rsrc(rsur, 0, pm, ldi);
+        const rsrc_t rp = sur_rsrc(rsur, o0, pm, ldi);
 #pragma unroll
         for (int q = 0; q < DMAX; ++q) rc[q] = bld_u16(FULL || q < nd ? rp : rz, vj2 + (p0 + q) * rb2);
       }
     }
   }
   FreqTab<T> tc;
-  Prefix<T> pc{};
-  // FP32 derives the tables from k (TabGen) and prefetches the prefix;
-  // FP64 loads both when needed (as in k_rates)
+  // FP32 derives the tables from k (TabGen); FP64 loads them when needed
+  // (as in k_rates)
   constexpr bool kDerive = sizeof(T) == 4;
   TabGen tg;
-  if constexpr (kDerive) {
-    tg.init(d, j, vj);
-    pc = load_prefix(pfxb, ldi, 0, j);
+  if constexpr (kDerive) tg.init(d, j, vj, o0);
+  [[maybe_unused]] Prefix P;
+  [[maybe_unused]] Mom<T> mo{};
+  [[maybe_unused]] T k3 = 0;
+  if constexpr (!kStoredPrefix<T>) {
+    P = prefix_at(d, o0, j, vj);
+    mo = load_mom(momb, ldi, o0, j);
+    k3 = bld<T>(row_rsrc(k3b, o0, ldi), vj);
   }
-  for (int o = 0; o < om; ++o) {
+  const int oend = min(om, o1 + 2);
+  for (int o = o0; o < oend; ++o) {
     const int on = o + 1 < om ? o + 1 : o;
     T en[DMAX];
     const rsrc_t epn = freq_rsrc(eb, on, pm, ldi);
@@ -1002,43 +1090,53 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
         for (int q = 0; q < DMAX; ++q) rn[q] = bld_u16(FULL || q < nd ? rp : rz, vj2 + (p0 + q) * rb2);
       }
     }
-    Prefix<T> pn{};
+    [[maybe_unused]] Mom<T> mn{};
+    [[maybe_unused]] T k3n = 0;
     float knext = 0.f;
+    T pa0, pac, pas;  // dth/2 times the prefix moments
     if constexpr (kDerive) {
       knext = tg.load_k(o + 4);
-      pn = load_prefix(pfxb, ldi, on, j);
       tg.table(o, tc);
     } else {
-      load_tab<kIntegrateSlots>(ftab, ldi, o, vr, tc);
-      pc = load_prefix(pfxb, ldi, o, j);
+      load_tab<kSweepSlots>(ftab, ldi, o, vr, tc);
+    }
+    if constexpr (kStoredPrefix<T>) {
+      const Mom<T> pc = load_mom(pfxb, ldi, o, j);
+      pa0 = pc.m0;
+      pac = pc.mc;
+      pas = pc.ms;
+    } else {
+      mn = load_mom(momb, ldi, on, j);
+      k3n = bld<T>(row_rsrc(k3b, on, ldi), vj);
+      const double hdth = 0.5 * d.dth;
+      pa0 = T(hdth * P.a0);
+      pac = T(hdth * P.ac);
+      pas = T(hdth * P.as);
     }
 
     const T k = tc[FT_K], fo = cld(fr, o);
-    const T sdt = s.csdt * k;
-    const T sice = T(2) * tc[FT_CG0] * s.ice;
-    const T ctail = sdt + nu4 * (k * k) - sice;  // sdt + sdv - sice
-    const T crest = tc[FT_SBF] + ctail;
+    T ctail = s.csdt * k + nu4 * (k * k);  // sdt + sdv - sice
+    if (anyice) ctail -= T(2) * s.ice * bld<T>(row_rsrc(d.cg0, o, ldi), vj);
     const SinFreq<T> sf = sin_freq(s, tc[FT_LOGL2], tc[FT_CP0], fo * k * ig, sin_diss1, fs2);
-    const T cf = tpsf * fo;
-    const T coth = tc[FT_COTH];
-    const T lk4 = T(4) * Tr<T>::lg(k);        // lg(k^4)
-    const T Lk = spow * lk4 + Tr<T>::lg(cf);  // sds before cothkd
-    const T c0 = -dtx * crest, dtc = dtx * coth;
-    const T icfc = Tr<T>::rcp(cf * coth);
+    const T Lk = tc[FT_L];  // lg(cf coth k^(4 p)): sds after cothkd
+    const T c0 = -dtx * (tc[FT_SBF] + ctail);
+    const T icoth = Tr<T>::rcp(tc[FT_COTH]);  // X is sds e before cothkd
     // the spreading factor's upper bound, from the zeroth-moment prefix
-    [[maybe_unused]] const T qhi = (T(1) + T(2) * mssf * pc.a0) * (T(1) + T(2) * mssf * pc.a0);
+    [[maybe_unused]] const T qhi = (T(1) + T(2) * mssf * pa0) * (T(1) + T(2) * mssf * pa0);
     // dm = q0 + qc cos 2th + qs sin 2th = (q0 - qc) + ct (2 qc ct + 2 qs st),
     // with cos 2th = 2 ct^2 - 1 and sin 2th = 2 ct st: the sweep keeps
     // only ct and st per direction
-    const T qc = mssf * pc.ac;
-    const T q0m = T(1) + mssf * pc.a0 - qc, qc2 = T(2) * qc, qs2 = T(2) * mssf * pc.as;
+    const T qc = mssf * pac;
+    const T q0m = T(1) + mssf * pa0 - qc, qc2 = T(2) * qc, qs2 = T(2) * mssf * pas;
+    const bool own = o < o1;  // false in the two frequencies past the chunk
     const bool prog = o <= oc;
     const bool in1 = (o >= 1) && (o - 1 <= oc);  // bin o-1 is prognostic
-    const bool fin = valid && (o >= 2) && (o - 2 <= oc);  // bin o-2 completes now
-    const T hdb1 = in1 ? T(0.5) * dts * b1m1 : T(0), hdb2 = T(0.5) * dts * b2m2;
-    const uint32_t vtail = (valid && !prog) ? vj : kDropOffset;
+    const bool fin = valid && (o >= o0 + 2) && (o - 2 <= oc);  // bin o-2 completes now
+    const T hdb1 = in1 ? T(0.5) * dts * b1m1 * icoth : T(0), hdb2 = T(0.5) * dts * b2m2 * icoth;
+    const T dsc = dsnl * icoth;
+    const uint32_t vtail = (valid && !prog && own) ? vj : kDropOffset;
     const uint32_t vfin = fin ? vj : kDropOffset;
-    const bool anyfin = __any(fin), anytail = __any(valid && !prog);
+    const bool anyfin = __any(fin), anytail = own && __any(valid && !prog);
     const rsrc_t rs0 = freq_rsrc(esb, o, pm, ldi);
     // max(o, 2) - 2 rather than a conditional: the latter becomes a vector
     // saturating subtract, which moves the descriptor to vector registers
@@ -1047,35 +1145,49 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
     // any lane of the wave integrates a prognostic bin, fills a tail bin
     // or completes bin o-2 at this frequency (wave-uniform, so each
     // combination is a straight-line loop).
-    auto sweep = [&](auto PROG, auto TAIL, auto FIN) {
+    // NEEDX: some bin of the wave takes snl gains or losses from this
+    // frequency; past the cut-off's two followers none does and the
+    // dissipation (an exponential and a logarithm per bin) is not formed.
+    uint32_t mbl = mb;  // opaque copies: see k_rates
+    int dz = 0;
+    asm volatile("" : "+v"(mbl), "+s"(dz));
+    auto sweep = [&](auto PROG, auto TAIL, auto FIN, auto NEEDX) {
 #pragma unroll
       for (int q = 0; q < DMAX; ++q) {
         const uint32_t so = (uint32_t)(p0 + q) * rb;
-        const T ct = ctq[q], st = stq[q];
+        T ct, st, c2, s2;
+        cld4(dir4, p0 + q + dz, ct, st, c2, s2);
         const T e = ec[q];
-        const T ss = sin_m(sf, sin_y(sf, ct, st), mq[q]);
+        const T y = sin_y(sf, ct, st);
+        const T pos = sf.pos, neg1 = sf.neg1, neg2 = sf.neg2;  // see sin_bin
+        const T neg = ((mbl >> q) & 1) ? neg2 : neg1;
+        const T ss = y * (y > T(0) ? pos : neg);
         T dm = fma(ct, fma(qc2, ct, qs2 * st), q0m);
         dm = dm * dm;
         if constexpr (SUR) {
           if (do_sur && use) dm = fmin(fmax(T(1) + bf16_bits_to_f(rc[q]), T(1)), qhi);  // dm^2 - 1
         }
-        // sds before cothkd; |e|: see k_rates
-        const T sdsp = dm * Tr<T>::ex(fma(spow, Tr<T>::lg(fabs(e)), Lk));
-        const T X = sdsp * e;
-        T G = 0;
-        if constexpr (decltype(PROG)::value) {
-          // E_s = e exp(dts (ssin - sds - sbf - sdt - sdv + sice)) + dts snl
-          const T a = fma(-dtc, sdsp, fma(dtx, ss, c0));
-          G = prog ? fma(-dsnl, X, e * Tr<T>::ex(a)) : T(0);
+        T X = 0, G = 0;  // X: sds e (after cothkd)
+        if constexpr (decltype(NEEDX)::value) {
+          // |e|: see k_rates; a NaN of e stays in X through e
+          const T sds = dm * Tr<T>::ex_nn(fma(spow, Tr<T>::lg_nn(fabs(e)), Lk));
+          X = sds * e;
+          if constexpr (decltype(PROG)::value) {
+            // E_s = e exp(dts (ssin - sds - sbf - sdt - sdv + sice)) + dts snl
+            const T a = fma(-dtx, sds, fma(dtx, ss, c0));
+            G = prog ? fma(-dsc, X, e * Tr<T>::ex(a)) : T(0);
+          }
         }
         if constexpr (decltype(TAIL)::value) {
-          // diagnostic tail, src/umwm_physics.F90:70-80
+          // diagnostic tail, src/umwm_physics.F90:70-80: k^-4 (num / (cf
+          // coth dm^2))^(1/p) = ex((lg(num / dm^2) - Lk) / p)
           const T num = fmax(ss, T(0)) - ctail;
-          const T t = fmax(num, T(0)) * (icfc * Tr<T>::rcp(dm));
-          const T es_ = Tr<T>::ex(fma(ipow, Tr<T>::lg(t), -lk4));  // k^-4 t^(1/p)
+          const T t = fmax(num, T(0)) * Tr<T>::rcp(dm);
+          const T es_ = Tr<T>::ex(ipow * (Tr<T>::lg(t) - Lk));
           bst(FULL || q < nd ? rs0 : rz, vtail, T(0.5) * (e + es_), so);
         }
-        const T h1 = fma(hdb1, X, H1[q]);  // bf1r(o-1) X(o) into bin o-1
+        T h1 = H1[q];
+        if constexpr (decltype(NEEDX)::value) h1 = fma(hdb1, X, h1);  // bf1r(o-1) X(o) into bin o-1
         if constexpr (decltype(FIN)::value)  // bf2r(o-2) X(o) completes bin o-2
           bst(FULL || q < nd ? rs2 : rz, vfin, fma(hdb2, X, H2[q]), so);
         H2[q] = h1;
@@ -1084,19 +1196,17 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
     };
     using Y = std::true_type;
     using N = std::false_type;
-    const bool anyprog = __any(valid && prog);
+    const bool anyprog = own && __any(valid && prog);
     if (anyprog) {
       if (anytail) {
-        if (anyfin) sweep(Y{}, Y{}, Y{}); else sweep(Y{}, Y{}, N{});
+        if (anyfin) sweep(Y{}, Y{}, Y{}, Y{}); else sweep(Y{}, Y{}, N{}, Y{});
       } else {
-        if (anyfin) sweep(Y{}, N{}, Y{}); else sweep(Y{}, N{}, N{});
+        if (anyfin) sweep(Y{}, N{}, Y{}, Y{}); else sweep(Y{}, N{}, N{}, Y{});
       }
-    } else {
-      if (anytail) {
-        if (anyfin) sweep(N{}, Y{}, Y{}); else sweep(N{}, Y{}, N{});
-      } else {
-        if (anyfin) sweep(N{}, N{}, Y{}); else sweep(N{}, N{}, N{});
-      }
+    } else if (anyfin || __any(valid && in1)) {
+      if (anytail) sweep(N{}, Y{}, Y{}, Y{}); else sweep(N{}, N{}, Y{}, Y{});
+    } else if (anytail) {
+      sweep(N{}, Y{}, N{}, N{});
     }
     b2m2 = b2m1;
     b2m1 = tc[FT_B2];
@@ -1109,10 +1219,12 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
         for (int q = 0; q < DMAX; ++q) rc[q] = rn[q];
       }
     }
-    if constexpr (kDerive) {
-      tg.advance(o, knext);
-      pc = pn;
+    if constexpr (!kStoredPrefix<T>) {
+      P.add(k3, mo);
+      mo = mn;
+      k3 = k3n;
     }
+    if constexpr (kDerive) tg.advance(o, knext);
   }
 }
 
@@ -1135,14 +1247,107 @@ struct AdvLoads {
   T en0;                 // E^n at the point
 };
 
-template <typename T, int NB>
-__global__ __launch_bounds__(256) void k_advect(const DomainDev<T>* __restrict__ doms,
+// Sums over the directions in the order of the moments (see Mom): `add`
+// takes directions in sequence, `quad` ends a group of four, `seg` a segment.
+template <typename T>
+struct DirSums {
+  T q[5];
+  double s[5], t[5];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+      q[i] = 0;
+      s[i] = t[i] = 0;
+    }
+  }
+  // e, and its wind input in the stress partials
+  __device__ __forceinline__ void add(T v, T wv, T ct, T st, T c2, T s2) {
+    q[0] += v;
+    q[1] = fma(v, c2, q[1]);
+    q[2] = fma(v, s2, q[2]);
+    q[3] = fma(wv, ct, q[3]);
+    q[4] = fma(wv, st, q[4]);
+  }
+  template <int N>
+  __device__ __forceinline__ void quad() {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      s[i] += (double)q[i];
+      q[i] = 0;
+    }
+  }
+  template <int N>
+  __device__ __forceinline__ void seg() {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      t[i] += s[i];
+      s[i] = 0;
+    }
+  }
+};
+
+// Stores the moments and the x stress partial of (o, j).
+template <typename T>
+__device__ __forceinline__ void store_mom(T* mom, size_t ldi, int o, int j, T m0, T mc, T ms,
+                                          T tx) {
+  const rsrc_t sp = freq_rsrc(mom, o, 4, ldi);
+  if constexpr (sizeof(T) == 4) {
+    bst16(sp, (uint32_t)j * 16u, f32x4{m0, mc, ms, tx});
+  } else {
+    bst16(sp, (uint32_t)j * 32u, f64x2{m0, mc});
+    bst16(sp, (uint32_t)j * 32u + 16u, f64x2{ms, tx});
+  }
+}
+
+// The moments of the current spectrum, after anything but k_advect wrote it;
+// one wave per (frequency, 64 sea points).
+template <typename T>
+__global__ __launch_bounds__(64) void k_moments(const DomainDev<T>* __restrict__ doms,
                                                 const BlockTask* __restrict__ tasks) {
   const BlockTask tk = tasks[blockIdx.x];
   const DomainDev<T>& d = doms[tk.dom];
-  const int o = (int)blockIdx.y * (int)(blockDim.x >> 6) + wave_id();
+  const int o = (int)blockIdx.y, pm = d.pm;
+  if (o >= d.om) return;
+  const int j = tk.i0 + (int)threadIdx.x;
+  const size_t ldi = d.ldi;
+  const uint32_t vj = (uint32_t)j * (uint32_t)sizeof(T), rb = (uint32_t)ldi * (uint32_t)sizeof(T);
+  const rsrc_t pe = freq_rsrc(d.e, o, pm, ldi);
+  const int seglen = pm / dir_segments(pm);
+  DirSums<T> S;
+  S.clear();
+  int segend = seglen;
+  for (int p = 0; p < pm; p += 4) {
+    T v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = bld<T>(pe, vj, (p + q) * rb);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      T ct, st, c2, s2;
+      cld4(d.dir4, p + q, ct, st, c2, s2);
+      S.add(v[q], T(0), ct, st, c2, s2);
+    }
+    S.template quad<3>();
+    if (p + 4 == segend) {
+      S.template seg<3>();
+      segend += seglen;
+    }
+  }
+  if (j < d.im) store_mom(d.mom, ldi, o, j, T(S.t[0]), T(S.t[1]), T(S.t[2]), T(0));
+}
+
+// SPLIT: one workgroup per (frequency, 64 sea points), a wave per direction
+// segment, for launches that would otherwise leave most of the GPU idle.
+// Else fw = blockDim / 64 frequencies per workgroup, a wave taking all
+// directions of one.  Both give the same sums bit for bit.
+template <typename T, int NB, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 512 : 256) void k_advect(
+    const DomainDev<T>* __restrict__ doms, const BlockTask* __restrict__ tasks, int nseg) {
+  const BlockTask tk = tasks[blockIdx.x];
+  const DomainDev<T>& d = doms[tk.dom];
+  const int wid = wave_id();
+  const int o = SPLIT ? (int)blockIdx.y : (int)blockIdx.y * (int)(blockDim.x >> 6) + wid;
   const Scalars* sc = d.sc;
-  if (o >= d.om || !sc->active) return;
+  if (o >= d.om || !sc->active) return;  // uniform over the workgroup when SPLIT
   const int j = tk.i0 + (threadIdx.x & 63);
   const bool valid = j < d.im;
   const int pm = d.pm;
@@ -1180,28 +1385,38 @@ __global__ __launch_bounds__(256) void k_advect(const DomainDev<T>* __restrict__
   const SinFreq<T> sf = sin_freq(s, logl2, cp0, fkovg, sin_diss1, fs2);
   const rsrc_t pe = freq_rsrc(d.e, o, pm, ldi);    // E^n in, E^{n+1} out
   const rsrc_t ps = freq_rsrc(d.es, o, pm, ldi);   // E*
-  // the stress partials' cp0(o, i-1) (src/umwm_stress.F90:219,316) and kdk,
-  // loaded here so that their latency hides behind the direction loop
+  // the stress partials' cp0(o, i-1) (src/umwm_stress.F90:219,316), loaded
+  // here so that its latency hides behind the direction loop
   const T cp_prev = bld<T>(cpr, (uint32_t)((j == 0) ? d.im : j - 1) * E);
-  const T kdk = bld<T>(row_rsrc(d.kdk, o, ldi), vj);
   // direction tables in registers (see k_rates)
   const T* const cthb = d.cth;
   const T* const sthb = d.sth;
-  // stress_vector_integral partial sums over the directions of this
-  // frequency (FP32 within the frequency in the FP32 path, FP64 across)
-  T tx = 0, ty = 0, hs = 0;
-  auto stress_acc = [&](T ct, T st, T v) {
+  const T* const dir4 = d.dir4;
+  const int seglen = uniform_div(pm, nseg);
+  const int plo = SPLIT ? wid * seglen : 0, phi = SPLIT ? plo + seglen : pm;
+  // the moments of the new spectrum and the stress_vector_integral sums
+  // over the directions of this frequency
+  DirSums<T> S;
+  S.clear();
+  int segend = plo + seglen;
+  auto stress_acc = [&](int p, T v) {
+    T ct, st, c2, s2;
+    cld4(dir4, p, ct, st, c2, s2);
     const T m = s.cw * ct + s.sw * st > T(0) ? fs2 : T(1);
     T ss = sin_m(sf, sin_y(sf, ct, st), m);
     if (!prog) ss = fmax(ss, T(0));
-    const T wv = v * ss;
-    tx = fma(wv, ct, tx);
-    ty = fma(wv, st, ty);
-    hs += v;
+    S.add(v, v * ss, ct, st, c2, s2);
+  };
+  auto sums_end = [&](int pnext) {  // wave-uniform
+    if ((pnext & 3) == 0) S.template quad<5>();
+    if (pnext == segend) {
+      S.template seg<5>();
+      segend += seglen;
+    }
   };
   if (__all(!prog || !valid)) {
     // above the cut-off only the diagnostic tail: e = ef = E_s
-    for (int pb = 0; pb < pm; pb += NB) {
+    for (int pb = plo; pb < phi; pb += NB) {
       T v[NB];
 #pragma unroll
       for (int q = 0; q < NB; ++q)
@@ -1209,8 +1424,9 @@ __global__ __launch_bounds__(256) void k_advect(const DomainDev<T>* __restrict__
 #pragma unroll
       for (int q = 0; q < NB; ++q) {
         bst_stream(pe, vst, v[q], (pb + q) * rb);
-        stress_acc(cld(cthb, pb + q), cld(sthb, pb + q), v[q]);
+        stress_acc(pb + q, v[q]);
       }
+      sums_end(pb + NB);
     }
   } else {
     const int ie = pload(d.ie, ldi, j), iw = pload(d.iw, ldi, j);
@@ -1269,12 +1485,14 @@ __global__ __launch_bounds__(256) void k_advect(const DomainDev<T>* __restrict__
       }
     };
     AdvLoads<T> A[NB], B[NB];
-    const T efirst = bld<T>(ps, vj, 0);  // E*(0), periodic neighbour of pm-1
-    T eprev = bld<T>(ps, vj, (pm - 1) * rb);
-    load_block(0, A);
-    T rprev = rotp(pm - 1), rcur = rotp(0);
-    for (int pb = 0; pb < pm; pb += NB) {
-      const bool more = pb + NB < pm;
+    // E* of the directions before and after this wave's (periodic in pm)
+    const int pbef = plo > 0 ? plo - 1 : pm - 1, paft = phi < pm ? phi : 0;
+    const T efirst = bld<T>(ps, vj, paft * rb);
+    T eprev = bld<T>(ps, vj, pbef * rb);
+    load_block(plo, A);
+    T rprev = rotp(pbef), rcur = rotp(plo);
+    for (int pb = plo; pb < phi; pb += NB) {
+      const bool more = pb + NB < phi;
       if (more) load_block(pb + NB, B);
 #pragma unroll
       for (int q = 0; q < NB; ++q) {
@@ -1298,24 +1516,31 @@ __global__ __launch_bounds__(256) void k_advect(const DomainDev<T>* __restrict__
         T v = fma(-kr, fr, fma(-kk, flux, Es));
         v = prog ? v * keep : Es;
         bst_stream(pe, vst, v, p * rb);
-        stress_acc(ct, st, v);
+        stress_acc(p, v);
         eprev = e0;
         rprev = rcur;
         rcur = rnext;
       }
 #pragma unroll
       for (int q = 0; q < NB; ++q) A[q] = B[q];
+      sums_end(pb + NB);
     }
+  }
+  if constexpr (SPLIT) {
+    __shared__ double red[8][5][64];
+    const int lane = (int)threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) red[wid][i][lane] = S.t[i];
+    __syncthreads();
+    if (wid != 0) return;
+    for (int q = 1; q < nseg; ++q)
+#pragma unroll
+      for (int i = 0; i < 5; ++i) S.t[i] += red[q][i][lane];
   }
   if (valid) {
     const T icp = T(1) / cp_prev;
-    const rsrc_t sp = freq_rsrc(d.spart, o, 4, ldi);
-    if constexpr (sizeof(T) == 4) {
-      bst16(sp, (uint32_t)j * 16u, f32x4{tx * icp, ty * icp, hs * kdk, T(0)});
-    } else {
-      bst16(sp, (uint32_t)j * 32u, f64x2{tx * icp, ty * icp});
-      bst(sp, (uint32_t)j * 32u + 16u, hs * kdk);
-    }
+    store_mom(d.mom, ldi, o, j, T(S.t[0]), T(S.t[1]), T(S.t[2]), T(S.t[3]) * icp);
+    bst(row_rsrc(d.sty, o, ldi), vj, T(S.t[4]) * icp);
   }
 }
 
@@ -1343,7 +1568,8 @@ __global__ __launch_bounds__(64) void k_keep(const DomainDev<T>* __restrict__ do
 // ---------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(64) void k_stress(const DomainDev<T>* __restrict__ doms,
-                                               const BlockTask* __restrict__ tasks) {
+                                               const BlockTask* __restrict__ tasks,
+                                               int rates_split) {
   const BlockTask tk = tasks[blockIdx.x];
   const DomainDev<T>& d = doms[tk.dom];
   if (!d.sc->active) return;
@@ -1360,19 +1586,17 @@ __global__ __launch_bounds__(64) void k_stress(const DomainDev<T>* __restrict__ 
   double hs = 0;
   for (int o = 0; o < om; ++o) {
     const double kdk = bld<T>(row_rsrc(d.kdk, o, ldi), (uint32_t)j * E);
-    const rsrc_t sp = freq_rsrc(d.spart, o, 4, ldi);
-    double tx, ty, hso;
+    const rsrc_t sp = freq_rsrc(d.mom, o, 4, ldi);
+    double m0, tx;
     if constexpr (sizeof(T) == 4) {
       const f32x4 v = bld16<float>(sp, (uint32_t)j * 16u);
-      tx = v[0];
-      ty = v[1];
-      hso = v[2];
+      m0 = v[0];
+      tx = v[3];
     } else {
-      const f64x2 v = bld16<double>(sp, (uint32_t)j * 32u);
-      tx = v[0];
-      ty = v[1];
-      hso = bld<double>(sp, (uint32_t)j * 32u + 16u);
+      m0 = bld<double>(sp, (uint32_t)j * 32u);
+      tx = bld<double>(sp, (uint32_t)j * 32u + 24u);
     }
+    const double ty = bld<T>(row_rsrc(d.sty, o, ldi), (uint32_t)j * E);
     si.sx += tx * kdk;
     si.sy += ty * kdk;
     if (o >= oc) {
@@ -1383,7 +1607,7 @@ __global__ __launch_bounds__(64) void k_stress(const DomainDev<T>* __restrict__ 
       si.tomx = tx;
       si.tomy = ty;
     }
-    hs += hso;
+    hs += m0 * kdk;
   }
   si.wspd = w;
   si.wdir = pload(d.wdir, ldq, j);
@@ -1396,81 +1620,198 @@ __global__ __launch_bounds__(64) void k_stress(const DomainDev<T>* __restrict__ 
   si.kom = bld<T>(row_rsrc(d.k, om - 1, ldi), (uint32_t)j * E);
   store_stress(d, j, stress_atm_point(si, d.dthg, d.z, d.nu_air, d.kappa));
   pstore(d.hs_ice, ldi, j, 4 * sqrt(hs * d.dth));
-}
-
-template <typename T, int D1, int D2, bool SUR>
-void launch_sweeps(const DomainDev<T>* doms, const BlockTask* tasks, dim3 grid, size_t sh1,
-                   int first, int rotation, Tile tile, hipStream_t s, hipEvent_t* ev) {
-  // a launch whose waves all hold DMAX directions (W D = pm) takes the
-  // variant with no per-slot masks
-  if (tile.W1 * D1 == tile.pmax)
-    hipLaunchKernelGGL((k_rates<T, D1, true, SUR>), grid, dim3(64 * tile.W1), sh1, s, doms, tasks,
-                       first, rotation);
-  else
-    hipLaunchKernelGGL((k_rates<T, D1, false, SUR>), grid, dim3(64 * tile.W1), sh1, s, doms, tasks,
-                       first, rotation);
-  if (ev) (void)hipEventRecord(ev[1], s);
-  if (tile.W2 * D2 == tile.pmax)
-    hipLaunchKernelGGL((k_integrate<T, D2, true, SUR>), grid, dim3(64 * tile.W2), 0, s, doms, tasks);
-  else
-    hipLaunchKernelGGL((k_integrate<T, D2, false, SUR>), grid, dim3(64 * tile.W2), 0, s, doms,
-                       tasks);
-}
-
-template <typename T, int D1, int D2>
-int launch_all(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, int omax, int first,
-               int rotation, Tile tile, bool keep, hipStream_t s, hipEvent_t* ev, bool sur) {
-  const dim3 grid(ntasks);
-  // the moments' double buffer, and the surrogate's four cross-wave sums
-  const size_t sh1 = (size_t)std::max(2 * 3 * tile.W1, 4 * tile.W1) * 64 * sizeof(double);
-  if (ev) (void)hipEventRecord(ev[0], s);
-  if constexpr (std::is_same_v<T, float>) {
-    if (sur)
-      launch_sweeps<T, D1, D2, true>(doms, tasks, grid, sh1, first, rotation, tile, s, ev);
-    else
-      launch_sweeps<T, D1, D2, false>(doms, tasks, grid, sh1, first, rotation, tile, s, ev);
-  } else {
-    if (sur) return fail(UMWM_ERR_ARGUMENT, "the surrogate serves the FP32 path only");
-    launch_sweeps<T, D1, D2, false>(doms, tasks, grid, sh1, first, rotation, tile, s, ev);
+  if (rates_split) {  // k_rates' maximum over a point's workgroups
+    d.pts[j] = d.explim / __longlong_as_double((long long)d.rkey[j]);
+    d.rkey[j] = 0;
   }
-  if (keep) hipLaunchKernelGGL((k_keep<T>), grid, dim3(64), 0, s, doms, tasks);
+}
+
+// Launch shape of the fused kernels: direction groups and frequency chunks of
+// the two sweeps, waves per workgroup, and whether k_advect is split.
+struct Shape {
+  int D1, ng1, c1, w1;
+  int D2, ng2, c2, w2;
+  bool paired;  // k_rates pairs opposite directions where it can
+  bool split;
+};
+
+template <typename T, int D, bool SUR>
+void launch_rates(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, int pm, int first,
+                  int rotation, const Shape& h, hipStream_t s) {
+  const int slots = h.ng1 * h.c1;
+  const dim3 grid(ntasks, (slots + h.w1 - 1) / h.w1), block(64 * h.w1);
+  // the cross-wave maximum, and the surrogate's four cross-wave sums
+  const size_t sh = (size_t)(SUR ? 4 : 1) * h.w1 * 64 * sizeof(double);
+  // a launch whose waves all hold D directions takes a variant with no
+  // per-slot masks
+  if (h.ng1 * D == pm) {
+    if constexpr (D % 2 == 0) {
+      if (h.paired) {
+        hipLaunchKernelGGL((k_rates<T, D, true, true, SUR>), grid, block, sh, s, doms, tasks, first,
+                           rotation, h.ng1, h.c1);
+        return;
+      }
+    }
+    if constexpr (!(SUR && D % 2 == 0))
+      hipLaunchKernelGGL((k_rates<T, D, true, false, SUR>), grid, block, sh, s, doms, tasks, first,
+                         rotation, h.ng1, h.c1);
+  } else if constexpr (D > 4) {
+    hipLaunchKernelGGL((k_rates<T, D, false, false, SUR>), grid, block, sh, s, doms, tasks, first,
+                       rotation, h.ng1, h.c1);
+  }
+}
+
+template <typename T, int D, bool SUR>
+void launch_integrate(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, int pm,
+                      const Shape& h, hipStream_t s) {
+  const int slots = h.ng2 * h.c2;
+  const dim3 grid(ntasks, (slots + h.w2 - 1) / h.w2), block(64 * h.w2);
+  if (h.ng2 * D == pm)
+    hipLaunchKernelGGL((k_integrate<T, D, true, SUR>), grid, block, 0, s, doms, tasks, h.ng2, h.c2);
+  else if constexpr (D != 2 && D != 4)
+    hipLaunchKernelGGL((k_integrate<T, D, false, SUR>), grid, block, 0, s, doms, tasks, h.ng2, h.c2);
+}
+
+template <typename T, bool SUR>
+int launch_kernels(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, int omax, int pm,
+                   int first, int rotation, const Shape& h, int nb, bool keep, hipStream_t s,
+                   hipEvent_t* ev) {
+  if (ev) (void)hipEventRecord(ev[0], s);
+#define UMWM_RATES(D_)                                                                       \
+  case D_: launch_rates<T, D_, SUR>(doms, tasks, ntasks, pm, first, rotation, h, s); break;
+  switch (h.D1) {
+    UMWM_RATES(6)
+    UMWM_RATES(9)
+    UMWM_RATES(18)
+    UMWM_RATES(36)
+    default:
+      if constexpr (!SUR) {
+        switch (h.D1) {
+          UMWM_RATES(2)
+          UMWM_RATES(4)
+          default: return fail(UMWM_ERR_ARGUMENT, "unsupported rates tile D");
+        }
+        break;
+      }
+      return fail(UMWM_ERR_ARGUMENT, "unsupported rates tile D");
+  }
+#undef UMWM_RATES
+  if (ev) (void)hipEventRecord(ev[1], s);
+#define UMWM_INTEGRATE(D_)                                                           \
+  case D_: launch_integrate<T, D_, SUR>(doms, tasks, ntasks, pm, h, s); break;
+  switch (h.D2) {
+    UMWM_INTEGRATE(3)
+    UMWM_INTEGRATE(6)
+    UMWM_INTEGRATE(9)
+    UMWM_INTEGRATE(12)
+    UMWM_INTEGRATE(18)
+    default:
+      if constexpr (!SUR) {
+        switch (h.D2) {
+          UMWM_INTEGRATE(2)
+          UMWM_INTEGRATE(4)
+          default: return fail(UMWM_ERR_ARGUMENT, "unsupported integrate tile D");
+        }
+        break;
+      }
+      return fail(UMWM_ERR_ARGUMENT, "unsupported integrate tile D");
+  }
+#undef UMWM_INTEGRATE
+  if (keep) hipLaunchKernelGGL((k_keep<T>), dim3(ntasks), dim3(64), 0, s, doms, tasks);
   if (ev) (void)hipEventRecord(ev[2], s);
-  // advect: one wave per (64 points, frequency), FW frequencies per
-  // workgroup (2 measured 1-2 % faster than 4 or 8 on C2)
-  const int fw = 2;
-  const dim3 ga(ntasks, (omax + fw - 1) / fw);
-  if (tile.NB == 4)
-    hipLaunchKernelGGL((k_advect<T, 4>), ga, dim3(64 * fw), 0, s, doms, tasks);
-  else
-    hipLaunchKernelGGL((k_advect<T, 2>), ga, dim3(64 * fw), 0, s, doms, tasks);
+  const int nseg = dir_segments(pm);
+  if (h.split && nseg > 1) {
+    const dim3 ga(ntasks, omax), block(64 * nseg);
+    if (nb == 4)
+      hipLaunchKernelGGL((k_advect<T, 4, true>), ga, block, 0, s, doms, tasks, nseg);
+    else
+      hipLaunchKernelGGL((k_advect<T, 2, true>), ga, block, 0, s, doms, tasks, nseg);
+  } else {
+    // one wave per (64 points, frequency), FW frequencies per workgroup (2
+    // measured 1-2 % faster than 4 or 8 on 720x360)
+    const int fw = 2;
+    const dim3 ga(ntasks, (omax + fw - 1) / fw);
+    if (nb == 4)
+      hipLaunchKernelGGL((k_advect<T, 4, false>), ga, dim3(64 * fw), 0, s, doms, tasks, nseg);
+    else
+      hipLaunchKernelGGL((k_advect<T, 2, false>), ga, dim3(64 * fw), 0, s, doms, tasks, nseg);
+  }
   if (ev) (void)hipEventRecord(ev[3], s);
-  hipLaunchKernelGGL((k_stress<T>), grid, dim3(64), 0, s, doms, tasks);
+  hipLaunchKernelGGL((k_stress<T>), dim3(ntasks), dim3(64), 0, s, doms, tasks,
+                     h.ng1 * h.c1 > h.w1 ? 1 : 0);
   if (ev) (void)hipEventRecord(ev[4], s);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(UMWM_ERR_HIP, std::string("fused launch: ") + hipGetErrorString(e));
   return 0;
 }
 
-template <typename T, int D1>
-int launch_d2(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, int omax, int first,
-              int rotation, Tile tile, bool keep, hipStream_t s, hipEvent_t* ev, bool sur) {
-#define UMWM_D2(D2_)                                                                         \
-  case D2_:                                                                                  \
-    return launch_all<T, D1, D2_>(doms, tasks, ntasks, omax, first, rotation, tile, keep, s, ev, sur);
-  switch (tile.D2) {
-    UMWM_D2(3)
-    UMWM_D2(6)
-    UMWM_D2(9)
-    UMWM_D2(12)
-    UMWM_D2(18)
-  }
-#undef UMWM_D2
-  return fail(UMWM_ERR_ARGUMENT, "unsupported integrate tile D");
+}  // namespace
+
+bool tile_supported(int D) { return D == 3 || D == 6 || D == 9 || D == 12 || D == 18 || D == 36; }
+
+namespace {
+
+// Waves per workgroup for `slots` waves of a point block: the largest divisor
+// up to 8, or 8 (the last workgroup then holds idle waves).
+int waves_for(int slots) {
+  for (int w = 8; w >= 4; --w)
+    if (slots % w == 0) return w;
+  return std::min(slots, 8);
+}
+
+// Launch shape of default tiles.  The sweeps need about kSweepWaves waves to
+// fill the GPU; a point block offers pm / D of them, and a frequency chunk
+// costs a prefix sum over the frequencies below it (both sweeps) and the
+// dissipation of two more (k_integrate), so small grids are split over
+// frequency as far as it takes, down to four frequencies a chunk, and then
+// over pairs of directions.  37 x 36 bins, k_rates + k_integrate in us, before
+// (one chunk of nine directions) and as chosen here:
+//   169 points    FP64 267 -> 38   FP32 102 -> 33
+//   2,809 points  FP64 284 -> 75   FP32 104 -> 41
+//   11,449 points FP64 303 -> 188  FP32 108 -> 78
+// D divides pm: masked slots cost as much as full ones (pm = 48 at 13,924
+// points, D = 6 against 9: FP64 633 -> 310 us, FP32 125 -> 98).
+// k_advect's split pays while its waves (one per frequency and point block)
+// leave the GPU short of work: 2,809 points FP64 29.7 -> 25.7, FP32 25.6 ->
+// 19.2 us; 11,449 points 84.9 -> 92.9 and 39.4 -> 49.1 us.
+constexpr int kSweepWaves = 1536;
+constexpr int kAdvectWaves = 4096;
+
+Shape choose_shape(const Tile& t, int ntasks, int omax, bool sur) {
+  Shape h{t.D1, t.W1, 1, t.W1, t.D2, t.W2, 1, t.W2, true, false};
+  const int pm = t.pmax;
+  // the network's checks need all of a point's waves in one workgroup; wide
+  // spectra keep the tile's own shape
+  if (t.chosen || sur || pm > 72) return h;
+  auto chunks = [&](int D) {
+    const int waves = ntasks * (pm / D);
+    return std::max(1, std::min((kSweepWaves + waves / 2) / waves, omax / 4));
+  };
+  int D = pm % 9 == 0 ? 9 : pm % 6 == 0 ? 6 : 4;
+  if (ntasks * (pm / D) * chunks(D) < kSweepWaves / 2) D = 2;
+  h.D1 = h.D2 = D;
+  h.ng1 = h.ng2 = pm / D;
+  h.c1 = h.c2 = chunks(D);
+  h.w1 = h.w2 = waves_for(h.ng1 * h.c1);
+  h.paired = false;  // one order of operations whatever D
+  h.split = ntasks * omax < kAdvectWaves;
+  return h;
 }
 
 }  // namespace
 
-bool tile_supported(int D) { return D == 3 || D == 6 || D == 9 || D == 12 || D == 18 || D == 36; }
+template <typename T>
+int launch_moments(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, int omax,
+                   hipStream_t s) {
+  if (ntasks <= 0) return 0;
+  hipLaunchKernelGGL((k_moments<T>), dim3(ntasks, omax), dim3(64), 0, s, doms, tasks);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(UMWM_ERR_HIP, std::string("k_moments: ") + hipGetErrorString(e));
+  return 0;
+}
+template int launch_moments<float>(const DomainDev<float>*, const BlockTask*, int, int, hipStream_t);
+template int launch_moments<double>(const DomainDev<double>*, const BlockTask*, int, int,
+                                    hipStream_t);
 
 template <typename T>
 int launch_fused(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, int omax,
@@ -1493,13 +1834,16 @@ int launch_fused(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, i
       tile.W2 *= 2;
     }
   }
-  switch (tile.D1) {
-    case 6: return launch_d2<T, 6>(doms, tasks, ntasks, omax, first, rotation, tile, keep, s, ev, sur);
-    case 9: return launch_d2<T, 9>(doms, tasks, ntasks, omax, first, rotation, tile, keep, s, ev, sur);
-    case 18: return launch_d2<T, 18>(doms, tasks, ntasks, omax, first, rotation, tile, keep, s, ev, sur);
-    case 36: return launch_d2<T, 36>(doms, tasks, ntasks, omax, first, rotation, tile, keep, s, ev, sur);
+  const Shape h = choose_shape(tile, ntasks, omax, sur);
+  if constexpr (std::is_same_v<T, float>) {
+    if (sur)
+      return launch_kernels<T, true>(doms, tasks, ntasks, omax, tile.pmax, first, rotation, h,
+                                     tile.NB, keep, s, ev);
+  } else if (sur) {
+    return fail(UMWM_ERR_ARGUMENT, "the surrogate serves the FP32 path only");
   }
-  return fail(UMWM_ERR_ARGUMENT, "unsupported rates tile D");
+  return launch_kernels<T, false>(doms, tasks, ntasks, omax, tile.pmax, first, rotation, h, tile.NB,
+                                  keep, s, ev);
 }
 
 template int launch_fused<float>(const DomainDev<float>*, const BlockTask*, int, int, int, int,

@@ -219,6 +219,12 @@ __device__ inline double wave_sum(double v) {
   return v;
 }
 
+// Maximum over the wavefront, in a scalar register.
+__device__ inline int wave_max_i32(int v) {
+  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+  return __builtin_amdgcn_readfirstlane(v);
+}
+
 // Order-preserving map of doubles (NaN aside) onto unsigned 64-bit keys, so
 // that an integer atomic max combines doubles; ~okey(x) does the same for a
 // min.  No double maps to key 0, which therefore stands for "no value".

@@ -262,7 +262,8 @@ void dispersion(HostSetup& S, double tol) {
   auto T = [ldi](std::vector<double>& a, int o, int j) -> double& { return a[(size_t)o * ldi + j]; };
   const size_t nt = (size_t)om * ldi;
   for (auto* v : {&S.k, &S.kdk, &S.k3dk, &S.k4, &S.oneoverk4, &S.cp0, &S.cg0, &S.invcp0, &S.fkovg,
-                  &S.logl2overz, &S.cothkd, &S.sbf, &S.sdv, &S.snl_arg, &S.bf1r, &S.bf2r, &S.dwn})
+                  &S.logl2overz, &S.cothkd, &S.sbf, &S.sdv, &S.snl_arg, &S.bf1r, &S.bf2r, &S.dwn,
+                  &S.lsds})
     v->assign(nt, 0.0);
   std::vector<double> kd(nt, 0.0);
   parallel_for(im, [&](int a, int b) {
@@ -309,6 +310,8 @@ void dispersion(HostSetup& S, double tol) {
         T(S.k3dk, o, j) = std::pow(kk, 3.) * T(S.dwn, o, j);
         T(S.fkovg, o, j) = fo * kk / g;
         T(S.cothkd, o, j) = std::cosh(0.2 * kdv) / std::sinh(0.2 * kdv);
+        T(S.lsds, o, j) = 4. * P.sds_power * std::log(kk) +
+                          std::log(S.twopisds_fac * fo * T(S.cothkd, o, j));
         T(S.invcp0, o, j) = 1. / cp;
         T(S.sbf, o, j) = P.sbf_fac * kk / (std::sinh(2. * kdv)) +
                          P.sbp_fac * kk / (std::cosh(kdv) * std::cosh(kdv));

@@ -32,6 +32,7 @@ struct HostSetup {
   // (o, j) tables, [o * ldi + j], ghost column j = im for cp0/cg0
   std::vector<double> k, kdk, k3dk, k4, oneoverk4, cp0, cg0, invcp0, fkovg;
   std::vector<double> logl2overz, cothkd, sbf, sdv, snl_arg, bf1r, bf2r, dwn;
+  std::vector<double> lsds;  // log(2 pi sds_fac f cothkd k^(4 sds_power)), FP64 sweeps
   // (p, j)
   std::vector<double> cth_curv, sth_curv;
   std::vector<double> ccurv, scurv;  // per sea point
