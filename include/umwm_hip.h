@@ -235,8 +235,8 @@ int umwm_hip_substeps(umwm_domain* dom, int32_t n, double* sumt, double* dts, in
  * reference: it is for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  Same results as umwm_hip_substeps, bit for bit.  The fused
- * kernels' scratch (the FP64 frequency prefix of the cos^2 moments and the
- * stress partial sums, with room for 2 x 4 x om x ldi values of the working
+ * kernels' scratch (the frequency prefix of the cos^2 moments and the stress
+ * partial sums, with room for 2 x 4 x om x ldi values of the working
  * precision, ldi = im + 1 rounded up to 64) lives in one file-scope device
  * array of 32 MiB per GPU, shared by every call on that GPU and kept until the
  * process ends; a domain needing more returns UMWM_ERR_SIZE (FP64 with

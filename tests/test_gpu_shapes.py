@@ -55,7 +55,9 @@ def test_default_shape_equals_explicit_tile(grid, precision):
 @pytest.mark.parametrize("grid", [(12, 11, 37, 36), (30, 21, 31, 28), (105, 101, 29, 24)])
 def test_moments_after_set_equal_advection(grid, precision):
     """Setting the spectrum to itself makes the next substep form the moments
-    anew: bit for bit what the advection had left."""
+    anew: what the advection had left.  FP64 agrees bit for bit; in FP32 the
+    host may flush subnormal bins (below 1.2e-38) on the way through set, so
+    the spectra agree to far below the rounding of a different sum."""
     a, b = fresh(grid, precision), fresh(grid, precision)
     try:
         for d in (a, b):
@@ -64,8 +66,10 @@ def test_moments_after_set_equal_advection(grid, precision):
         b.set("e", e)
         a.substeps(2)
         b.substeps(2)
+        tol = 0.0 if precision == 8 else 1e-12
         for name in ("e", "ustar"):
-            assert np.array_equal(a.get(name), b.get(name)), name
+            x, y = a.get(name), b.get(name)
+            assert np.linalg.norm(x - y) <= tol * np.linalg.norm(y), name
     finally:
         a.close()
         b.close()

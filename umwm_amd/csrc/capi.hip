@@ -16,9 +16,9 @@
 #include "rawio.hpp"
 #include "surrogate.hpp"
 
-// Scratch of umwm_hip_substeps_noalloc: the fused kernels' FP64 prefix
-// moments ([om][ldi][4]) and y stress partials ([om][ldi]), which the other
-// entry points keep in buffers allocated with the domain.  Every
+// Scratch of umwm_hip_substeps_noalloc: the fused kernels' prefix
+// moments ([om][3][ldi]) and stress partials ([om][2 or 3][ldi]), which the
+// other entry points keep in buffers allocated with the domain.  Every
 // GPU the library runs on holds one copy until the process ends; in host
 // code the name is only a stand-in, and the device address comes from
 // hipGetSymbolAddress (umwm::noalloc_scratch).
@@ -227,6 +227,12 @@ int ensure_ops(DomainImpl<T>& D) {
   UMWM_HIP_TRY(hipStreamSynchronize(D.stream));
   D.ops_ready = true;
   return 0;
+}
+
+// stokes_drift and/or diag of one domain.
+template <typename T>
+int launch_end(DomainImpl<T>& D, bool stokes, bool diag) {
+  return launch_integrals<T>(D.d, D.tasks, D.ntasks, D.end_d, D.h.lm, stokes, diag, D.stream);
 }
 
 template <typename T>
@@ -439,17 +445,17 @@ int create_impl(const umwm_params& P, const umwm_grid_input* g, const umwm_forci
   // reduction scratch and scalars
   h.nblocks = (S.im + kLanes - 1) / kLanes;
   h.block0 = 0;
-  h.mom = A.template alloc<T>(4 * nt);
-  h.sty = A.template alloc<T>(nt);
+  h.mom = A.template alloc<double>(3 * nt);
+  h.sp = A.template alloc<T>(kPartials<T> * nt);
   h.rkey = A.template alloc<unsigned long long>(ldi);
-  h.pfx = sizeof(T) == 8 ? A.template alloc<T>(4 * nt) : nullptr;
+  h.pfx = A.template alloc<T>(3 * nt);
   h.sc = A.template alloc<Scalars>(1);
-  if (!h.sc || !h.mom || !h.sty || !h.rkey || (sizeof(T) == 8 && !h.pfx)) {
+  if (!h.sc || !h.mom || !h.sp || !h.rkey || !h.pfx) {
     delete D;
     return fail(UMWM_ERR_NOMEM, "device allocation failed");
   }
-  if (h.pfx && (rc = dfill<T>(h.pfx, 4 * nt, T(0), s))) { delete D; return rc; }
-  if ((rc = dfill<T>(h.mom, 4 * nt, T(0), s)) || (rc = dfill<T>(h.sty, nt, T(0), s)) ||
+  if ((rc = dfill<T>(h.pfx, 3 * nt, T(0), s)) || (rc = dfill<double>(h.mom, 3 * nt, 0.0, s)) ||
+      (rc = dfill<T>(h.sp, kPartials<T> * nt, T(0), s)) ||
       (rc = dfill<unsigned long long>(h.rkey, ldi, 0ull, s))) {
     delete D;
     return rc;
@@ -463,10 +469,10 @@ int create_impl(const umwm_params& P, const umwm_grid_input* g, const umwm_forci
   UMWM_HIP_TRY(hipMemcpyAsync(h.sc, &sc0, sizeof(Scalars), hipMemcpyHostToDevice, s));
   UMWM_HIP_TRY(hipHostMalloc((void**)&D->sc_host, sizeof(Scalars), hipHostMallocDefault));
   // diag and Stokes outputs
-  double** dg[] = {&D->diag.ht, &D->diag.mwp, &D->diag.mwd, &D->diag.mss, &D->diag.mwl,
-                   &D->diag.momx, &D->diag.momy, &D->diag.cgmxx, &D->diag.cgmxy, &D->diag.cgmyy,
-                   &D->diag.dwd, &D->diag.dwl, &D->diag.dwp, &D->diag.dcp0, &D->diag.dcg0,
-                   &D->diag.dcp, &D->diag.dcg};
+  double** dg[] = {&D->end.diag.ht, &D->end.diag.mwp, &D->end.diag.mwd, &D->end.diag.mss, &D->end.diag.mwl,
+                   &D->end.diag.momx, &D->end.diag.momy, &D->end.diag.cgmxx, &D->end.diag.cgmxy, &D->end.diag.cgmyy,
+                   &D->end.diag.dwd, &D->end.diag.dwl, &D->end.diag.dwp, &D->end.diag.dcp0, &D->end.diag.dcg0,
+                   &D->end.diag.dcp, &D->end.diag.dcg};
   for (double** p : dg) {
     *p = A.template alloc<double>(ldi);
     UMWM_HIP_TRY(hipMemsetAsync(*p, 0, ldi * sizeof(double), s));
@@ -476,18 +482,24 @@ int create_impl(const umwm_params& P, const umwm_grid_input* g, const umwm_forci
   std::vector<double> dlh(lm, 0.0);
   for (int l = 0; l < S.lm; ++l) dlh[l] = S.depth_l[l];
   UMWM_HIP_TRY(hipMemcpyAsync(dl, dlh.data(), lm * sizeof(double), hipMemcpyHostToDevice, s));
-  D->stokes.depth = dl;
+  D->end.stokes.depth = dl;
   const size_t nus = (size_t)lm * ldi;
-  D->stokes.us = A.template alloc<double>(nus);
-  D->stokes.vs = A.template alloc<double>(nus);
-  D->stokes.ds = A.template alloc<double>(ldi);
-  if (!D->stokes.ds) {
+  D->end.stokes.us = A.template alloc<double>(nus);
+  D->end.stokes.vs = A.template alloc<double>(nus);
+  D->end.stokes.ds = A.template alloc<double>(ldi);
+  if (!D->end.stokes.ds) {
     delete D;
     return fail(UMWM_ERR_NOMEM, "device allocation of Stokes arrays failed");
   }
-  UMWM_HIP_TRY(hipMemsetAsync(D->stokes.us, 0, nus * sizeof(double), s));
-  UMWM_HIP_TRY(hipMemsetAsync(D->stokes.vs, 0, nus * sizeof(double), s));
-  UMWM_HIP_TRY(hipMemsetAsync(D->stokes.ds, 0, ldi * sizeof(double), s));
+  UMWM_HIP_TRY(hipMemsetAsync(D->end.stokes.us, 0, nus * sizeof(double), s));
+  UMWM_HIP_TRY(hipMemsetAsync(D->end.stokes.vs, 0, nus * sizeof(double), s));
+  UMWM_HIP_TRY(hipMemsetAsync(D->end.stokes.ds, 0, ldi * sizeof(double), s));
+  D->end_d = A.template alloc<EndDev>(1);
+  if (!D->end_d) {
+    delete D;
+    return fail(UMWM_ERR_NOMEM, "device allocation failed");
+  }
+  UMWM_HIP_TRY(hipMemcpyAsync(D->end_d, &D->end, sizeof(EndDev), hipMemcpyHostToDevice, s));
   // forcing levels
   ForcingDev<T>& F = D->fh;
   const size_t n2 = (size_t)S.mm * S.nm;
@@ -556,7 +568,7 @@ int create_impl(const umwm_params& P, const umwm_grid_input* g, const umwm_forci
   for (auto& e : D->ev) UMWM_HIP_TRY(hipEventCreate(&e));
   UMWM_HIP_TRY(hipStreamSynchronize(s));
   // stokes_drift('init') on the cold-start spectrum, as umwm_initialize does
-  if ((rc = launch_stokes(*D))) { delete D; return rc; }
+  if ((rc = launch_end(*D, true, false))) { delete D; return rc; }
   if ((rc = launch_hs_ice(*D))) { delete D; return rc; }
   UMWM_HIP_TRY(hipStreamSynchronize(s));
   out = D;
@@ -661,7 +673,7 @@ int fused_substep(DomainImpl<T>& D, const DomainDev<T>* dd = nullptr) {
   D.ef_mirrors_e = true;
   D.rot_valid = true;
   if (D.first) {
-    if ((rc = launch_diag(D))) return rc;
+    if ((rc = launch_end(D, false, true))) return rc;
     D.first = false;
   }
   if (D.timing) {
@@ -742,7 +754,7 @@ int substeps_impl(DomainImpl<T>& D, int n) {
   return read_scalars(D);
 }
 
-// umwm_hip_substeps_noalloc: the same substeps with the prefix moments and y
+// umwm_hip_substeps_noalloc: the same substeps with the prefix moments and
 // stress partials in the device's shared scratch array (room for two records
 // of four values per frequency and point).
 // Calls no allocating routine: the record copy and the scratch address were
@@ -759,8 +771,8 @@ int substeps_noalloc_impl(DomainImpl<T>& D, int n) {
                                    " bytes of the shared array; use umwm_hip_substeps");
   if (!D.scr || !D.d_scr) return fail(UMWM_ERR_STATE, "substeps_noalloc: no scratch set up");
   D.h_scr = D.h;
-  if (D.h.pfx) D.h_scr.pfx = reinterpret_cast<T*>(D.scr);
-  D.h_scr.sty = reinterpret_cast<T*>(D.scr + off);
+  D.h_scr.pfx = reinterpret_cast<T*>(D.scr);
+  D.h_scr.sp = reinterpret_cast<T*>(D.scr + off);
   UMWM_HIP_TRY(hipMemcpyAsync(D.d_scr, &D.h_scr, sizeof(DomainDev<T>), hipMemcpyHostToDevice,
                               D.stream));
   // the array keeps the previous call's contents: start from zeros, as the
@@ -793,8 +805,7 @@ int run_dtg_impl(DomainImpl<T>& D, int32_t* nsub) {
   }
   n = D.sc_host->nsub;
   if (D.firstdtg) D.firstdtg = false;
-  if (D.S.P.stokes && (rc = launch_stokes(D))) return rc;
-  if ((rc = launch_diag(D))) return rc;
+  if ((rc = launch_end(D, D.S.P.stokes != 0, true))) return rc;
   UMWM_HIP_TRY(hipStreamSynchronize(D.stream));
   if (nsub) *nsub = n;
   return 0;
@@ -860,11 +871,11 @@ bool find_field(DomainImpl<T>& D, const std::string& n, FieldRef& r) {
       {"taux_form", h.taux_form}, {"tauy_form", h.tauy_form}, {"taux_skin", h.taux_skin},
       {"tauy_skin", h.tauy_skin}, {"taux_diag", h.taux_diag}, {"tauy_diag", h.tauy_diag},
       {"tailatmx", h.tailatmx}, {"tailatmy", h.tailatmy}, {"physics_time_step", h.pts},
-      {"ht", D.diag.ht}, {"mwp", D.diag.mwp}, {"mwd", D.diag.mwd}, {"mss", D.diag.mss},
-      {"mwl", D.diag.mwl}, {"momx", D.diag.momx}, {"momy", D.diag.momy},
-      {"cgmxx", D.diag.cgmxx}, {"cgmxy", D.diag.cgmxy}, {"cgmyy", D.diag.cgmyy},
-      {"dwd", D.diag.dwd}, {"dwl", D.diag.dwl}, {"dwp", D.diag.dwp}, {"dcp0", D.diag.dcp0},
-      {"dcg0", D.diag.dcg0}, {"dcp", D.diag.dcp}, {"dcg", D.diag.dcg}, {"ds", D.stokes.ds},
+      {"ht", D.end.diag.ht}, {"mwp", D.end.diag.mwp}, {"mwd", D.end.diag.mwd}, {"mss", D.end.diag.mss},
+      {"mwl", D.end.diag.mwl}, {"momx", D.end.diag.momx}, {"momy", D.end.diag.momy},
+      {"cgmxx", D.end.diag.cgmxx}, {"cgmxy", D.end.diag.cgmxy}, {"cgmyy", D.end.diag.cgmyy},
+      {"dwd", D.end.diag.dwd}, {"dwl", D.end.diag.dwl}, {"dwp", D.end.diag.dwp}, {"dcp0", D.end.diag.dcp0},
+      {"dcg0", D.end.diag.dcg0}, {"dcp", D.end.diag.dcp}, {"dcg", D.end.diag.dcg}, {"ds", D.end.stokes.ds},
       {"hs_ice", h.hs_ice}};
   for (auto& t : ptd)
     if (n == t.first) return set(F_PT_D, t.second);
@@ -875,8 +886,8 @@ bool find_field(DomainImpl<T>& D, const std::string& n, FieldRef& r) {
     }
   if (n == "oc") return set(F_PT_I, h.oc);
   if (n == "oc_rot") return set(F_PT_I, h.oc_rot);
-  if (n == "us") return set(F_STOKES, D.stokes.us);
-  if (n == "vs") return set(F_STOKES, D.stokes.vs);
+  if (n == "us") return set(F_STOKES, D.end.stokes.us);
+  if (n == "vs") return set(F_STOKES, D.end.stokes.vs);
   // host-side setup products
   const std::pair<const char*, const std::vector<int>*> maps[] = {
       {"iw", &S.iw}, {"ie", &S.ie}, {"is", &S.is}, {"in", &S.in},
@@ -1036,6 +1047,7 @@ struct BatchImpl {
   // of D directions each, W = ceil(pm / D) for the batch's D
   struct Group {
     int pm = 0, omax = 0, ntasks = 0;
+    int lm = 0, members = 0, drift = 0;  // levels; members, and those with Stokes drift
     BlockTask* tasks = nullptr;
     Tile tile;
   };
@@ -1054,6 +1066,7 @@ struct BatchImpl {
   // start of every run, so that forcinginput's level swaps reach the
   // kernels and the captured graph) and the list of forced members
   ForcingDev<T>* d_fds = nullptr;
+  EndDev* d_ends = nullptr;  // the members' diag and Stokes outputs
   int32_t* d_flist = nullptr;
   int nforced = 0, maximm = 0;
   bool forced_currents = false;
@@ -1209,7 +1222,7 @@ int umwm_hip_init_jonswap(umwm_domain* dom, const umwm_jonswap* js) {
 int umwm_hip_stokes_drift(umwm_domain* dom, int init) {
   (void)init;  // transfer coefficients are evaluated on the fly
   return dispatch(dom, [&](auto& D) {
-    int rc = launch_stokes(D);
+    int rc = launch_end(D, true, false);
     return rc ? rc : sync_and_check(D);
   });
 }
@@ -1369,7 +1382,7 @@ int umwm_hip_stress(umwm_domain* dom, const char* option) {
 
 int umwm_hip_diag(umwm_domain* dom) {
   return dispatch(dom, [&](auto& D) {
-    int rc = launch_diag(D);
+    int rc = launch_end(D, false, true);
     return rc ? rc : sync_and_check(D);
   });
 }
@@ -1811,6 +1824,9 @@ int batch_create_impl(umwm_domain* const* doms, int n, BatchImpl<T>*& out) {
     for (int k : order) {
       if (B->doms[k]->S.pm != pm) continue;
       g.omax = std::max(g.omax, B->doms[k]->S.om);
+      g.lm = std::max(g.lm, B->doms[k]->S.lm);
+      g.members += 1;
+      g.drift += B->doms[k]->S.P.stokes && B->doms[k]->S.lm > 0 ? 1 : 0;
       for (int b = 0; b < hd[k].nblocks; ++b) tk.push_back(BlockTask{k, b * kLanes, b, 0});
     }
     std::vector<int> ord = xcd_order((int)tk.size());
@@ -1828,6 +1844,14 @@ int batch_create_impl(umwm_domain* const* doms, int n, BatchImpl<T>*& out) {
   }
   std::vector<Scalars*> scs(n);
   for (int k = 0; k < n; ++k) scs[k] = hd[k].sc;
+  std::vector<EndDev> ends(n);
+  for (int k = 0; k < n; ++k) ends[k] = B->doms[k]->end;
+  B->d_ends = B->arena.template alloc<EndDev>(n);
+  if (!B->d_ends) {
+    delete B;
+    return fail(UMWM_ERR_NOMEM, "batch allocation failed");
+  }
+  UMWM_HIP_TRY(hipMemcpy(B->d_ends, ends.data(), n * sizeof(EndDev), hipMemcpyHostToDevice));
   std::vector<int32_t> fl;
   for (int k = 0; k < n; ++k)
     if (any_forcing(*B->doms[k])) {
@@ -1845,15 +1869,24 @@ int batch_create_impl(umwm_domain* const* doms, int n, BatchImpl<T>*& out) {
   return 0;
 }
 
-// Runs a per-domain launcher on another stream (batch members share the
-// batch stream so a whole substep can be captured as one graph).
+// diag of every member, and stokes_drift of those that have it when `stokes`:
+// one launch per pm class (two where only some members drift).
 template <typename T>
-int on_stream(DomainImpl<T>& D, hipStream_t s, int (*fn)(DomainImpl<T>&)) {
-  hipStream_t keep = D.stream;
-  D.stream = s;
-  const int rc = fn(D);
-  D.stream = keep;
-  return rc;
+int batch_integrals(BatchImpl<T>& B, bool stokes) {
+  for (const auto& g : B.groups) {
+    if (!stokes || g.drift == 0 || g.drift == g.members) {
+      if (int rc = launch_integrals<T>(B.d_doms, g.tasks, g.ntasks, B.d_ends, g.lm,
+                                       stokes && g.drift, true, B.stream))
+        return rc;
+      continue;
+    }
+    for (auto* D : B.doms)
+      if (D->S.pm == g.pm)
+        if (int rc = launch_integrals<T>(D->d, D->tasks, D->ntasks, D->end_d, D->h.lm,
+                                         D->S.P.stokes != 0, true, B.stream))
+          return rc;
+  }
+  return 0;
 }
 
 // Uploads every member's current domain and forcing records (a member's
@@ -1926,8 +1959,8 @@ int batch_prepare(BatchImpl<T>& B, int use_graph) {
     for (auto* D : B.doms) {
       D->first = false;
       D->rot_valid = true;
-      if ((rc = on_stream(*D, B.stream, launch_diag<T>))) return rc;
     }
+    if ((rc = batch_integrals(B, false))) return rc;
   }
   if (use_graph && !B.exec) {
     UMWM_HIP_TRY(hipStreamBeginCapture(B.stream, hipStreamCaptureModeThreadLocal));
@@ -1996,11 +2029,8 @@ int batch_run_dtg_impl(BatchImpl<T>& B, int use_graph, int32_t* nsub) {
     if (total > 10000000) return fail(UMWM_ERR_STATE, "batch run_dtg: substep count runaway");
     chunk = std::min(chunk * 2, 32);
   }
-  for (auto* D : B.doms) {
-    if (D->firstdtg) D->firstdtg = false;
-    if (D->S.P.stokes && (rc = on_stream(*D, B.stream, launch_stokes<T>))) return rc;
-    if ((rc = on_stream(*D, B.stream, launch_diag<T>))) return rc;
-  }
+  for (auto* D : B.doms) D->firstdtg = false;
+  if ((rc = batch_integrals(B, true))) return rc;
   UMWM_HIP_TRY(hipStreamSynchronize(B.stream));
   if (nsub)
     for (int k = 0; k < n; ++k) nsub[k] = B.h_view[k].nsub;

@@ -57,6 +57,11 @@ struct Scalars {
   int32_t sur_closed, sur_pad;
 };
 
+// Planes of DomainDev::sp: x and y stress partials; FP32 keeps the wave
+// height's own sum beside them (FP64 reads it from the zeroth moment).
+template <typename T>
+constexpr int kPartials = sizeof(T) == 4 ? 3 : 2;
+
 // Everything a kernel needs to know about one domain.
 template <typename T>
 struct DomainDev {
@@ -108,16 +113,16 @@ struct DomainDev {
   double *us1, *vs1;  // surface Stokes drift used by stress('atm')
   // fused-path copy of the (o, j) tables, [om][ldi][FT_N]: the FT_N values
   // of one (frequency, point) are contiguous, so a lane fetches them with a
-  // few 16-byte loads and a wave reads one contiguous span; the directional
-  // moments of e and the x stress partial, [om][ldi][4] (m0, mc, ms, x), and
-  // the y stress partial, [om][ldi], all written by k_advect; per point the
-  // bits of the largest rate while k_rates' workgroups of it collect it;
-  // FP64 only, dth/2 times the exclusive frequency prefix of the moments,
-  // [om][ldi][4] (3 used), from k_rates to k_integrate
+  // few 16-byte loads and a wave reads one contiguous span; as planes, the
+  // directional moments of e in FP64, [om][3][ldi], and the stress partials
+  // with (FP32) the share of the wave height, [om][kPartials][ldi], all
+  // written by k_advect; dth/2 times the exclusive frequency prefix of the
+  // moments, [om][3][ldi], from k_rates to k_integrate; per point the bits of
+  // the largest rate while k_rates' workgroups of it collect it
   T* ftab;
+  double* mom;
+  T* sp;
   T* pfx;
-  T* mom;
-  T* sty;
   unsigned long long* rkey;
   Scalars* sc;
   // learned surrogate of the FP32 path (null sur_r: none attached): the
@@ -181,6 +186,12 @@ inline const char* const* ocn_field_names() {
 struct StokesDev {
   const double* depth;  // lm levels, negative down
   double *us, *vs, *ds; // us/vs [l][ldi]
+};
+
+// Outputs of the spectral integrals of one domain (integrals.hip).
+struct EndDev {
+  DiagDev diag;
+  StokesDev stokes;
 };
 
 // Forcing levels kept on the device (src/umwm_forcing.F90:11-99).

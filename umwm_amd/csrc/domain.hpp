@@ -86,7 +86,7 @@ struct DomainImpl : DomainBase {
   int32_t* list0 = nullptr;
   // umwm_hip_substeps_noalloc: the device's shared scratch array (from
   // hipGetSymbolAddress at creation) and a second device copy of the domain
-  // record whose pfx and sty point into it, with its host image
+  // record whose pfx and sp point into it, with its host image
   unsigned char* scr = nullptr;
   DomainDev<T>* d_scr = nullptr;
   DomainDev<T> h_scr{};
@@ -99,9 +99,9 @@ struct DomainImpl : DomainBase {
   hipGraphExec_t gexec = nullptr;
   uint64_t gsig = 0;
   bool use_graph = true;
-  DiagDev diag{};
+  EndDev end{};              // diag and Stokes outputs
+  EndDev* end_d = nullptr;   // device copy (array of one)
   OcnDev ocn{};  // allocated with the operator arrays
-  StokesDev stokes{};
   BlockTask* tasks = nullptr;
   int ntasks = 0;
   Tile tile;
@@ -132,10 +132,14 @@ template <typename T> int launch_op_refraction(DomainImpl<T>& D);
 template <typename T> int launch_op_update(DomainImpl<T>& D);
 template <typename T> int launch_op_stress_atm(DomainImpl<T>& D);
 template <typename T> int launch_op_stress_ocn(DomainImpl<T>& D);
-template <typename T> int launch_diag(DomainImpl<T>& D);
-template <typename T> int launch_stokes(DomainImpl<T>& D);
 template <typename T> int launch_hs_ice(DomainImpl<T>& D);
 template <typename T> int launch_jonswap(DomainImpl<T>& D, const umwm_jonswap& js);
+
+// stokes_drift and/or diag of the domains of a task list, in one pass over
+// the spectra; lm is the largest level count among them.
+template <typename T>
+int launch_integrals(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks,
+                     const EndDev* ends, int lm, bool stokes, bool diag, hipStream_t s);
 
 // Forcing interpolation of the n domains list[0..n) (indices into doms and
 // fds) in one launch, plus the reset of their anycur flags when any has

@@ -255,7 +255,7 @@ struct TabGen {
   size_t ldi;
   uint32_t vj;
   int om;
-  float dep, sgr, sbf, sbp, s1, s2, l2z, lz, sp4, tpsf;
+  float dep, sgr, sbf, sbp, s1, s2, l2z, lz;
   float k0, k1, k2, kn;   // k(o), k(o+1), k(o+2), k(o+3) (loaded ahead)
   float kdk0, kdk1, kdk2;
 
@@ -291,8 +291,6 @@ struct TabGen {
     s2 = float(d.snl_fac * d.bf2);
     lz = float(log(d.z));
     l2z = float(log(20.0 / d.z));
-    sp4 = float(4 * d.sds_power);
-    tpsf = float(d.twopisds_fac);
     k0 = load_k(o0);
     k1 = load_k(o0 + 1);
     k2 = load_k(o0 + 2);
@@ -318,7 +316,7 @@ struct TabGen {
     r.v[FT_LOGL2] = l2 > 20.f ? l2z : 0.6931471805599453f * __builtin_amdgcn_logf(l2) - lz;
     const float coth = (1.f + w) * __builtin_amdgcn_rcpf(1.f - w);
     r.v[FT_COTH] = coth;
-    r.v[FT_L] = sp4 * __builtin_amdgcn_logf(k) + __builtin_amdgcn_logf(tpsf * fo * coth);
+    r.v[FT_L] = 0.f;  // FP64 only
     r.v[FT_SBF] = sbf * k * isinh2 + sbp * k * __builtin_amdgcn_rcpf(ch * ch);
     r.v[FT_K] = k;
     r.v[FT_CG0] = cp * (0.5f + k * dep * isinh2 + sk2 * __builtin_amdgcn_rcpf(1.f + sk2));
@@ -415,19 +413,16 @@ __device__ __forceinline__ T sin_m(const SinFreq<T>& q, T y, T m) {
 // ---------------------------------------------------------------------
 // Directional moments of E^n, the raw material of the sds prefix: per
 // (frequency, point) the sums over the directions of e, e cos 2th and
-// e sin 2th, [om][ldi][4] (the fourth value is the x stress partial).
-// k_advect forms them from the spectrum it writes, so the sweeps need no
-// exchange between the waves of a point and may be split over directions
-// and frequencies freely; k_moments forms them after anything else wrote
-// the spectrum.  The order of the sums does not depend on the launch: four
-// consecutive directions in the working precision, these quads in FP64 over
-// the pm / kSegs directions of a segment, the segments in FP64.
+// e sin 2th in FP64, planes [om][3][ldi].  k_advect forms them from the spectrum it writes, so the sweeps
+// need no exchange between the waves of a point and may be split over
+// directions and frequencies freely; k_moments forms them after anything else
+// wrote the spectrum.  The order of the sums does not depend on the launch:
+// the directions of a group in the working precision, the groups in FP64.
 // ---------------------------------------------------------------------
-// Segments of the directional sums: the largest divisor of pm / 4 up to 8.
-__host__ __device__ inline int dir_segments(int pm) {
-  int n = 8;
-  while ((pm / 4) % n) --n;
-  return n;
+// Direction groups of the sums: the fewest of up to 9 (18, 36 for wide
+// spectra) directions, as evenly as they divide.
+__host__ __device__ inline int dir_groups(int pm) {
+  return pm <= 72 ? (pm + 8) / 9 : pm <= 144 ? (pm + 17) / 18 : (pm + 35) / 36;
 }
 
 template <typename T>
@@ -435,51 +430,55 @@ struct Mom {
   T m0, mc, ms;
 };
 
+// Three planes of frequency o at point j: the moments, or dth/2 times their
+// prefix (DomainDev::pfx).
 template <typename T>
 __device__ __forceinline__ Mom<T> load_mom(const T* mom, size_t ldi, int o, int j) {
-  const rsrc_t pf = freq_rsrc(mom, o, 4, ldi);
-  Mom<T> r;
-  if constexpr (sizeof(T) == 4) {
-    const auto v = bld16<T>(pf, (uint32_t)j * 16u);
-    r.m0 = v[0];
-    r.mc = v[1];
-    r.ms = v[2];
-  } else {
-    const auto v = bld16<T>(pf, (uint32_t)j * 32u);
-    r.m0 = v[0];
-    r.mc = v[1];
-    r.ms = bld<T>(pf, (uint32_t)j * 32u + 16u);
-  }
-  return r;
+  const rsrc_t pf = row_rsrc(mom, (size_t)o, 3 * ldi);
+  const uint32_t v = (uint32_t)j * (uint32_t)sizeof(T), pl = (uint32_t)ldi * (uint32_t)sizeof(T);
+  return Mom<T>{bld<T>(pf, v), bld<T>(pf, v, pl), bld<T>(pf, v, 2 * pl)};
 }
 
 // Running prefix of the moments over frequency, sum_{o' < o} k^3 dk m(o'),
 // in FP64 (src/umwm_source_functions.F90:92-97).
 struct Prefix {
   double a0 = 0, ac = 0, as = 0;
-  template <typename T>
-  __device__ __forceinline__ void add(T k3dk, const Mom<T>& m) {
-    const double k3 = k3dk;
-    a0 += k3 * (double)m.m0;
-    ac += k3 * (double)m.mc;
-    as += k3 * (double)m.ms;
+  __device__ __forceinline__ void add(double k3, const Mom<double>& m) {
+    a0 += k3 * m.m0;
+    ac += k3 * m.mc;
+    as += k3 * m.ms;
   }
 };
 
-// In FP64 k_rates stores dth/2 times the prefix ([om][ldi][4], 3 used) for
-// k_integrate, which has no registers left for the running sums (keeping
-// them there spilled: 155 -> 350 us on 2,852 points); in FP32 k_integrate
-// forms its own and the 8 values of traffic per (frequency, point) are saved.
+// Whether k_rates leaves the prefix for k_integrate or k_integrate sums it
+// again: in FP64 that spilled (155 -> 350 us at 2,852 points) and in the
+// surrogate's variant it cost a tenth (968 -> 1,064 us at 129,000 points x
+// 49x72); in plain FP32 the store costs k_rates more than k_integrate saves
+// (256 + 427 against 301 + 415 us at 179,776 points).
+template <typename T, bool SUR>
+constexpr bool kStoredPrefix = sizeof(T) == 8 || SUR;
+
+// k^3 dk of (o, j): FP64 reads the table, FP32 forms it from k as the sweeps
+// do (TabGen).
 template <typename T>
-constexpr bool kStoredPrefix = sizeof(T) == 8;
+__device__ __forceinline__ double k3dk_at(const DomainDev<T>& d, const TabGen& tg, int o,
+                                          uint32_t vj) {
+  if constexpr (sizeof(T) == 4) {
+    const float k = tg.load_k(o);
+    return k * k * tg.kdk_of(k, o);
+  } else {
+    return bld<T>(row_rsrc(d.k3dk, o, (size_t)d.ldi), vj);
+  }
+}
 
 // The prefix at frequency o0 of a sweep that starts there.
 template <typename T>
-__device__ __forceinline__ Prefix prefix_at(const DomainDev<T>& d, int o0, int j, uint32_t vj) {
+__device__ __forceinline__ Prefix prefix_at(const DomainDev<T>& d, const TabGen& tg, int o0, int j,
+                                            uint32_t vj) {
   Prefix P;
 #pragma unroll 4
   for (int o = 0; o < o0; ++o)
-    P.add(bld<T>(row_rsrc(d.k3dk, o, (size_t)d.ldi), vj), load_mom(d.mom, d.ldi, o, j));
+    P.add(k3dk_at(d, tg, o, vj), load_mom(d.mom, d.ldi, o, j));
   return P;
 }
 
@@ -528,8 +527,7 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
   // opaque to the compiler, which would otherwise reload these pointers
   // from the domain record after every store.
   const T* const eb = d.e;
-  const T* const momb = d.mom;
-  const T* const k3b = d.k3dk;
+  const double* const momb = d.mom;
   [[maybe_unused]] T* const pfxb = d.pfx;
   const T* const ftab = d.ftab;
   const T* const fr = d.f;
@@ -540,9 +538,8 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
     const PointState<T> s = point_fresh(d, j, valid && slot == 0);
     const int oc = s.oc;
     const int ocmax = wave_max_i32(valid ? oc : -1);
-    const bool anyice = __any(valid && s.ice != T(0));
-    // cg0, which the FP64 record leaves out: only ice attenuation needs it
-    auto ice_cg0 = [&](int o) { return bld<T>(row_rsrc(d.cg0, o, ldi), vj); };
+    // cg0 is not in the FP64 record: only ice attenuation needs it
+    [[maybe_unused]] const bool anyice = __any(valid && s.ice != T(0));
     if (rotation && valid && slot == 0) pstore(d.oc_rot, ldi, j, (int32_t)oc);
     uint32_t vie = 0, viw = 0, vin = 0, vis = 0;
     T dvc = 0, duc = 0, odx = 0, ody = 0;
@@ -557,6 +554,7 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
       ody = pload(d.oneovdy, ldi, j);
     }
     const T sin_diss1 = T(d.sin_fac * d.fieldscale1), fs2 = T(d.fieldscale2);
+    [[maybe_unused]] const T tpsf = T(d.twopisds_fac);
     const T spow = T(d.sds_power), mssf = T(d.mss_fac);
     const T nu4 = T(4 * d.nu_water), ig = T(1 / d.g);
     const double hdth = 0.5 * d.dth;
@@ -628,15 +626,20 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
     // wave's points there is nothing to evaluate (16 of 37 frequencies at
     // 15 m/s) unless the network's share of the energy is being measured
     const int omain = ds ? o1 : min(o1, ocmax + 1);
-    Prefix P = prefix_at(d, o0, j, vj);
+    // FP32 derives the tables from k (TabGen); FP64 loads the record
+    constexpr bool kDerive = sizeof(T) == 4;
+    TabGen tg;
+    if constexpr (kDerive) tg.init(d, j, vj, o0);
+    Prefix P = prefix_at(d, tg, o0, j, vj);
     T ec[DMAX];
     // the network's dm^2 - 1 of this and the next frequency as raw bf16
     // bits; the direction's row offset joins the lane offset (a vector add)
     // rather than holding DMAX more scalar registers
     [[maybe_unused]] uint32_t rc[DMAX];
     FreqTab<T> tc;
-    Mom<T> mo = load_mom(momb, ldi, o0, j);
-    T k3 = bld<T>(row_rsrc(k3b, o0, ldi), vj);
+    Mom<double> mo = load_mom(momb, ldi, o0, j);
+    [[maybe_unused]] double k3 = 0;
+    if constexpr (!kDerive) k3 = k3dk_at(d, tg, o0, vj);
     {
       const rsrc_t ep = freq_rsrc(eb, o0, pm, ldi);
 #pragma unroll
@@ -649,16 +652,13 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
         }
       }
     }
-    // FP32 derives the tables from k (TabGen); FP64 loads the record
-    constexpr bool kDerive = sizeof(T) == 4;
-    TabGen tg;
-    if constexpr (kDerive) tg.init(d, j, vj, o0);
     auto store_prefix = [&](int o, T pa0, T pac, T pas) {
-      if constexpr (kStoredPrefix<T>) {
+      if constexpr (kStoredPrefix<T, SUR>) {
         if (valid && grp == 0) {
-          const rsrc_t pf = freq_rsrc(pfxb, o, 4, ldi);
-          bst16(pf, (uint32_t)j * 32u, typename Vec16<T>::type{pa0, pac});
-          bst(pf, (uint32_t)j * 32u + 16u, pas);
+          const rsrc_t pf = freq_rsrc(pfxb, o, 3, ldi);
+          bst(pf, vj, pa0);
+          bst(pf, vj, pac, rb);
+          bst(pf, vj, pas, 2 * rb);
         }
       }
     };
@@ -677,8 +677,9 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
           for (int q = 0; q < DMAX; ++q) rn[q] = bld_u16(FULL || q < nd ? rp : rz, vj2 + dirp(q) * rb2);
         }
       }
-      const Mom<T> mn = load_mom(momb, ldi, on, j);
-      const T k3n = bld<T>(row_rsrc(k3b, on, ldi), vj);
+      const Mom<double> mn = load_mom(momb, ldi, on, j);
+      [[maybe_unused]] double k3n = 0;
+      if constexpr (!kDerive) k3n = k3dk_at(d, tg, on, vj);
       float knext = 0.f;
       if constexpr (kDerive) {
         knext = tg.load_k(o + 4);
@@ -687,14 +688,28 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
         load_tab<kSweepSlots>(ftab, ldi, o, vr, tc);
       }
 
-      const T k = tc[FT_K], fo = cld(fr, o);
-      T crest = tc[FT_SBF] + s.csdt * k + nu4 * (k * k);  // sbf + sdt + sdv - sice
-      if (anyice) crest -= T(2) * s.ice * ice_cg0(o);
+      const T k = tc[FT_K], k2 = k * k, fo = cld(fr, o);
+      const T sdt = s.csdt * k;
+      T crest;  // sbf + sdt + sdv - sice
+      if constexpr (kDerive) {
+        const T sice = T(2) * tc[FT_CG0] * s.ice;
+        crest = tc[FT_SBF] + sdt + nu4 * k2 - sice;
+        k3 = k2 * tc[FT_KDK];
+      } else {
+        crest = tc[FT_SBF] + sdt + nu4 * k2;
+        if (anyice) crest -= T(2) * s.ice * bld<T>(row_rsrc(d.cg0, o, ldi), vj);
+      }
       const SinFreq<T> sf = sin_freq(s, tc[FT_LOGL2], tc[FT_CP0], fo * k * ig, sin_diss1, fs2);
       const T pa0 = T(hdth * P.a0), pac = T(hdth * P.ac), pas = T(hdth * P.as);
       store_prefix(o, pa0, pac, pas);
       // sds (after cothkd) = cf coth dm^2 (e k4)^p = dm^2 ex(p lg e + Lk)
-      const T Lk = tc[FT_L];  // lg(cf coth k^(4 p))
+      T Lk;  // lg(cf coth k^(4 p)), in the FP64 record
+      if constexpr (kDerive) {
+        const T cfo = tpsf * fo * tc[FT_COTH];
+        Lk = T(4) * spow * Tr<T>::lg_nn(k) + Tr<T>::lg_nn(cfo);  // lg(k^4) = 4 lg k
+      } else {
+        Lk = tc[FT_L];
+      }
       const T cs = T(1) - (tc[FT_B1] + tc[FT_B2]);                // snl_arg
       const T q0 = T(1) + mssf * pa0, qc = mssf * pac, qs = mssf * pas;
       [[maybe_unused]] const T kdkv = tc[FT_KDK];
@@ -791,7 +806,7 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
       }
       P.add(k3, mo);
       mo = mn;
-      k3 = k3n;
+      if constexpr (!kDerive) k3 = k3n;
 #pragma unroll
       for (int q = 0; q < DMAX; ++q) ec[q] = en[q];
       if constexpr (SUR) {
@@ -802,12 +817,13 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
       }
       if constexpr (kDerive) tg.advance(o, knext);
     }
-    if constexpr (kStoredPrefix<T>) {
+    if constexpr (kStoredPrefix<T, SUR>) {
       // the prefix of the diagnostic tail's bins, for k_integrate
       if (grp == 0) {
+#pragma unroll 4
         for (int o = max(o0, omain); o < o1; ++o) {
           store_prefix(o, T(hdth * P.a0), T(hdth * P.ac), T(hdth * P.as));
-          P.add(bld<T>(row_rsrc(k3b, o, ldi), vj), load_mom(momb, ldi, o, j));
+          P.add(k3dk_at(d, tg, o, vj), load_mom(momb, ldi, o, j));
         }
       }
     }
@@ -998,15 +1014,16 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
   const T* const eb = d.e;
   T* const esb = d.es;
   const T* const ftab = d.ftab;
-  [[maybe_unused]] const T* const momb = d.mom;
-  [[maybe_unused]] const T* const k3b = d.k3dk;
+  constexpr bool kStored = kStoredPrefix<T, SUR>, kRegDirs = sizeof(T) == 4;
+  [[maybe_unused]] const double* const momb = d.mom;
   [[maybe_unused]] const T* const pfxb = d.pfx;
   const T* const fr = d.f;
 
   const PointState<T> s = point_stored(d, j);
   const int oc = s.oc;
-  const bool anyice = __any(valid && s.ice != T(0));
+  [[maybe_unused]] const bool anyice = __any(valid && s.ice != T(0));
   const T sin_diss1 = T(d.sin_fac * d.fieldscale1), fs2 = T(d.fieldscale2);
+  [[maybe_unused]] const T tpsf = T(d.twopisds_fac);
   const T spow = T(d.sds_power), ipow = T(d.inv_sds_power);
   const T mssf = T(d.mss_fac), dsnl = dts * T(d.snl_fac);
   const T nu4 = T(4 * d.nu_water), ig = T(1 / d.g);
@@ -1016,15 +1033,23 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
   // direction loop has no per-slot branch and the compiler can interleave
   // the directions.
   const rsrc_t rz = make_rsrc(eb, 0u);
-  // wind overrunning a direction (fieldscale2, see sin_m) as bits of mb, and
-  // the direction records re-read per frequency: both in registers cost
-  // k_integrate a wave per SIMD in FP64
-  uint32_t mb = 0;
+  // direction constants of this wave.  FP32 keeps them in registers; in FP64
+  // that cost a wave per SIMD, so it keeps the overrun factors (fieldscale2,
+  // see sin_m) as bits of mb and re-reads the direction records per frequency
+  [[maybe_unused]] uint32_t mb = 0;
+  [[maybe_unused]] T mq[DMAX], ctq[DMAX], stq[DMAX];
 #pragma unroll
   for (int q = 0; q < DMAX; ++q) {
     T ct, st, c2, s2;
     cld4(d.dir4, p0 + q, ct, st, c2, s2);
-    if (s.cw * ct + s.sw * st > T(0)) mb |= 1u << q;
+    const bool over = s.cw * ct + s.sw * st > T(0);
+    if constexpr (kRegDirs) {
+      mq[q] = over ? fs2 : T(1);
+      ctq[q] = ct;
+      stq[q] = st;
+    } else {
+      if (over) mb |= 1u << q;
+    }
   }
   const T* const dir4 = d.dir4;
   // per direction, the partial E* = (E^n + partial E_s) / 2 of the two
@@ -1067,13 +1092,16 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
   constexpr bool kDerive = sizeof(T) == 4;
   TabGen tg;
   if constexpr (kDerive) tg.init(d, j, vj, o0);
+  // the stored prefix (prefetched in FP32, loaded when needed in FP64) or
+  // the moments it is summed from
+  [[maybe_unused]] Mom<T> pc{};
   [[maybe_unused]] Prefix P;
-  [[maybe_unused]] Mom<T> mo{};
-  [[maybe_unused]] T k3 = 0;
-  if constexpr (!kStoredPrefix<T>) {
-    P = prefix_at(d, o0, j, vj);
+  [[maybe_unused]] Mom<double> mo{};
+  if constexpr (!kStored) {
+    P = prefix_at(d, tg, o0, j, vj);
     mo = load_mom(momb, ldi, o0, j);
-    k3 = bld<T>(row_rsrc(k3b, o0, ldi), vj);
+  } else if constexpr (kDerive) {
+    pc = load_mom(pfxb, ldi, o0, j);
   }
   const int oend = min(om, o1 + 2);
   for (int o = o0; o < oend; ++o) {
@@ -1090,37 +1118,56 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
         for (int q = 0; q < DMAX; ++q) rn[q] = bld_u16(FULL || q < nd ? rp : rz, vj2 + (p0 + q) * rb2);
       }
     }
-    [[maybe_unused]] Mom<T> mn{};
-    [[maybe_unused]] T k3n = 0;
+    [[maybe_unused]] Mom<T> pn{};
+    [[maybe_unused]] Mom<double> mn{};
     float knext = 0.f;
-    T pa0, pac, pas;  // dth/2 times the prefix moments
     if constexpr (kDerive) {
       knext = tg.load_k(o + 4);
+      if constexpr (kStored)
+        pn = load_mom(pfxb, ldi, on, j);
+      else
+        mn = load_mom(momb, ldi, on, j);
       tg.table(o, tc);
     } else {
       load_tab<kSweepSlots>(ftab, ldi, o, vr, tc);
+      pc = load_mom(pfxb, ldi, o, j);
     }
-    if constexpr (kStoredPrefix<T>) {
-      const Mom<T> pc = load_mom(pfxb, ldi, o, j);
-      pa0 = pc.m0;
-      pac = pc.mc;
-      pas = pc.ms;
-    } else {
-      mn = load_mom(momb, ldi, on, j);
-      k3n = bld<T>(row_rsrc(k3b, on, ldi), vj);
+    if constexpr (!kStored) {
       const double hdth = 0.5 * d.dth;
-      pa0 = T(hdth * P.a0);
-      pac = T(hdth * P.ac);
-      pas = T(hdth * P.as);
+      pc = Mom<T>{T(hdth * P.a0), T(hdth * P.ac), T(hdth * P.as)};
     }
+    const T pa0 = pc.m0, pac = pc.mc, pas = pc.ms;
 
     const T k = tc[FT_K], fo = cld(fr, o);
-    T ctail = s.csdt * k + nu4 * (k * k);  // sdt + sdv - sice
-    if (anyice) ctail -= T(2) * s.ice * bld<T>(row_rsrc(d.cg0, o, ldi), vj);
+    const T sdt = s.csdt * k;
+    T ctail;  // sdt + sdv - sice
+    if constexpr (kDerive) {
+      const T sice = T(2) * tc[FT_CG0] * s.ice;
+      ctail = sdt + nu4 * (k * k) - sice;
+    } else {
+      ctail = sdt + nu4 * (k * k);
+      if (anyice) ctail -= T(2) * s.ice * bld<T>(row_rsrc(d.cg0, o, ldi), vj);
+    }
+    const T crest = tc[FT_SBF] + ctail;
     const SinFreq<T> sf = sin_freq(s, tc[FT_LOGL2], tc[FT_CP0], fo * k * ig, sin_diss1, fs2);
-    const T Lk = tc[FT_L];  // lg(cf coth k^(4 p)): sds after cothkd
-    const T c0 = -dtx * (tc[FT_SBF] + ctail);
-    const T icoth = Tr<T>::rcp(tc[FT_COTH]);  // X is sds e before cothkd
+    // FP32 forms sds before cothkd; FP64 takes lg(cf coth k^(4 p)) from its
+    // record, so its sds and X are after cothkd and the snl weights carry
+    // icx = 1 / cothkd instead
+    T Lk, dtc, icx = T(1);
+    [[maybe_unused]] T icfc = 0, lk4 = 0;
+    if constexpr (kDerive) {
+      const T cf = tpsf * fo;
+      const T coth = tc[FT_COTH];
+      lk4 = T(4) * Tr<T>::lg(k);          // lg(k^4)
+      Lk = spow * lk4 + Tr<T>::lg(cf);
+      dtc = dtx * coth;
+      icfc = Tr<T>::rcp(cf * coth);
+    } else {
+      Lk = tc[FT_L];
+      dtc = dtx;
+      icx = Tr<T>::rcp(tc[FT_COTH]);
+    }
+    const T c0 = -dtx * crest;
     // the spreading factor's upper bound, from the zeroth-moment prefix
     [[maybe_unused]] const T qhi = (T(1) + T(2) * mssf * pa0) * (T(1) + T(2) * mssf * pa0);
     // dm = q0 + qc cos 2th + qs sin 2th = (q0 - qc) + ct (2 qc ct + 2 qs st),
@@ -1132,8 +1179,12 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
     const bool prog = o <= oc;
     const bool in1 = (o >= 1) && (o - 1 <= oc);  // bin o-1 is prognostic
     const bool fin = valid && (o >= o0 + 2) && (o - 2 <= oc);  // bin o-2 completes now
-    const T hdb1 = in1 ? T(0.5) * dts * b1m1 * icoth : T(0), hdb2 = T(0.5) * dts * b2m2 * icoth;
-    const T dsc = dsnl * icoth;
+    T hdb1 = in1 ? T(0.5) * dts * b1m1 : T(0), hdb2 = T(0.5) * dts * b2m2, dsc = dsnl;
+    if constexpr (!kDerive) {
+      hdb1 *= icx;
+      hdb2 *= icx;
+      dsc *= icx;
+    }
     const uint32_t vtail = (valid && !prog && own) ? vj : kDropOffset;
     const uint32_t vfin = fin ? vj : kDropOffset;
     const bool anyfin = __any(fin), anytail = own && __any(valid && !prog);
@@ -1155,35 +1206,47 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
 #pragma unroll
       for (int q = 0; q < DMAX; ++q) {
         const uint32_t so = (uint32_t)(p0 + q) * rb;
-        T ct, st, c2, s2;
-        cld4(dir4, p0 + q + dz, ct, st, c2, s2);
         const T e = ec[q];
-        const T y = sin_y(sf, ct, st);
-        const T pos = sf.pos, neg1 = sf.neg1, neg2 = sf.neg2;  // see sin_bin
-        const T neg = ((mbl >> q) & 1) ? neg2 : neg1;
-        const T ss = y * (y > T(0) ? pos : neg);
+        T ct, st, ss;
+        if constexpr (kRegDirs) {
+          ct = ctq[q];
+          st = stq[q];
+          ss = sin_m(sf, sin_y(sf, ct, st), mq[q]);
+        } else {
+          T c2, s2;
+          cld4(dir4, p0 + q + dz, ct, st, c2, s2);
+          const T y = sin_y(sf, ct, st);
+          const T pos = sf.pos, neg1 = sf.neg1, neg2 = sf.neg2;  // see sin_bin
+          const T neg = ((mbl >> q) & 1) ? neg2 : neg1;
+          ss = y * (y > T(0) ? pos : neg);
+        }
         T dm = fma(ct, fma(qc2, ct, qs2 * st), q0m);
         dm = dm * dm;
         if constexpr (SUR) {
           if (do_sur && use) dm = fmin(fmax(T(1) + bf16_bits_to_f(rc[q]), T(1)), qhi);  // dm^2 - 1
         }
-        T X = 0, G = 0;  // X: sds e (after cothkd)
+        T X = 0, G = 0;  // X: sds e
         if constexpr (decltype(NEEDX)::value) {
           // |e|: see k_rates; a NaN of e stays in X through e
           const T sds = dm * Tr<T>::ex_nn(fma(spow, Tr<T>::lg_nn(fabs(e)), Lk));
           X = sds * e;
           if constexpr (decltype(PROG)::value) {
             // E_s = e exp(dts (ssin - sds - sbf - sdt - sdv + sice)) + dts snl
-            const T a = fma(-dtx, sds, fma(dtx, ss, c0));
+            const T a = fma(-dtc, sds, fma(dtx, ss, c0));
             G = prog ? fma(-dsc, X, e * Tr<T>::ex(a)) : T(0);
           }
         }
         if constexpr (decltype(TAIL)::value) {
-          // diagnostic tail, src/umwm_physics.F90:70-80: k^-4 (num / (cf
-          // coth dm^2))^(1/p) = ex((lg(num / dm^2) - Lk) / p)
+          // diagnostic tail, src/umwm_physics.F90:70-80: k^-4 t^(1/p), t =
+          // num / (cf coth dm^2); in FP64 ex((lg(num / dm^2) - Lk) / p)
           const T num = fmax(ss, T(0)) - ctail;
-          const T t = fmax(num, T(0)) * Tr<T>::rcp(dm);
-          const T es_ = Tr<T>::ex(ipow * (Tr<T>::lg(t) - Lk));
+          T es_;
+          if constexpr (kDerive) {
+            const T t = fmax(num, T(0)) * (icfc * Tr<T>::rcp(dm));
+            es_ = Tr<T>::ex(fma(ipow, Tr<T>::lg(t), -lk4));
+          } else {
+            es_ = Tr<T>::ex(ipow * (Tr<T>::lg(fmax(num, T(0)) * Tr<T>::rcp(dm)) - Lk));
+          }
           bst(FULL || q < nd ? rs0 : rz, vtail, T(0.5) * (e + es_), so);
         }
         T h1 = H1[q];
@@ -1219,12 +1282,15 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
         for (int q = 0; q < DMAX; ++q) rc[q] = rn[q];
       }
     }
-    if constexpr (!kStoredPrefix<T>) {
+    if constexpr (!kStored) {
+      const double k3 = k * k * tc[FT_KDK];  // k^3 dk
       P.add(k3, mo);
       mo = mn;
-      k3 = k3n;
     }
-    if constexpr (kDerive) tg.advance(o, knext);
+    if constexpr (kDerive) {
+      tg.advance(o, knext);
+      if constexpr (kStored) pc = pn;
+    }
   }
 }
 
@@ -1248,16 +1314,20 @@ struct AdvLoads {
 };
 
 // Sums over the directions in the order of the moments (see Mom): `add`
-// takes directions in sequence, `quad` ends a group of four, `seg` a segment.
-template <typename T>
+// takes directions in sequence, `group` ends a group.  t: e, e cos 2th,
+// e sin 2th and the stress partials; kSeq (FP32 where a wave takes every
+// direction) keeps the stress partials and the wave height as one running
+// FP32 sum each.
+template <typename T, bool kSeq>
 struct DirSums {
-  T q[5];
-  double s[5], t[5];
+  T q[5], hs;
+  double t[5];
   __device__ __forceinline__ void clear() {
+    hs = 0;
 #pragma unroll
     for (int i = 0; i < 5; ++i) {
       q[i] = 0;
-      s[i] = t[i] = 0;
+      t[i] = 0;
     }
   }
   // e, and its wind input in the stress partials
@@ -1267,36 +1337,27 @@ struct DirSums {
     q[2] = fma(v, s2, q[2]);
     q[3] = fma(wv, ct, q[3]);
     q[4] = fma(wv, st, q[4]);
+    if constexpr (kSeq) hs += v;
   }
-  template <int N>
-  __device__ __forceinline__ void quad() {
+  __device__ __forceinline__ void group() {
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      s[i] += (double)q[i];
+    for (int i = 0; i < (kSeq ? 3 : 5); ++i) {
+      t[i] += (double)q[i];
       q[i] = 0;
-    }
-  }
-  template <int N>
-  __device__ __forceinline__ void seg() {
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      t[i] += s[i];
-      s[i] = 0;
     }
   }
 };
 
-// Stores the moments and the x stress partial of (o, j).
+// Stores the moments of (o, j), and the stress partials and (FP32) the
+// frequency's share of the wave height, e dk, as planes of sp.
 template <typename T>
-__device__ __forceinline__ void store_mom(T* mom, size_t ldi, int o, int j, T m0, T mc, T ms,
-                                          T tx) {
-  const rsrc_t sp = freq_rsrc(mom, o, 4, ldi);
-  if constexpr (sizeof(T) == 4) {
-    bst16(sp, (uint32_t)j * 16u, f32x4{m0, mc, ms, tx});
-  } else {
-    bst16(sp, (uint32_t)j * 32u, f64x2{m0, mc});
-    bst16(sp, (uint32_t)j * 32u + 16u, f64x2{ms, tx});
-  }
+__device__ __forceinline__ void store_mom(const DomainDev<T>& d, int o, int j, double m0, double mc,
+                                          double ms) {
+  const rsrc_t r = row_rsrc(d.mom, (size_t)o, 3 * (size_t)d.ldi);
+  const uint32_t v = (uint32_t)j * 8u, pl = (uint32_t)d.ldi * 8u;
+  bst(r, v, m0);
+  bst(r, v, mc, pl);
+  bst(r, v, ms, 2 * pl);
 }
 
 // The moments of the current spectrum, after anything but k_advect wrote it;
@@ -1312,10 +1373,10 @@ __global__ __launch_bounds__(64) void k_moments(const DomainDev<T>* __restrict__
   const size_t ldi = d.ldi;
   const uint32_t vj = (uint32_t)j * (uint32_t)sizeof(T), rb = (uint32_t)ldi * (uint32_t)sizeof(T);
   const rsrc_t pe = freq_rsrc(d.e, o, pm, ldi);
-  const int seglen = pm / dir_segments(pm);
-  DirSums<T> S;
+  const int ng = dir_groups(pm), glen = uniform_div(pm + ng - 1, ng);
+  DirSums<T, true> S;
   S.clear();
-  int segend = seglen;
+  int gend = glen;
   for (int p = 0; p < pm; p += 4) {
     T v[4];
 #pragma unroll
@@ -1325,23 +1386,24 @@ __global__ __launch_bounds__(64) void k_moments(const DomainDev<T>* __restrict__
       T ct, st, c2, s2;
       cld4(d.dir4, p + q, ct, st, c2, s2);
       S.add(v[q], T(0), ct, st, c2, s2);
-    }
-    S.template quad<3>();
-    if (p + 4 == segend) {
-      S.template seg<3>();
-      segend += seglen;
+      if (p + q + 1 == gend) {
+        S.group();
+        gend += glen;
+      }
     }
   }
-  if (j < d.im) store_mom(d.mom, ldi, o, j, T(S.t[0]), T(S.t[1]), T(S.t[2]), T(0));
+  S.group();
+  if (j < d.im) store_mom(d, o, j, S.t[0], S.t[1], S.t[2]);
 }
 
 // SPLIT: one workgroup per (frequency, 64 sea points), a wave per direction
-// segment, for launches that would otherwise leave most of the GPU idle.
+// group, for launches that would otherwise leave most of the GPU idle.
 // Else fw = blockDim / 64 frequencies per workgroup, a wave taking all
-// directions of one.  Both give the same sums bit for bit.
+// directions of one.  Both give the same moments bit for bit, and in FP64 the
+// same stress partials.
 template <typename T, int NB, bool SPLIT>
 __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_advect(
-    const DomainDev<T>* __restrict__ doms, const BlockTask* __restrict__ tasks, int nseg) {
+    const DomainDev<T>* __restrict__ doms, const BlockTask* __restrict__ tasks, int ng) {
   const BlockTask tk = tasks[blockIdx.x];
   const DomainDev<T>& d = doms[tk.dom];
   const int wid = wave_id();
@@ -1392,13 +1454,14 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_advect(
   const T* const cthb = d.cth;
   const T* const sthb = d.sth;
   const T* const dir4 = d.dir4;
-  const int seglen = uniform_div(pm, nseg);
-  const int plo = SPLIT ? wid * seglen : 0, phi = SPLIT ? plo + seglen : pm;
+  const int glen = uniform_div(pm + ng - 1, ng);
+  const int plo = SPLIT ? wid * glen : 0, phi = SPLIT ? min(pm, plo + glen) : pm;
   // the moments of the new spectrum and the stress_vector_integral sums
   // over the directions of this frequency
-  DirSums<T> S;
+  constexpr bool kSeq = sizeof(T) == 4 && !SPLIT;
+  DirSums<T, kSeq> S;
   S.clear();
-  int segend = plo + seglen;
+  int gend = plo + glen;
   auto stress_acc = [&](int p, T v) {
     T ct, st, c2, s2;
     cld4(dir4, p, ct, st, c2, s2);
@@ -1406,12 +1469,9 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_advect(
     T ss = sin_m(sf, sin_y(sf, ct, st), m);
     if (!prog) ss = fmax(ss, T(0));
     S.add(v, v * ss, ct, st, c2, s2);
-  };
-  auto sums_end = [&](int pnext) {  // wave-uniform
-    if ((pnext & 3) == 0) S.template quad<5>();
-    if (pnext == segend) {
-      S.template seg<5>();
-      segend += seglen;
+    if (p + 1 == gend) {  // wave-uniform
+      S.group();
+      gend += glen;
     }
   };
   if (__all(!prog || !valid)) {
@@ -1419,14 +1479,16 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_advect(
     for (int pb = plo; pb < phi; pb += NB) {
       T v[NB];
 #pragma unroll
-      for (int q = 0; q < NB; ++q)
-        v[q] = fma(T(2), bld<T>(ps, vj, (pb + q) * rb), -bld_nt<T>(pe, vj, (pb + q) * rb));
+      for (int q = 0; q < NB; ++q) {
+        const int p = SPLIT && pb + q >= pm ? 0 : pb + q;
+        v[q] = fma(T(2), bld<T>(ps, vj, p * rb), -bld_nt<T>(pe, vj, p * rb));
+      }
 #pragma unroll
       for (int q = 0; q < NB; ++q) {
+        if (SPLIT && pb + q >= phi) break;  // a group of odd length
         bst_stream(pe, vst, v[q], (pb + q) * rb);
         stress_acc(pb + q, v[q]);
       }
-      sums_end(pb + NB);
     }
   } else {
     const int ie = pload(d.ie, ldi, j), iw = pload(d.iw, ldi, j);
@@ -1475,7 +1537,10 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_advect(
     auto load_block = [&](int pb, AdvLoads<T>* L) {
 #pragma unroll
       for (int q = 0; q < NB; ++q) {
-        const uint32_t so = (pb + q) * rb;
+        // past the last direction (a group of odd length) the first one, the
+        // periodic neighbour
+        const int p = SPLIT && pb + q >= pm ? 0 : pb + q;
+        const uint32_t so = p * rb;
         L[q].eo = bld<T>(ps, vj, so);
         L[q].ee = bld<T>(ps, vie, so);
         L[q].ew = bld<T>(ps, viw, so);
@@ -1497,6 +1562,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_advect(
 #pragma unroll
       for (int q = 0; q < NB; ++q) {
         const int p = pb + q;
+        if (SPLIT && p >= phi) break;  // a group of odd length
         const T enext = q + 1 < NB ? A[(q + 1) < NB ? q + 1 : 0].eo : (more ? B[0].eo : efirst);
         const int pn = p + 1 < pm ? p + 1 : 0;
         const T rnext = rotp(pn);
@@ -1523,9 +1589,9 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_advect(
       }
 #pragma unroll
       for (int q = 0; q < NB; ++q) A[q] = B[q];
-      sums_end(pb + NB);
     }
   }
+  S.group();  // the last group, where it is short
   if constexpr (SPLIT) {
     __shared__ double red[8][5][64];
     const int lane = (int)threadIdx.x & 63;
@@ -1533,14 +1599,27 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_advect(
     for (int i = 0; i < 5; ++i) red[wid][i][lane] = S.t[i];
     __syncthreads();
     if (wid != 0) return;
-    for (int q = 1; q < nseg; ++q)
+    for (int q = 1; q < ng; ++q)
 #pragma unroll
       for (int i = 0; i < 5; ++i) S.t[i] += red[q][i][lane];
   }
   if (valid) {
     const T icp = T(1) / cp_prev;
-    store_mom(d.mom, ldi, o, j, T(S.t[0]), T(S.t[1]), T(S.t[2]), T(S.t[3]) * icp);
-    bst(row_rsrc(d.sty, o, ldi), vj, T(S.t[4]) * icp);
+    T tx, ty, hs = 0;
+    if constexpr (kSeq) {
+      tx = S.q[3];
+      ty = S.q[4];
+      hs = S.hs * bld<T>(row_rsrc(d.kdk, o, ldi), vj);
+    } else {
+      tx = T(S.t[3]);
+      ty = T(S.t[4]);
+      if constexpr (sizeof(T) == 4) hs = T(S.t[0]) * bld<T>(row_rsrc(d.kdk, o, ldi), vj);
+    }
+    store_mom(d, o, j, S.t[0], S.t[1], S.t[2]);
+    const rsrc_t sp = freq_rsrc(d.sp, o, kPartials<T>, ldi);
+    bst(sp, vj, tx * icp);
+    bst(sp, vj, ty * icp, rb);
+    if constexpr (kPartials<T> == 3) bst(sp, vj, hs, 2 * rb);
   }
 }
 
@@ -1586,17 +1665,14 @@ __global__ __launch_bounds__(64) void k_stress(const DomainDev<T>* __restrict__ 
   double hs = 0;
   for (int o = 0; o < om; ++o) {
     const double kdk = bld<T>(row_rsrc(d.kdk, o, ldi), (uint32_t)j * E);
-    const rsrc_t sp = freq_rsrc(d.mom, o, 4, ldi);
-    double m0, tx;
-    if constexpr (sizeof(T) == 4) {
-      const f32x4 v = bld16<float>(sp, (uint32_t)j * 16u);
-      m0 = v[0];
-      tx = v[3];
-    } else {
-      m0 = bld<double>(sp, (uint32_t)j * 32u);
-      tx = bld<double>(sp, (uint32_t)j * 32u + 24u);
-    }
-    const double ty = bld<T>(row_rsrc(d.sty, o, ldi), (uint32_t)j * E);
+    const rsrc_t sp = freq_rsrc(d.sp, o, kPartials<T>, ldi);
+    const uint32_t vj = (uint32_t)j * E, rb = (uint32_t)ldi * E;
+    const double tx = bld<T>(sp, vj), ty = bld<T>(sp, vj, rb);
+    double hso;
+    if constexpr (kPartials<T> == 3)
+      hso = bld<T>(sp, vj, 2 * rb);
+    else
+      hso = bld<double>(row_rsrc(d.mom, (size_t)o, 3 * ldi), vj) * kdk;
     si.sx += tx * kdk;
     si.sy += ty * kdk;
     if (o >= oc) {
@@ -1607,7 +1683,7 @@ __global__ __launch_bounds__(64) void k_stress(const DomainDev<T>* __restrict__ 
       si.tomx = tx;
       si.tomy = ty;
     }
-    hs += m0 * kdk;
+    hs += hso;
   }
   si.wspd = w;
   si.wdir = pload(d.wdir, ldq, j);
@@ -1719,22 +1795,22 @@ int launch_kernels(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks,
 #undef UMWM_INTEGRATE
   if (keep) hipLaunchKernelGGL((k_keep<T>), dim3(ntasks), dim3(64), 0, s, doms, tasks);
   if (ev) (void)hipEventRecord(ev[2], s);
-  const int nseg = dir_segments(pm);
-  if (h.split && nseg > 1) {
-    const dim3 ga(ntasks, omax), block(64 * nseg);
+  const int ng = dir_groups(pm);
+  if (h.split && ng <= 8) {
+    const dim3 ga(ntasks, omax), block(64 * ng);
     if (nb == 4)
-      hipLaunchKernelGGL((k_advect<T, 4, true>), ga, block, 0, s, doms, tasks, nseg);
+      hipLaunchKernelGGL((k_advect<T, 4, true>), ga, block, 0, s, doms, tasks, ng);
     else
-      hipLaunchKernelGGL((k_advect<T, 2, true>), ga, block, 0, s, doms, tasks, nseg);
+      hipLaunchKernelGGL((k_advect<T, 2, true>), ga, block, 0, s, doms, tasks, ng);
   } else {
     // one wave per (64 points, frequency), FW frequencies per workgroup (2
     // measured 1-2 % faster than 4 or 8 on 720x360)
     const int fw = 2;
     const dim3 ga(ntasks, (omax + fw - 1) / fw);
     if (nb == 4)
-      hipLaunchKernelGGL((k_advect<T, 4, false>), ga, dim3(64 * fw), 0, s, doms, tasks, nseg);
+      hipLaunchKernelGGL((k_advect<T, 4, false>), ga, dim3(64 * fw), 0, s, doms, tasks, ng);
     else
-      hipLaunchKernelGGL((k_advect<T, 2, false>), ga, dim3(64 * fw), 0, s, doms, tasks, nseg);
+      hipLaunchKernelGGL((k_advect<T, 2, false>), ga, dim3(64 * fw), 0, s, doms, tasks, ng);
   }
   if (ev) (void)hipEventRecord(ev[3], s);
   hipLaunchKernelGGL((k_stress<T>), dim3(ntasks), dim3(64), 0, s, doms, tasks,

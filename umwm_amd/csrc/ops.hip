@@ -555,204 +555,6 @@ __global__ void k_stress_ocn(DomainDev<T> d, OcnDev out, double bf1, double bf2)
 }
 
 // ---------------------------------------------------------------------
-// src/umwm_physics.F90:89-205 diag
-// ---------------------------------------------------------------------
-// One pass over the point's spectrum, frequency by frequency: the tables of
-// a frequency are read once and the directions of its spectrum rows (one
-// coalesced row per (o, p) across the lanes) are summed in FP64.  The
-// dominant bin is the reference's maxloc over e kdk (o fastest,
-// src/umwm_physics.F90:157-160): of equal maxima the one first in (p, o)
-// order.
-template <typename T>
-__global__ void k_diag(DomainDev<T> d, DiagDev g) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= d.im) return;
-  const size_t ldi = d.ldi;
-  const int om = d.om, pm = d.pm, oc = d.oc[j];
-  double m0 = 0, m2 = 0, mk = 0, mx = 0, my = 0, gxx = 0, gxy = 0, gyy = 0, xc = 0, yc = 0;
-  double best = -INFINITY;
-  int opk = 0, ppk = 0;
-  for (int o = 0; o < om; ++o) {
-    const size_t t = (size_t)o * ldi + j;
-    const double kdk = d.kdk[t], f = d.f[o], k3dk = d.k3dk[t];
-    const double icp = d.invcp0[t], cg = d.cg0[t];
-    const bool prog = o <= oc;
-    const T* eo = d.e + (size_t)o * pm * ldi + j;
-    double s0 = 0, sk = 0, sx = 0, sy = 0, sxx = 0, sxy = 0, syy = 0;
-    for (int p = 0; p < pm; ++p) {
-      const double c = d.cth[p], s = d.sth[p];
-      const double e = eo[(size_t)p * ldi];
-      const double ek = e * kdk;
-      s0 += ek;
-      sk += e * k3dk;
-      sx += ek * c;
-      sy += ek * s;
-      if (prog) {
-        sxx += ek * (c * c);
-        sxy += ek * c * s;
-        syy += ek * (s * s);
-      }
-      if (ek > best || (ek == best && (p < ppk || (p == ppk && o < opk)))) {
-        best = ek;
-        opk = o;
-        ppk = p;
-      }
-    }
-    m0 += s0;
-    m2 += (f * f) * s0;
-    mk += sk;
-    xc += sx;
-    yc += sy;
-    if (prog) {
-      mx += sx * icp;
-      my += sy * icp;
-      gxx += cg * icp * sxx;
-      gxy += cg * icp * sxy;
-      gyy += cg * icp * syy;
-    }
-  }
-  const double tiny = 2.2250738585072014e-308, rw = d.rhow[j];
-  g.mwp[j] = sqrt(m0 / (m2 + tiny));
-  g.momx[j] = mx * rw * d.dthg;
-  g.momy[j] = my * rw * d.dthg;
-  g.cgmxx[j] = gxx * rw * d.dthg;
-  g.cgmxy[j] = gxy * rw * d.dthg;
-  g.cgmyy[j] = gyy * rw * d.dthg;
-  g.ht[j] = 4 * sqrt(m0 * d.dth);
-  g.mwd[j] = atan2(yc, xc);
-  g.mss[j] = mk * d.dth;
-  g.mwl[j] = kTwoPiD * sqrt(m0 / (mk + tiny));
-  const size_t tp = (size_t)opk * ldi + j;
-  g.dwd[j] = d.th[ppk];
-  g.dwl[j] = kTwoPiD / (double)d.k[tp];
-  g.dwp[j] = 1. / (double)d.f[opk];
-  g.dcp0[j] = d.cp0[tp];
-  g.dcg0[j] = d.cg0[tp];
-  const double cur = (double)d.uc[j] * d.cth[ppk] + (double)d.vc[j] * d.sth[ppk];
-  g.dcp[j] = g.dcp0[j] + cur;
-  g.dcg[j] = g.dcg0[j] + cur;
-}
-
-// Significant wave height of E^n for the fused path's s_ice.
-template <typename T>
-__global__ void k_hs_ice(DomainDev<T> d) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= d.im) return;
-  // four independent partial sums (o mod 4): one serial chain of FP64
-  // adds per point made the kernel latency-bound
-  double h4[4] = {0, 0, 0, 0};
-  auto term = [&](int o, int p) {
-    return (double)d.e[((size_t)o * d.pm + p) * d.ldi + j] * (double)d.kdk[(size_t)o * d.ldi + j];
-  };
-  for (int p = 0; p < d.pm; ++p) {
-    int o = 0;
-    for (; o + 3 < d.om; o += 4) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) h4[r] += term(o + r, p);
-    }
-    for (; o < d.om; ++o) h4[0] += term(o, p);
-  }
-  const double h = (h4[0] + h4[1]) + (h4[2] + h4[3]);
-  d.hs_ice[j] = 4 * sqrt(h * d.dth);
-}
-
-// ---------------------------------------------------------------------
-// src/umwm_stokes.F90:13-132 stokes_drift
-// ---------------------------------------------------------------------
-// us(l), vs(l) = sum over o of util(o,l) sum over p of e cos th, e sin th
-// (src/umwm_stokes.F90:59-105) in one pass over the spectrum: per
-// frequency the point's directional sums are formed once and added into
-// the lm level accumulators it keeps in LDS (in o order at every level),
-// which are written once at the end.
-template <typename T>
-__global__ __launch_bounds__(64) void k_stokes(DomainDev<T> d, StokesDev S) {
-  extern __shared__ double acc[];  // [lm][2][points of the block]
-  const int t = threadIdx.x, np = blockDim.x;
-  const int j = blockIdx.x * np + t;
-  const int lm = d.lm;
-  double* au = acc + t;
-  for (int l = 0; l < lm; ++l) {
-    au[(2 * l) * np] = 0;
-    au[(2 * l + 1) * np] = 0;
-  }
-  if (j >= d.im) return;  // no barrier follows: each lane owns its column
-  const size_t ldi = d.ldi;
-  const double dj = d.depth[j];
-  for (int o = 0; o < d.om; ++o) {
-    // four independent partial sums over the directions: one serial chain
-    // of FP64 adds per point made the kernel latency-bound
-    double a4[4] = {0, 0, 0, 0}, b4[4] = {0, 0, 0, 0};
-    const T* eo = d.e + (size_t)o * d.pm * ldi + j;
-    int p = 0;
-    for (; p + 3 < d.pm; p += 4) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const double e = eo[(size_t)(p + r) * ldi];
-        a4[r] += e * (double)d.cth[p + r];
-        b4[r] += e * (double)d.sth[p + r];
-      }
-    }
-    for (; p < d.pm; ++p) {
-      const double e = eo[(size_t)p * ldi];
-      a4[0] += e * (double)d.cth[p];
-      b4[0] += e * (double)d.sth[p];
-    }
-    const double a = (a4[0] + a4[1]) + (a4[2] + a4[3]);
-    const double b = (b4[0] + b4[1]) + (b4[2] + b4[3]);
-    const size_t tq = (size_t)o * ldi + j;
-    const double k = d.k[tq], kd = k * dj, dwn = d.dwn[tq];
-    const double fo = kTwoPiD * (double)d.f[o];
-    const double sh = sinh(kd);
-    for (int l = 0; l < lm; ++l) {
-      const double dep = S.depth[l];
-      if (fabs(dep) > dj) continue;  // level below the sea bed: zero drift
-      const double arg = 2 * k * (dep + dj);
-      double ut;
-      if (fabs(arg) > 50 || kd > 50) {
-        ut = fo * 2 * (k * k) * exp(2 * k * dep) * dwn * d.dth;
-      } else {
-        ut = fo * (k * k) * cosh(2 * k * (dep + dj)) / (sh * sh) * dwn * d.dth;
-      }
-      au[(2 * l) * np] += ut * a;
-      au[(2 * l + 1) * np] += ut * b;
-    }
-  }
-  for (int l = 0; l < lm; ++l) {
-    const double u = au[(2 * l) * np], v = au[(2 * l + 1) * np];
-    S.us[(size_t)l * ldi + j] = u;
-    S.vs[(size_t)l * ldi + j] = v;
-    if (l == 0) {
-      d.us1[j] = u;
-      d.vs1[j] = v;
-    }
-  }
-}
-
-template <typename T>
-__global__ void k_stokes_efold(DomainDev<T> d, StokesDev S) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= d.im) return;
-  const size_t ldi = d.ldi;
-  auto mag = [&](int l) {
-    const double u = S.us[(size_t)l * ldi + j], v = S.vs[(size_t)l * ldi + j];
-    return sqrt(u * u + v * v);
-  };
-  double ds = 0;
-  const double m1 = mag(0);
-  if (m1 != 0) {
-    const double ef = m1 * (1 / exp(1.0));
-    for (int l = 1; l < d.lm; ++l) {
-      const double ma = mag(l - 1), mb = mag(l);
-      if (mb < ef) {
-        ds = (fabs(ma - ef) * S.depth[l] + fabs(mb - ef) * S.depth[l - 1]) / (ma - mb);
-        break;
-      }
-    }
-  }
-  S.ds[j] = -ds;
-}
-
-// ---------------------------------------------------------------------
 // JONSWAP x cos^2 initial spectrum (build-defined initializer)
 // ---------------------------------------------------------------------
 template <typename T>
@@ -879,33 +681,6 @@ int launch_op_stress_ocn(DomainImpl<T>& D) {
 }
 
 template <typename T>
-int launch_diag(DomainImpl<T>& D) {
-  LAUNCH(k_diag<T>, grid1(D.h.im), dim3(kBlock), D.h, D.diag);
-  return 0;
-}
-
-template <typename T>
-int launch_hs_ice(DomainImpl<T>& D) {
-  LAUNCH(k_hs_ice<T>, grid1(D.h.im), dim3(kBlock), D.h);
-  return 0;
-}
-
-template <typename T>
-int launch_stokes(DomainImpl<T>& D) {
-  if (D.h.lm < 1) return 0;
-  // 64 points per block, fewer when the levels' accumulators would pass
-  // 64 KB of LDS (lm > 64)
-  const int np = D.h.lm <= 64 ? 64 : 32;
-  const size_t sh = (size_t)2 * D.h.lm * np * sizeof(double);
-  hipLaunchKernelGGL(k_stokes<T>, dim3((D.h.im + np - 1) / np), dim3(np), sh, D.stream, D.h,
-                     D.stokes);
-  hipError_t e_ = hipGetLastError();
-  if (e_ != hipSuccess) return fail(UMWM_ERR_HIP, std::string("k_stokes: ") + hipGetErrorString(e_));
-  LAUNCH(k_stokes_efold<T>, grid1(D.h.im), dim3(kBlock), D.h, D.stokes);
-  return 0;
-}
-
-template <typename T>
 int launch_jonswap(DomainImpl<T>& D, const umwm_jonswap& js) {
   LAUNCH(k_jonswap<T>, dim3(grid1(D.h.im).x, D.h.om * D.h.pm), dim3(kBlock), D.h, js, D.S.dlnf);
   return 0;
@@ -925,9 +700,6 @@ int launch_jonswap(DomainImpl<T>& D, const umwm_jonswap& js) {
   template int launch_op_update<T>(DomainImpl<T>&);                      \
   template int launch_op_stress_atm<T>(DomainImpl<T>&);                  \
   template int launch_op_stress_ocn<T>(DomainImpl<T>&);                  \
-  template int launch_diag<T>(DomainImpl<T>&);                           \
-  template int launch_hs_ice<T>(DomainImpl<T>&);                         \
-  template int launch_stokes<T>(DomainImpl<T>&);                         \
   template int launch_jonswap<T>(DomainImpl<T>&, const umwm_jonswap&);
 INST(float)
 INST(double)
