@@ -7,6 +7,7 @@
 
 #include <cfloat>
 
+#include "bufio.hpp"
 #include "domain.hpp"
 #include "physics.hpp"
 
@@ -16,6 +17,7 @@ namespace {
 constexpr int kBlock = 256;
 
 inline dim3 grid1(int n) { return dim3((unsigned)((n + kBlock - 1) / kBlock)); }
+inline dim3 rows1(int n) { return dim3((unsigned)((n + 63) / 64)); }
 
 // ---------------------------------------------------------------------
 // src/umwm_forcing.F90:40-99 forcinginterpolate (gustiness = 0)
@@ -109,42 +111,102 @@ __device__ inline SinPoint<T> sin_point(const DomainDev<T>& d, int j) {
   return s;
 }
 
+// One thread per (frequency, point), over its directions: the point's inputs
+// and tables are read once.  In FP64 cos(wdir - th) comes from the angle-sum
+// identity, one cosine and sine instead of a cosine per bin.
 template <typename T>
 __global__ void k_sin_bins(DomainDev<T> d) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  const int op = blockIdx.y, o = op / d.pm, p = op % d.pm;
+  const int o = blockIdx.y;
   if (j >= d.im) return;
   const SinPoint<T> s = sin_point(d, j);
   const size_t t = (size_t)o * d.ldi + j;
-  const T cwt = cos(d.wdir[j] - d.th[p]);
-  d.ssin[((size_t)o * d.pm + p) * d.ldi + j] =
-      ssin_bin(s, d.logl2overz[t], cwt, d.cp0[t], d.cth[p], d.sth[p], d.fkovg[t], T(d.sin_fac),
-               T(d.fieldscale1), T(d.fieldscale2), o);
+  const T wdir = d.wdir[j], logl2 = d.logl2overz[t], cp0 = d.cp0[t], fkovg = d.fkovg[t];
+  [[maybe_unused]] T cw = 0, sw = 0;
+  if constexpr (sizeof(T) == 8) {
+    cw = cos(wdir);
+    sw = sin(wdir);
+  }
+#pragma unroll 4
+  for (int p = 0; p < d.pm; ++p) {
+    const T ct = d.cth[p], st = d.sth[p];
+    T cwt;
+    if constexpr (sizeof(T) == 8)
+      cwt = fma(cw, ct, sw * st);
+    else
+      cwt = cos(wdir - d.th[p]);
+    d.ssin[((size_t)o * d.pm + p) * d.ldi + j] =
+        ssin_bin(s, logl2, cwt, cp0, ct, st, fkovg, T(d.sin_fac), T(d.fieldscale1),
+                 T(d.fieldscale2), o);
+  }
 }
 
 // ---------------------------------------------------------------------
 // src/umwm_source_functions.F90:85-105 sds_d12, directional convolution
 // in the reference's order
 // ---------------------------------------------------------------------
+// The convolution reads every direction of a frequency for every direction:
+// pm^2 spectrum values a point.  k_sds_conv stages the rows of a frequency and
+// 64 points in LDS, kSdsRows at a time, for kSdsWaves waves that take kSdsDirs
+// directions at once, and leaves the sums in `dummy` a frequency later, where
+// k_sds_sum adds them up over frequency, term by term as the reference does.
+// One kernel per (direction, point) that did both had taken 450 us for 8,397
+// points x 37x36 in FP64; now 169.
+constexpr int kSdsWaves = 4, kSdsDirs = 3, kSdsRows = 64;
+
 template <typename T>
-__global__ void k_sds(DomainDev<T> d) {
+__global__ __launch_bounds__(64 * kSdsWaves) void k_sds_conv(DomainDev<T> d) {
+  __shared__ T tile[kSdsRows][64];
+  const int lane = threadIdx.x & 63, w = wave_id();
+  const int j = blockIdx.x * 64 + lane, o = blockIdx.y;
+  const bool valid = j < d.im;
+  const int pm = d.pm;
+  const size_t ldi = d.ldi;
+  const T* eo = d.e + (size_t)o * pm * ldi + j;
+  T* out = d.dummy + (size_t)(o + 1) * pm * ldi + j;
+  const bool one = pm <= kSdsRows;  // all rows at once
+  for (int pb = 0; pb < pm; pb += kSdsWaves * kSdsDirs) {
+    const int p0 = pb + w * kSdsDirs;
+    T acc[kSdsDirs];
+#pragma unroll
+    for (int q = 0; q < kSdsDirs; ++q) acc[q] = 0;
+    for (int r0 = 0; r0 < pm; r0 += kSdsRows) {
+      const int rows = min(kSdsRows, pm - r0);
+      if (pb == 0 || !one) {
+        __syncthreads();  // the previous rows are read
+        for (int r = w; r < rows; r += kSdsWaves) tile[r][lane] = valid ? eo[(r0 + r) * ldi] : T(0);
+        __syncthreads();
+      }
+      for (int r = 0; r < rows; ++r) {
+        const T e = tile[r][lane];
+#pragma unroll
+        for (int q = 0; q < kSdsDirs; ++q) {
+          const int p = min(p0 + q, pm - 1);  // wave-uniform
+          acc[q] += e * cld(d.cth2pp, p * pm + r0 + r);
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kSdsDirs; ++q)
+      if (valid && p0 + q < pm) out[(p0 + q) * ldi] = acc[q];
+  }
+}
+
+template <typename T>
+__global__ void k_sds_sum(DomainDev<T> d) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   const int p = blockIdx.y;
   if (j >= d.im) return;
-  const int pm = d.pm;
   const size_t ldi = d.ldi;
   T raw = 0;
   for (int o = 0; o < d.om; ++o) {
+    const size_t b = ((size_t)o * d.pm + p) * ldi + j;
     if (o > 0 && d.mss_fac > 0) {
-      T acc = 0;
-      const T* eo = d.e + (size_t)(o - 1) * pm * ldi + j;
-      const T* w = d.cth2pp + (size_t)p * pm;
-      for (int pp = 0; pp < pm; ++pp) acc += eo[pp * ldi] * w[pp];
+      const T acc = d.dummy[b];
       raw = raw + acc * d.k3dk[(size_t)(o - 1) * ldi + j];
     }
     T dm = T(1) + T(d.mss_fac) * raw;
     dm = dm * dm;
-    const size_t b = ((size_t)o * pm + p) * ldi + j;
     d.dummy[b] = dm;
     d.sds[b] = T(d.twopisds_fac) * d.f[o] * dm *
                pw(d.e[b] * d.k4[(size_t)o * ldi + j], T(d.sds_power));
@@ -184,22 +246,57 @@ __global__ void k_snl_post(DomainDev<T> d) {
 // ---------------------------------------------------------------------
 // src/umwm_source_functions.F90:108-153 s_ice
 // ---------------------------------------------------------------------
-template <typename T>
-__global__ void k_sice(DomainDev<T> d) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= d.im) return;
-  const size_t ldi = d.ldi;
-  if (d.fice[j] > T(d.fice_lth)) {
-    double ht = 0;
-    for (int p = 0; p < d.pm; ++p)
-      for (int o = 0; o < d.om; ++o)
-        ht += (double)(d.e[((size_t)o * d.pm + p) * ldi + j] * d.kdk[(size_t)o * ldi + j]);
-    ht = 4 * sqrt(ht * d.dth);
-    const double c = sice_coef(ht);
-    for (int o = 0; o < d.om; ++o) d.sice[(size_t)o * ldi + j] = T(2 * (double)d.cg0[(size_t)o * ldi + j] * c);
-  } else {
-    for (int o = 0; o < d.om; ++o) d.sice[(size_t)o * ldi + j] = 0;
+// Per-point sums over the whole spectrum (s_ice, source's largest rate and
+// both stresses): a workgroup of kRowWaves waves owns 64 points, each wave
+// takes every kRowWaves-th frequency with all its directions, and the waves'
+// sums are added in order through LDS.  One thread a point had run the bins
+// one after another on a fifth of the GPU's waves: 10,505 points x 37x36 in
+// FP64 1,013 us for the rates, 670 for stress('atm') and 822 for
+// stress('ocn'), now some 70, 45 and 113.
+constexpr int kRowWaves = 16;
+
+// v[i] of all waves of the workgroup, summed per lane into wave 0 (which also
+// returns true there); every wave must call it.
+template <int N>
+__device__ __forceinline__ bool sum_rows(double (&v)[N]) {
+  __shared__ double red[kRowWaves - 1][N][64];
+  const int lane = threadIdx.x & 63, w = wave_id();
+  __syncthreads();  // the sums of an earlier call are read
+  if (w > 0) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) red[w - 1][i][lane] = v[i];
   }
+  __syncthreads();
+  if (w > 0) return false;
+  for (int q = 0; q < kRowWaves - 1; ++q)
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] += red[q][i][lane];
+  return true;
+}
+
+template <typename T>
+__global__ __launch_bounds__(64 * kRowWaves) void k_sice(DomainDev<T> d) {
+  const int j0 = blockIdx.x * 64 + (threadIdx.x & 63), w = wave_id();
+  const int j = min(j0, d.im - 1);
+  const size_t ldi = d.ldi;
+  const bool ice = d.fice[j] > T(d.fice_lth);
+  double ht[1] = {0};
+  if (__any(ice)) {
+    for (int o = w; o < d.om; o += kRowWaves) {
+      const T kdk = d.kdk[(size_t)o * ldi + j];
+      for (int p = 0; p < d.pm; ++p) ht[0] += (double)(d.e[((size_t)o * d.pm + p) * ldi + j] * kdk);
+    }
+  }
+  __shared__ double coef[64];
+  if (sum_rows(ht)) {
+    const double h = 4 * sqrt(ht[0] * d.dth);
+    coef[threadIdx.x & 63] = ice ? sice_coef(h) : 0.0;
+  }
+  __syncthreads();
+  const double c = coef[threadIdx.x & 63];
+  if (j0 >= d.im) return;
+  for (int o = w; o < d.om; o += kRowWaves)
+    d.sice[(size_t)o * ldi + j] = ice ? T(2 * (double)d.cg0[(size_t)o * ldi + j] * c) : T(0);
 }
 
 // ---------------------------------------------------------------------
@@ -207,7 +304,7 @@ __global__ void k_sice(DomainDev<T> d) {
 // ---------------------------------------------------------------------
 template <typename T>
 __device__ inline void last_block_dts(const DomainDev<T>& d, double bmin, int first) {
-  __shared__ double red[kBlock / 64];
+  __shared__ double red[kRowWaves];
   __shared__ int is_last;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   bmin = wave_min(bmin);
@@ -239,23 +336,33 @@ __device__ inline void last_block_dts(const DomainDev<T>& d, double bmin, int fi
 }
 
 template <typename T>
-__global__ void k_src_rate(DomainDev<T> d, int first) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(64 * kRowWaves) void k_src_rate(DomainDev<T> d, int first) {
+  __shared__ T mw[kRowWaves][64];
+  const int lane = threadIdx.x & 63, w = wave_id();
+  const int j = blockIdx.x * 64 + lane;
   double pts = INFINITY;
+  T mx = 0;
   if (j < d.im) {
     const size_t ldi = d.ldi;
     const int oc = d.oc[j];
-    T mx = 0;
-    for (int p = 0; p < d.pm; ++p)
-      for (int o = 0; o < d.om; ++o) {
-        const size_t b = ((size_t)o * d.pm + p) * ldi + j, t = (size_t)o * ldi + j;
+    for (int o = w; o < d.om; o += kRowWaves) {
+      const size_t t = (size_t)o * ldi + j;
+      const T arg = d.snl_arg[t], sbf = d.sbf[t], sdt = d.sdt[t], sdv = d.sdv[t], ice = d.sice[t];
+#pragma unroll 4
+      for (int p = 0; p < d.pm; ++p) {
+        const size_t b = ((size_t)o * d.pm + p) * ldi + j;
         T r = 0;
-        if (o <= oc)
-          r = d.ssin[b] - d.sds[b] * d.snl_arg[t] - d.sbf[t] - d.sdt[t] - d.sdv[t] + d.sice[t];
+        if (o <= oc) r = d.ssin[b] - d.sds[b] * arg - sbf - sdt - sdv + ice;
         d.ef[b] = r;
         T a = fabs(r);
         mx = a > mx ? a : mx;
       }
+    }
+  }
+  mw[w][lane] = mx;
+  __syncthreads();
+  if (w == 0 && j < d.im) {
+    for (int q = 1; q < kRowWaves; ++q) mx = mw[q][lane] > mx ? mw[q][lane] : mx;
     pts = d.explim / (double)mx;
     d.pts[j] = pts;
   }
@@ -336,14 +443,15 @@ __device__ inline T rotation(const DomainDev<T>& d, int o, int p, int j) {
                        d.oneovdy[j]);
 }
 
+// One frequency per block row.
 template <typename T>
 __global__ void k_rotation(DomainDev<T> d) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  const int j = blockIdx.x * blockDim.x + threadIdx.x, o = blockIdx.y;
   double mx = -INFINITY;
   if (j < d.im) {
     const int oc = d.oc[j];
-    d.oc_rot[j] = oc;
-    for (int o = 0; o < d.om; ++o)
+    if (o == 0) d.oc_rot[j] = oc;
+    {
       for (int p = 0; p < d.pm; ++p) {
         const size_t b = ((size_t)o * d.pm + p) * d.ldi + j;
         T rl = 0, rr = 0;
@@ -358,6 +466,7 @@ __global__ void k_rotation(DomainDev<T> d) {
         d.rotl[b] = rl;
         d.rotr[b] = rr;
       }
+    }
   }
   // block max -> last block sets dtr_temp (signed maxval, :352-361)
   __shared__ double red[kBlock / 64];
@@ -372,7 +481,7 @@ __global__ void k_rotation(DomainDev<T> d) {
     atomicMax(&d.sc->rot_key, okey(m));
     __builtin_amdgcn_s_waitcnt(0);  // the atomic completes before the arrival count
     unsigned t = atomicAdd(&d.sc->counter_rot, 1u);
-    is_last = (t == gridDim.x - 1);
+    is_last = (t == gridDim.x * gridDim.y - 1);
   }
   __syncthreads();
   if (!is_last || threadIdx.x != 0) return;
@@ -417,36 +526,46 @@ __global__ void k_update(DomainDev<T> d) {
 // src/umwm_stress.F90:216-264 stress('atm') from materialised ssin
 // ---------------------------------------------------------------------
 template <typename T>
-__global__ void k_stress_atm(DomainDev<T> d) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= d.im) return;
+__global__ __launch_bounds__(64 * kRowWaves) void k_stress_atm(DomainDev<T> d) {
+  const int j0 = blockIdx.x * 64 + (threadIdx.x & 63), w = wave_id();
+  const int j = min(j0, d.im - 1);  // lanes past the end repeat the last point
   const size_t ldi = d.ldi;
   const int om = d.om, oc = d.oc[j];
   // stress_vector_integral divides by cp0(o, i-1) (src/umwm_stress.F90:219,316)
   const int jc = (j == 0) ? d.im : j - 1;
-  StressIn s;
-  s.sx = s.sy = s.dx = s.dy = s.tomx = s.tomy = 0;
-  for (int o = 0; o < om; ++o) {
+  double v[6] = {0, 0, 0, 0, 0, 0};  // sx, sy; over o >= oc; of the last frequency
+  for (int o = w; o < om; o += kRowWaves) {
     const double cp = d.cp0[(size_t)o * ldi + jc];
     double tx = 0, ty = 0;
+#pragma unroll 4
     for (int p = 0; p < d.pm; ++p) {
       const size_t b = ((size_t)o * d.pm + p) * ldi + j;
       const double es = (double)d.e[b] * (double)d.ssin[b];
-      tx = tx + es * (double)d.cth[p] / cp;
-      ty = ty + es * (double)d.sth[p] / cp;
+      tx = fma(es, (double)d.cth[p], tx);
+      ty = fma(es, (double)d.sth[p], ty);
     }
+    tx /= cp;
+    ty /= cp;
     const double kdk = d.kdk[(size_t)o * ldi + j];
-    s.sx += tx * kdk;
-    s.sy += ty * kdk;
+    v[0] += tx * kdk;
+    v[1] += ty * kdk;
     if (o >= oc) {
-      s.dx += tx * kdk;
-      s.dy += ty * kdk;
+      v[2] += tx * kdk;
+      v[3] += ty * kdk;
     }
     if (o == om - 1) {
-      s.tomx = tx;
-      s.tomy = ty;
+      v[4] = tx;
+      v[5] = ty;
     }
   }
+  if (!sum_rows(v) || j0 >= d.im) return;
+  StressIn s;
+  s.sx = v[0];
+  s.sy = v[1];
+  s.dx = v[2];
+  s.dy = v[3];
+  s.tomx = v[4];
+  s.tomy = v[5];
   s.wspd = d.wspd[j];
   s.wdir = d.wdir[j];
   s.uc = d.uc[j];
@@ -464,12 +583,13 @@ __global__ void k_stress_atm(DomainDev<T> d) {
 // and bottom, Snl momentum loss, energy fluxes into the ocean and from the
 // air, and the form-drag partitions, from the current e and the source
 // arrays (ssin, sds after cothkd, snl) of the last source evaluation.
-// FP64 sums; one thread per sea point.
+// FP64 sums.
 // ---------------------------------------------------------------------
 template <typename T>
-__global__ void k_stress_ocn(DomainDev<T> d, OcnDev out, double bf1, double bf2) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= d.im) return;
+__global__ __launch_bounds__(64 * kRowWaves) void k_stress_ocn(DomainDev<T> d, OcnDev out,
+                                                               double bf1, double bf2) {
+  const int j0 = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int j = min(j0, d.im - 1);  // lanes past the end repeat the last point
   const size_t ldi = d.ldi;
   const int om = d.om, pm = d.pm, oc = d.oc[j];
   const double rw = d.rhow[j], dthg = d.dthg;
@@ -479,7 +599,7 @@ __global__ void k_stress_ocn(DomainDev<T> d, OcnDev out, double bf1, double bf2)
   double eo_x = 0, eo_y = 0, ea_x = 0, ea_y = 0, tomx = 0, tomy = 0;
   double t1x = 0, t1y = 0, t2x = 0, t2y = 0, t3x = 0, t3y = 0;
   const double cwd = cos((double)d.wdir[j]), swd = sin((double)d.wdir[j]);
-  for (int o = 0; o < om; ++o) {
+  for (int o = wave_id(); o < om; o += kRowWaves) {
     const double icp = tab(d.invcp0, o), cp = tab(d.cp0, o), kdk = tab(d.kdk, o);
     const double sdt = tab(d.sdt, o), sdv = tab(d.sdv, o), sbf = tab(d.sbf, o);
     // Snl weights of bins o-1, o-2 (o >= 2, 0-based)
@@ -539,6 +659,17 @@ __global__ void k_stress_ocn(DomainDev<T> d, OcnDev out, double bf1, double bf2)
       tomy = uy;
     }
   }
+  // five at a time: one exchange of all 18 would take 138 KB of LDS
+  double va[5] = {top_x, top_y, bot_x, bot_y, tomx}, vb[5] = {snl_x, snl_y, eo_x, eo_y, tomy};
+  double vc[5] = {ea_x, ea_y, t1x, t1y, t2x}, vd[5] = {t2y, t3x, t3y, 0, 0};
+  sum_rows(va);
+  sum_rows(vb);
+  sum_rows(vc);
+  if (!sum_rows(vd) || j0 >= d.im) return;
+  top_x = va[0]; top_y = va[1]; bot_x = va[2]; bot_y = va[3]; tomx = va[4];
+  snl_x = vb[0]; snl_y = vb[1]; eo_x = vb[2]; eo_y = vb[3]; tomy = vb[4];
+  ea_x = vc[0]; ea_y = vc[1]; t1x = vc[2]; t1y = vc[3]; t2x = vc[4];
+  t2y = vd[0]; t3x = vd[1]; t3y = vd[2];
   double w = d.wspd[j];
   w = w > 1e-2 ? w : 1e-2;
   const double kom = tab(d.k, om - 1);
@@ -615,13 +746,15 @@ int launch_forcinginterpolate(DomainImpl<T>& D, bool gate) {
 template <typename T>
 int launch_op_sin(DomainImpl<T>& D) {
   LAUNCH(k_sin_prologue<T>, grid1(D.h.imm), dim3(kBlock), D.h);
-  LAUNCH(k_sin_bins<T>, dim3(grid1(D.h.im).x, D.h.om * D.h.pm), dim3(kBlock), D.h);
+  LAUNCH(k_sin_bins<T>, dim3(grid1(D.h.im).x, D.h.om), dim3(kBlock), D.h);
   return 0;
 }
 
 template <typename T>
 int launch_op_sds(DomainImpl<T>& D) {
-  LAUNCH(k_sds<T>, dim3(grid1(D.h.im).x, D.h.pm), dim3(kBlock), D.h);
+  if (D.h.mss_fac > 0)
+    LAUNCH(k_sds_conv<T>, dim3(rows1(D.h.im).x, D.h.om - 1), dim3(64 * kSdsWaves), D.h);
+  LAUNCH(k_sds_sum<T>, dim3(grid1(D.h.im).x, D.h.pm), dim3(kBlock), D.h);
   return 0;
 }
 
@@ -635,13 +768,13 @@ int launch_op_snl(DomainImpl<T>& D) {
 
 template <typename T>
 int launch_op_sice(DomainImpl<T>& D) {
-  LAUNCH(k_sice<T>, grid1(D.h.im), dim3(kBlock), D.h);
+  LAUNCH(k_sice<T>, rows1(D.h.im), dim3(64 * kRowWaves), D.h);
   return 0;
 }
 
 template <typename T>
 int launch_op_source(DomainImpl<T>& D) {
-  LAUNCH(k_src_rate<T>, grid1(D.h.im), dim3(kBlock), D.h, (int)D.first);
+  LAUNCH(k_src_rate<T>, rows1(D.h.im), dim3(64 * kRowWaves), D.h, (int)D.first);
   LAUNCH(k_src_int<T>, dim3(grid1(D.h.im).x, D.h.om * D.h.pm), dim3(kBlock), D.h);
   return 0;
 }
@@ -655,7 +788,7 @@ int launch_op_propagation(DomainImpl<T>& D) {
 template <typename T>
 int launch_op_refraction(DomainImpl<T>& D) {
   if (D.S.P.currents || D.first || !D.rot_valid) {
-    LAUNCH(k_rotation<T>, grid1(D.h.im), dim3(kBlock), D.h);
+    LAUNCH(k_rotation<T>, dim3(grid1(D.h.im).x, D.h.om), dim3(kBlock), D.h);
     D.rot_valid = true;
   }
   LAUNCH(k_refraction<T>, dim3(grid1(D.h.im).x, D.h.om * D.h.pm), dim3(kBlock), D.h);
@@ -670,13 +803,13 @@ int launch_op_update(DomainImpl<T>& D) {
 
 template <typename T>
 int launch_op_stress_atm(DomainImpl<T>& D) {
-  LAUNCH(k_stress_atm<T>, grid1(D.h.im), dim3(kBlock), D.h);
+  LAUNCH(k_stress_atm<T>, rows1(D.h.im), dim3(64 * kRowWaves), D.h);
   return 0;
 }
 
 template <typename T>
 int launch_op_stress_ocn(DomainImpl<T>& D) {
-  LAUNCH(k_stress_ocn<T>, grid1(D.h.im), dim3(kBlock), D.h, D.ocn, D.S.bf1, D.S.bf2);
+  LAUNCH(k_stress_ocn<T>, rows1(D.h.im), dim3(64 * kRowWaves), D.h, D.ocn, D.S.bf1, D.S.bf2);
   return 0;
 }
 
