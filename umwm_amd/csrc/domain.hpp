@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -101,6 +102,11 @@ struct DomainImpl : DomainBase {
   bool use_graph = true;
   EndDev end{};              // diag and Stokes outputs
   EndDev* end_d = nullptr;   // device copy (array of one)
+  // staging for spectra on their way to and from the host: allocated at the
+  // first such transfer, at most kStageBytes, of stage_pts points
+  double* stage = nullptr;
+  int stage_pts = 0;
+  std::mutex stage_mutex;  // threads may read one domain's fields at once
   OcnDev ocn{};  // allocated with the operator arrays
   BlockTask* tasks = nullptr;
   int ntasks = 0;
@@ -133,6 +139,11 @@ template <typename T> int launch_op_update(DomainImpl<T>& D);
 template <typename T> int launch_op_stress_atm(DomainImpl<T>& D);
 template <typename T> int launch_op_stress_ocn(DomainImpl<T>& D);
 template <typename T> int launch_hs_ice(DomainImpl<T>& D);
+// points j0 .. j0 + nj - 1 of a spectrum to and from (om,pm,im) doubles
+template <typename T>
+int launch_spec_out(DomainImpl<T>& D, const T* src, double* out, int j0, int nj);
+template <typename T>
+int launch_spec_in(DomainImpl<T>& D, T* dst, const double* in, int j0, int nj);
 template <typename T> int launch_jonswap(DomainImpl<T>& D, const umwm_jonswap& js);
 
 // stokes_drift and/or diag of the domains of a task list, in one pass over

@@ -711,6 +711,53 @@ __global__ void k_jonswap(DomainDev<T> d, umwm_jonswap js, double dlnf) {
       T(S * fo * dlnf * D / (double)d.kdk[(size_t)o * d.ldi + j]);
 }
 
+// ---------------------------------------------------------------------
+// spectra between the device's [o][p][ldi] planes and the reference's
+// (om,pm,im) order in doubles, points j0 .. j0 + nj - 1 at a time
+// ---------------------------------------------------------------------
+// Bound by the copy over the bus, so the reordering and the conversion belong
+// on the device: a workgroup turns 64 points x kTurn rows in LDS, whole cache
+// lines on both sides.  With the loops on the host a field of 2,323 points x
+// 37x36 (25 MB) took 4.1 ms to get and 5.2 to set, which also read it back
+// first; now 1.35 (18 GB/s) and 0.71 (35 GB/s).
+constexpr int kTurn = 32;
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_spec_out(DomainDev<T> d, const T* __restrict__ src,
+                                                  double* __restrict__ out, int j0, int nj) {
+  __shared__ double tile[64][kTurn + 1];
+  const int om = d.om, np = om * d.pm, r0 = blockIdx.y * kTurn, b0 = blockIdx.x * 64;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (b0 + lane < nj)
+    for (int r = w; r < kTurn && r0 + r < np; r += 4) {
+      const int p = (r0 + r) / om, o = r0 + r - p * om;
+      tile[lane][r] = src[(size_t)(o * d.pm + p) * d.ldi + j0 + b0 + lane];
+    }
+  __syncthreads();
+  const int r = threadIdx.x & (kTurn - 1);
+  if (r0 + r < np)
+    for (int j = threadIdx.x / kTurn; j < 64 && b0 + j < nj; j += 256 / kTurn)
+      out[(size_t)(b0 + j) * np + r0 + r] = tile[j][r];
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_spec_in(DomainDev<T> d, T* __restrict__ dst,
+                                                 const double* __restrict__ in, int j0, int nj) {
+  __shared__ double tile[64][kTurn + 1];
+  const int om = d.om, np = om * d.pm, r0 = blockIdx.y * kTurn, b0 = blockIdx.x * 64;
+  const int rr = threadIdx.x & (kTurn - 1);
+  if (r0 + rr < np)
+    for (int j = threadIdx.x / kTurn; j < 64 && b0 + j < nj; j += 256 / kTurn)
+      tile[j][rr] = in[(size_t)(b0 + j) * np + r0 + rr];
+  __syncthreads();
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (b0 + lane < nj)
+    for (int r = w; r < kTurn && r0 + r < np; r += 4) {
+      const int p = (r0 + r) / om, o = r0 + r - p * om;
+      dst[(size_t)(o * d.pm + p) * d.ldi + j0 + b0 + lane] = T(tile[lane][r]);
+    }
+}
+
 }  // namespace
 
 // =====================================================================
@@ -752,7 +799,7 @@ int launch_op_sin(DomainImpl<T>& D) {
 
 template <typename T>
 int launch_op_sds(DomainImpl<T>& D) {
-  if (D.h.mss_fac > 0)
+  if (D.h.mss_fac > 0 && D.h.om > 1)
     LAUNCH(k_sds_conv<T>, dim3(rows1(D.h.im).x, D.h.om - 1), dim3(64 * kSdsWaves), D.h);
   LAUNCH(k_sds_sum<T>, dim3(grid1(D.h.im).x, D.h.pm), dim3(kBlock), D.h);
   return 0;
@@ -814,6 +861,20 @@ int launch_op_stress_ocn(DomainImpl<T>& D) {
 }
 
 template <typename T>
+int launch_spec_out(DomainImpl<T>& D, const T* src, double* out, int j0, int nj) {
+  LAUNCH(k_spec_out<T>, dim3(rows1(nj).x, (D.h.om * D.h.pm + kTurn - 1) / kTurn), dim3(256), D.h,
+         src, out, j0, nj);
+  return 0;
+}
+
+template <typename T>
+int launch_spec_in(DomainImpl<T>& D, T* dst, const double* in, int j0, int nj) {
+  LAUNCH(k_spec_in<T>, dim3(rows1(nj).x, (D.h.om * D.h.pm + kTurn - 1) / kTurn), dim3(256), D.h,
+         dst, in, j0, nj);
+  return 0;
+}
+
+template <typename T>
 int launch_jonswap(DomainImpl<T>& D, const umwm_jonswap& js) {
   LAUNCH(k_jonswap<T>, dim3(grid1(D.h.im).x, D.h.om * D.h.pm), dim3(kBlock), D.h, js, D.S.dlnf);
   return 0;
@@ -833,6 +894,8 @@ int launch_jonswap(DomainImpl<T>& D, const umwm_jonswap& js) {
   template int launch_op_update<T>(DomainImpl<T>&);                      \
   template int launch_op_stress_atm<T>(DomainImpl<T>&);                  \
   template int launch_op_stress_ocn<T>(DomainImpl<T>&);                  \
+  template int launch_spec_out<T>(DomainImpl<T>&, const T*, double*, int, int); \
+  template int launch_spec_in<T>(DomainImpl<T>&, T*, const double*, int, int); \
   template int launch_jonswap<T>(DomainImpl<T>&, const umwm_jonswap&);
 INST(float)
 INST(double)
