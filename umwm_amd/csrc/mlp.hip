@@ -1,17 +1,6 @@
-// BF16 MFMA kernels of the surrogate network (mlp.hpp): one tiled GEMM
-// with operand-layout and epilogue variants, the loss, the gradient
-// reductions and the Adam step.
-//
-// GEMM tiling: a workgroup of 4 waves computes a 128x128 block of C; wave
-// (wm, wn) owns the 64x64 quarter (wm, wn) as 2x2 tiles of the 32x32x16
-// bf16 MFMA (v_mfma_f32_32x32x16_bf16, FP32 accumulators).  The K loop
-// steps by 32: each thread stages two 16-byte chunks of A and of B in
-// registers while the waves multiply the tile held in LDS, then writes
-// them to the other LDS buffer (one barrier per step).  In LDS both tiles
-// are k-contiguous rows ([m][k], [n][k], padded by 8 to spread banks), so
-// every MFMA operand is one 16-byte read; operands stored m- or
-// n-contiguous in memory (the weight-gradient products over the batch)
-// are transposed on their way into LDS.
+// BF16 MFMA kernels of the surrogate network (mlp.hpp): the training GEMM
+// with operand-layout and epilogue variants (the loss among them), the
+// inference GEMM, and the Adam step that reduces the gradients' partials.
 //
 // MFMA operand layout (32x32x16): lane l supplies A(m = l%32, k = 8(l/32)
 // + j) and B(k = 8(l/32) + j, n = l%32), j = 0..7; accumulator register i
@@ -32,127 +21,192 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
-constexpr int BM = 128, BN = 128, BK = 32, LDK = BK + 8;
+constexpr int BK = 32;  // K tile of the inference GEMM
+
+// Training GEMM.  A step's products are small (2048 x 512 x 1344 and down to
+// 2048 x 512 x 512): the time is the chain of K tiles, not the MFMA rate, so
+// a workgroup takes only 64 x 64 of C (256 workgroups for 2048 x 512, one a
+// compute unit, where 128 x 128 blocks left three quarters of them idle),
+// steps K by 64 and keeps two tiles in registers ahead of the one in LDS.
+// Wave (wm, wn) of its four owns 32 x 32 as one accumulator of the 32x32x16
+// MFMA.
+//
+// An operand lies in LDS as it lies in memory, k-contiguous rows ([m][k], one
+// 16-byte read per MFMA operand; 144-byte rows put 16 lanes on distinct
+// banks) or m- or n-contiguous rows ([k][m]: the products over the batch and
+// the weights in the backward pass), which ds_read_tr16_b64 transposes as it
+// reads: a group of 16 lanes reads 4 k rows of 16 values, lane i the 8 bytes
+// of row i / 4 at value 4 (i % 4), and receives value i of the 4 rows
+// (192-byte rows put a half wave on distinct banks).  Turning the operand on
+// its way into LDS took a 2-byte store per value.
+//
+// One training step of 2048 rows through 1335-512-512-512-1332 took 790 us
+// (GEMMs 430 of them), now 175 us of kernels (138).
+constexpr int TT = 64;             // block of C and K tile
+constexpr int LMK = TT + 8, LKM = TT + 32;
+
+template <int KMAJOR>
+struct Tile64 {
+  static constexpr int LD = KMAJOR ? LKM : LMK;
+  // the 8 k values of this lane's row: r0 the wave's first row of C, ks the
+  // 16-wide K step
+  static __device__ __forceinline__ bf16x8 frag(const bf16* t, int r0, int ks, int lane) {
+    if constexpr (KMAJOR) {
+      typedef __attribute__((address_space(3))) bf16x4 lds4;
+      const int g = lane >> 4, i = lane & 15;
+      const bf16* q = t + (ks * 16 + 8 * (g >> 1) + (i >> 2)) * LD + r0 + 16 * (g & 1) + 4 * (i & 3);
+      const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds4*)q);
+      const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds4*)(q + 4 * LD));
+      return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    } else {
+      return *(const bf16x8*)(t + (r0 + (lane & 31)) * LD + ks * 16 + (lane >> 5) * 8);
+    }
+  }
+};
 
 template <int AL, int BL, int EP>
-__global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) bf16 As[2][BM][LDK];
-  __shared__ __attribute__((aligned(16))) bf16 Bs[2][BN][LDK];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+__global__ __launch_bounds__(256, 2) void k_gemm(GemmArgs g, int ntm, int ntn, int nz) {
+  using TA = Tile64<AL == A_KM>;
+  using TB = Tile64<BL == B_KN>;
+  __shared__ __attribute__((aligned(16))) bf16 As[2][TT * TA::LD];
+  __shared__ __attribute__((aligned(16))) bf16 Bs[2][TT * TB::LD];
+  // blocks sharing rows of A and of the K range run on one XCD (workgroups go
+  // round-robin over the 8), whose L2 then holds them
+  const int per = (int)(gridDim.x / 8);
+  const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  if (t >= ntm * ntn * nz) return;
+  const int tz = t / (ntm * ntn), tm = t / ntn % ntm, tn = t % ntn;
+  const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
   const int wm = w >> 1, wn = w & 1;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  const int kb = blockIdx.z * g.kchunk;
-  const int ke = min(g.K, kb + g.kchunk);
-  const bf16x8 zero = {};
-  bf16x8 ra[2], rb[2];
-  // Every index below stays inside the operand: rows (m, n) are checked
-  // against M and N, k against the chunk end; a 16-byte chunk never
-  // straddles the end because K, and M or N on their contiguous axis, are
-  // multiples of 8 (checked by gemm()).
-  auto gload = [&](int k0) {
+  const int m0 = tm * TT, n0 = tn * TT;
+  const int kb = tz * g.kchunk, ke = min(g.K, kb + g.kchunk);
+  // Chunks of 16 bytes, two of each operand a thread and K tile, through a
+  // buffer resource at the tile's first byte: rows past M or N and k past the
+  // range read from beyond it, which gives 0 (a masked load would make the
+  // compiler wait for every load in flight).  A chunk never straddles the
+  // end: K, and M or N on their contiguous axis, are multiples of 8 (checked
+  // by gemm()).
+  constexpr uint32_t kOut = 0x80000000u;  // beyond every resource
+  uint32_t oa[2], ob[2];
+  int ka[2], kbv[2];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int q = tid + c * 256;
-      if constexpr (AL == A_MK) {
-        const int r = q >> 2, kc = (q & 3) * 8, m = m0 + r, k = k0 + kc;
-        ra[c] = (m < g.M && k < ke) ? *(const bf16x8*)(g.A + (int64_t)m * g.lda + k) : zero;
-      } else {
-        const int kr = q >> 4, mc = (q & 15) * 8, m = m0 + mc, k = k0 + kr;
-        ra[c] = (k < ke && m < g.M) ? *(const bf16x8*)(g.A + (int64_t)k * g.lda + m) : zero;
-      }
-      if constexpr (BL == B_NK) {
-        const int r = q >> 2, kc = (q & 3) * 8, n = n0 + r, k = k0 + kc;
-        rb[c] = (n < g.N && k < ke) ? *(const bf16x8*)(g.B + (int64_t)n * g.ldb + k) : zero;
-      } else {
-        const int kr = q >> 4, nc = (q & 15) * 8, n = n0 + nc, k = k0 + kr;
-        rb[c] = (k < ke && n < g.N) ? *(const bf16x8*)(g.B + (int64_t)k * g.ldb + n) : zero;
-      }
-    }
-  };
-  auto sstore = [&](int buf) {
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int q = tid + c * 256;
-      if constexpr (AL == A_MK) {
-        *(bf16x8*)&As[buf][q >> 2][(q & 3) * 8] = ra[c];
-      } else {
-        const int kr = q >> 4, mc = (q & 15) * 8;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) As[buf][mc + i][kr] = ra[c][i];
-      }
-      if constexpr (BL == B_NK) {
-        *(bf16x8*)&Bs[buf][q >> 2][(q & 3) * 8] = rb[c];
-      } else {
-        const int kr = q >> 4, nc = (q & 15) * 8;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) Bs[buf][nc + i][kr] = rb[c][i];
-      }
-    }
-  };
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
-  int buf = 0;
-  if (kb < ke) {
-    gload(kb);
-    sstore(0);
+  for (int c = 0; c < 2; ++c) {
+    const int q = tid + c * 256, r = q >> 3, x = (q & 7) * 8;
+    const bool ina = AL == A_MK ? m0 + r < g.M : m0 + x < g.M;
+    const bool inb = BL == B_NK ? n0 + r < g.N : n0 + x < g.N;
+    oa[c] = ina ? (uint32_t)(r * g.lda + x) * 2u : kOut;
+    ob[c] = inb ? (uint32_t)(r * g.ldb + x) * 2u : kOut;
+    ka[c] = AL == A_MK ? x : r;
+    kbv[c] = BL == B_NK ? x : r;
   }
-  __syncthreads();
-  for (int k0 = kb; k0 < ke; k0 += BK) {
-    const bool more = k0 + BK < ke;
-    if (more) gload(k0 + BK);
+  struct Stage {
+    bf16x8 a[2], b[2];
+  };
+  auto gload = [&](Stage& S, int k0) {
+    const rsrc_t rA = make_rsrc(AL == A_MK ? g.A + (int64_t)m0 * g.lda + k0
+                                           : g.A + (int64_t)k0 * g.lda + m0, kOut);
+    const rsrc_t rB = make_rsrc(BL == B_NK ? g.B + (int64_t)n0 * g.ldb + k0
+                                           : g.B + (int64_t)k0 * g.ldb + n0, kOut);
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const int kk = ks * 16 + (lane >> 5) * 8;
-      bf16x8 fa[2], fb[2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        fa[t] = *(const bf16x8*)&As[buf][wm * 64 + t * 32 + (lane & 31)][kk];
-        fb[t] = *(const bf16x8*)&Bs[buf][wn * 64 + t * 32 + (lane & 31)][kk];
-      }
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-          acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[a], fb[b], acc[a][b], 0, 0, 0);
+    for (int c = 0; c < 2; ++c) {
+      S.a[c] = __builtin_bit_cast(bf16x8, bld16<float>(rA, k0 + ka[c] < ke ? oa[c] : kOut));
+      S.b[c] = __builtin_bit_cast(bf16x8, bld16<float>(rB, k0 + kbv[c] < ke ? ob[c] : kOut));
     }
-    if (more) sstore(buf ^ 1);
+  };
+  // EP_PART, first column of blocks: the sums over k of A's rows, the bias
+  // gradient of the products over the batch
+  [[maybe_unused]] float csum[8] = {};
+  const bool sums = EP == EP_PART && AL == A_KM && tn == 0 && g.asum;
+  auto sstore = [&](const Stage& S, int buf) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int q = tid + c * 256, r = q >> 3, x = (q & 7) * 8;
+      *(bf16x8*)&As[buf][r * TA::LD + x] = S.a[c];
+      *(bf16x8*)&Bs[buf][r * TB::LD + x] = S.b[c];
+      if (sums)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) csum[i] += (float)S.a[c][i];
+    }
+  };
+  f32x16 acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  auto mfma = [&](int buf) {
+#pragma unroll
+    for (int ks = 0; ks < TT / 16; ++ks)
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(TA::frag(As[buf], wm * 32, ks, lane),
+                                                    TB::frag(Bs[buf], wn * 32, ks, lane), acc, 0, 0, 0);
+  };
+  // K tile u in LDS buffer u % 2; tiles past the range load zeros
+  Stage st[2];
+  gload(st[0], kb);
+  gload(st[1], kb + TT);
+  sstore(st[0], 0);
+  gload(st[0], kb + 2 * TT);
+  __syncthreads();
+#pragma unroll 1
+  for (int k0 = kb; k0 < ke; k0 += 2 * TT) {
+    sstore(st[1], 1);
+    gload(st[1], k0 + 3 * TT);
+    mfma(0);
     __syncthreads();
-    buf ^= 1;
+    sstore(st[0], 0);
+    gload(st[0], k0 + 4 * TT);
+    mfma(1);  // all zero past an odd number of tiles
+    __syncthreads();
+  }
+  if constexpr (EP == EP_PART) {
+    if (sums) {  // 32 rows of threads per group of 8 columns, in order
+      float* red = reinterpret_cast<float*>(As);  // [32][64]
+#pragma unroll
+      for (int i = 0; i < 8; ++i) red[(tid >> 3) * TT + (tid & 7) * 8 + i] = csum[i];
+      __syncthreads();
+      if (tid < TT && m0 + tid < g.M) {
+        float s = 0.f;
+        for (int r = 0; r < 32; ++r) s += red[r * TT + tid];
+        g.asum[(int64_t)tz * g.M + m0 + tid] = s;
+      }
+    }
   }
   // epilogue
+  [[maybe_unused]] double loss = 0;
+  const int n = n0 + wn * 32 + (lane & 31);
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int m = m0 + wm * 64 + a * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-        const int n = n0 + wn * 64 + b * 32 + (lane & 31);
-        if (m >= g.M || n >= g.N) continue;
-        const float v = acc[a][b][i];
-        const int64_t o = (int64_t)m * g.ldc + n;
-        if constexpr (EP == EP_GELU) {
-          const float z = v + g.bias[n];
-          if (g.Zout) g.Zout[o] = (bf16)z;
-          ((bf16*)g.C)[o] = (bf16)gelu_f(z);
-        } else if constexpr (EP == EP_F32) {
-          ((float*)g.C)[o] = v + (g.bias ? g.bias[n] : 0.f);
-        } else if constexpr (EP == EP_BF16_BM) {
-          ((bf16*)g.C)[o] = (bf16)(v + g.bias[m]);
-        } else if constexpr (EP == EP_DGELU) {
-          ((bf16*)g.C)[o] = (bf16)(v * gelu_grad_f((float)g.Zin[(int64_t)m * g.ldz + n]));
-        } else if constexpr (EP == EP_SUR) {
-          ((bf16*)g.C)[o] = (bf16)expm1f(fminf(g.osd[m] * (v + g.bias[m]) + g.omu[m], 30.f));
-        } else {
-          ((float*)g.C)[(int64_t)blockIdx.z * g.M * g.ldc + o] = v;
-        }
+  for (int i = 0; i < 16; ++i) {
+    const int m = m0 + wm * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+    if (m >= g.M || n >= g.N) continue;
+    const float v = acc[i];
+    const int64_t o = (int64_t)m * g.ldc + n;
+    if constexpr (EP == EP_GELU) {
+      const float z = v + g.bias[n];
+      g.Zout[o] = (bf16)z;
+      ((bf16*)g.C)[o] = (bf16)gelu_f(z);
+    } else if constexpr (EP == EP_F32) {
+      ((float*)g.C)[o] = v + g.bias[n];
+    } else if constexpr (EP == EP_LOSS) {
+      float gr = 0.f;
+      if (n < g.nout) {
+        const float d = v + g.bias[n] - g.target[o];
+        gr = 2.f * d * g.inv;
+        loss += (double)d * d * g.inv;
       }
+      ((bf16*)g.C)[o] = (bf16)gr;
+    } else if constexpr (EP == EP_DGELU) {
+      ((bf16*)g.C)[o] = (bf16)(v * gelu_grad_f((float)g.Zin[(int64_t)m * g.ldz + n]));
+    } else {
+      static_assert(EP == EP_PART, "training epilogues");
+      ((float*)g.C)[(int64_t)tz * g.M * g.ldc + o] = v;
+    }
+  }
+  if constexpr (EP == EP_LOSS) {
+    __shared__ double wsum[4];
+    for (int off = 32; off > 0; off >>= 1) loss += __shfl_down(loss, off, 64);
+    if (lane == 0) wsum[w] = loss;
+    __syncthreads();
+    if (tid == 0) atomicAdd(g.loss, wsum[0] + wsum[1] + wsum[2] + wsum[3]);
+  }
 }
 
 // Inference GEMM.  A workgroup of 4 waves (2 x 2) computes a BMT x BNT
@@ -443,78 +497,51 @@ __global__ __launch_bounds__(256, 2) void k_gemm_inf(GemmArgs g, int ntm, int nt
     }
 }
 
-// gw[i] = sum over s of part[s][i] (deterministic split-K reduction).
-__global__ void k_reduce_parts(const float* __restrict__ part, int splits, int64_t n,
-                               float* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+// A layer's weight and bias gradients from the partials of the products over
+// the batch, added in order (the result does not depend on scheduling): the
+// first n elements are the weights, the next nbias the biases.
+struct LayerParts {
+  const float *pw, *pb;  // [splits][n], [splits][nbias]
+  int splits;
+  int64_t n;
+  int nbias;
+};
+__device__ __forceinline__ float part_sum(const LayerParts& a, int64_t i) {
+  const bool wt = i < a.n;
+  const float* p = wt ? a.pw + i : a.pb + (i - a.n);
+  const int64_t step = wt ? a.n : a.nbias;
   float s = 0.f;
-  for (int k = 0; k < splits; ++k) s += part[(int64_t)k * n + i];
-  out[i] = s;
+  for (int k = 0; k < a.splits; ++k) s += p[k * step];
+  return s;
 }
 
-// gb[n] = sum over rows of d[r][n] (bf16 [rows][ld]).  A block of 256
-// threads takes 32 columns: 8 row groups sum every 8th row each, then the 8
-// partial sums are added in a fixed order (the result does not depend on
-// scheduling).
-__global__ __launch_bounds__(256) void k_colsum(const bf16* __restrict__ d, int rows, int cols,
-                                                int64_t ld, float* __restrict__ out) {
-  __shared__ float part[8][33];
-  const int c = threadIdx.x & 31, rg = threadIdx.x >> 5, n = blockIdx.x * 32 + c;
-  float s = 0.f;
-  if (n < cols)
-    for (int r = rg; r < rows; r += 8) s += (float)d[(int64_t)r * ld + n];
-  part[rg][c] = s;
-  __syncthreads();
-  if (rg == 0 && n < cols) {
-    float t = 0.f;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) t += part[q][c];
-    out[n] = t;
-  }
-}
-
-// Mean squared error over the real outputs with per-output weights: one
-// block per row (no index division), one atomic per block.
-__global__ __launch_bounds__(256) void k_loss(const float* __restrict__ y,
-                                              const float* __restrict__ t,
-                                              const float* __restrict__ wout, int rows, int nout,
-                                              int ld, bf16* __restrict__ dy,
-                                              double* __restrict__ loss) {
-  __shared__ double wsum[4];
-  const int64_t r0 = (int64_t)blockIdx.x * ld;
-  const float inv = 1.f / ((float)rows * (float)nout);
-  double l = 0;
-  for (int c = threadIdx.x; c < ld; c += 256) {
-    float g = 0.f;
-    if (c < nout) {
-      const float wo = wout ? wout[c] : 1.f;
-      const float d = y[r0 + c] - t[r0 + c];
-      g = 2.f * wo * d * inv;
-      l += (double)wo * d * d * inv;
-    }
-    dy[r0 + c] = (bf16)g;
-  }
-  for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off, 64);
-  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = l;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const double b = wsum[0] + wsum[1] + wsum[2] + wsum[3];
-    if (b != 0) atomicAdd(loss, b);
-  }
-}
-
-__global__ void k_adam(float* __restrict__ p, const float* __restrict__ gr, float* __restrict__ m,
-                       float* __restrict__ v, int64_t n, float lr, float b1, float b2, float eps,
-                       float wd, float c1, float c2) {
+__global__ void k_reduce_parts(LayerParts a, float* __restrict__ gw, float* __restrict__ gb) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = gr[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gi;
-  const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  p[i] = p[i] * (1.f - lr * wd) - lr * (mi * c1) / (sqrtf(vi * c2) + eps);
+  if (i >= a.n + a.nbias) return;
+  const float s = part_sum(a, i);
+  if (i < a.n) gw[i] = s; else gb[i - a.n] = s;
+}
+
+// The Adam step of one layer straight from the partials, with the bf16 copy
+// of the new weights.  Bound by its 4 + splits reads and 3.5 writes a weight;
+// as a reduction, two Adam launches and a conversion the gradient and the
+// weights went through memory three times.
+__global__ void k_adam(LayerParts a, MlpLayerDev L, AdamStep h) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= a.n + a.nbias) return;
+  const float gi = part_sum(a, i);
+  const bool wt = i < a.n;
+  const int64_t q = wt ? i : i - a.n;
+  float* const p = wt ? L.w : L.b;
+  float* const m = wt ? L.mw : L.mb;
+  float* const v = wt ? L.vw : L.vb;
+  const float mi = h.b1 * m[q] + (1.f - h.b1) * gi;
+  const float vi = h.b2 * v[q] + (1.f - h.b2) * gi * gi;
+  m[q] = mi;
+  v[q] = vi;
+  const float x = p[q] - h.lr * (mi * h.c1) / (sqrtf(vi * h.c2) + h.eps);
+  p[q] = x;
+  if (wt) L.wb[q] = (bf16)x;
 }
 
 __global__ void k_to_bf16(const float* __restrict__ a, bf16* __restrict__ b, int64_t n) {
@@ -524,18 +551,10 @@ __global__ void k_to_bf16(const float* __restrict__ a, bf16* __restrict__ b, int
 
 inline dim3 grid_for(int64_t n, int t = 256) { return dim3((unsigned)((n + t - 1) / t)); }
 
-template <int AL, int BL>
-int gemm_ep(int ep, const GemmArgs& g, dim3 grid, hipStream_t s) {
-  switch (ep) {
-    case EP_GELU: hipLaunchKernelGGL((k_gemm<AL, BL, EP_GELU>), grid, dim3(256), 0, s, g); break;
-    case EP_F32: hipLaunchKernelGGL((k_gemm<AL, BL, EP_F32>), grid, dim3(256), 0, s, g); break;
-    case EP_BF16_BM: hipLaunchKernelGGL((k_gemm<AL, BL, EP_BF16_BM>), grid, dim3(256), 0, s, g); break;
-    case EP_DGELU: hipLaunchKernelGGL((k_gemm<AL, BL, EP_DGELU>), grid, dim3(256), 0, s, g); break;
-    case EP_PART: hipLaunchKernelGGL((k_gemm<AL, BL, EP_PART>), grid, dim3(256), 0, s, g); break;
-    case EP_SUR: hipLaunchKernelGGL((k_gemm<AL, BL, EP_SUR>), grid, dim3(256), 0, s, g); break;
-    default: return fail(UMWM_ERR_ARGUMENT, "gemm: unknown epilogue");
-  }
-  return 0;
+// K range of one split: whole K tiles
+inline int gemm_chunk(int K, int splits) {
+  const int k = (K + std::max(1, splits) - 1) / std::max(1, splits);
+  return (k + TT - 1) / TT * TT;
 }
 
 }  // namespace
@@ -548,19 +567,26 @@ int gemm(int alay, int blay, int ep, const GemmArgs& g0, int splits, hipStream_t
   if (g.K % 8 || g.lda % 8 || g.ldb % 8 || (alay == A_KM && g.M % 8) || (blay == B_KN && g.N % 8))
     return fail(UMWM_ERR_ARGUMENT, "gemm: K, lda, ldb (and M or N when transposed) must be "
                                    "multiples of 8");
-  splits = std::max(1, splits);
-  int kchunk = (g.K + splits - 1) / splits;
-  kchunk = (kchunk + BK - 1) / BK * BK;
-  splits = (g.K + kchunk - 1) / kchunk;
-  g.kchunk = kchunk;
-  if (ep != EP_PART && splits != 1) return fail(UMWM_ERR_ARGUMENT, "gemm: split-K needs EP_PART");
-  const dim3 grid((g.N + BN - 1) / BN, (g.M + BM - 1) / BM, splits);
-  int rc;
-  if (alay == A_MK && blay == B_NK) rc = gemm_ep<A_MK, B_NK>(ep, g, grid, s);
-  else if (alay == A_MK && blay == B_KN) rc = gemm_ep<A_MK, B_KN>(ep, g, grid, s);
-  else if (alay == A_KM && blay == B_KN) rc = gemm_ep<A_KM, B_KN>(ep, g, grid, s);
-  else rc = gemm_ep<A_KM, B_NK>(ep, g, grid, s);
-  if (rc) return rc;
+  if (g.lda > (1 << 23) || g.ldb > (1 << 23))
+    return fail(UMWM_ERR_SIZE, "gemm: an operand's rows are longer than 8 M values");
+  if (ep != EP_PART) splits = 1;
+  g.kchunk = gemm_chunk(g.K, splits);
+  const int nz = (g.K + g.kchunk - 1) / g.kchunk;
+  const int ntm = (g.M + TT - 1) / TT, ntn = (g.N + TT - 1) / TT;
+  const int64_t nt = (int64_t)ntm * ntn * nz;
+  if (nt > (1ll << 30)) return fail(UMWM_ERR_SIZE, "gemm: too many tiles");
+  const dim3 grid((unsigned)((nt + 7) / 8 * 8));
+#define UMWM_GEMM(AL_, BL_, EP_)                                                            \
+  if (alay == AL_ && blay == BL_ && ep == EP_) {                                            \
+    hipLaunchKernelGGL((k_gemm<AL_, BL_, EP_>), grid, dim3(256), 0, s, g, ntm, ntn, nz);    \
+  } else
+  UMWM_GEMM(A_MK, B_NK, EP_GELU)
+  UMWM_GEMM(A_MK, B_NK, EP_F32)
+  UMWM_GEMM(A_MK, B_NK, EP_LOSS)
+  UMWM_GEMM(A_MK, B_KN, EP_DGELU)
+  UMWM_GEMM(A_KM, B_KN, EP_PART)
+  return fail(UMWM_ERR_ARGUMENT, "gemm: unsupported operands and epilogue");
+#undef UMWM_GEMM
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(UMWM_ERR_HIP, std::string("gemm: ") + hipGetErrorString(e));
   return 0;
@@ -668,11 +694,13 @@ int mlp_create(const std::vector<int>& dims, uint64_t seed, int rows, Mlp& m) {
   m.dy = dalloc<bf16>(m, (size_t)rows * m.L.back().N);
   m.da = dalloc<bf16>(m, (size_t)rows * wmax);
   m.db = dalloc<bf16>(m, (size_t)rows * wmax);
-  // split-K partials: at most 32 splits of the largest weight matrix
+  // split-K partials: at most 32 splits of the largest weight matrix and of
+  // the longest bias
   m.part_elems = part * 32;
   m.part = dalloc<float>(m, m.part_elems);
+  m.partb = dalloc<float>(m, (size_t)wmax * 32);
   m.loss_acc = dalloc<double>(m, 1);
-  if (!m.loss_acc || !m.part || !m.db) return fail(UMWM_ERR_NOMEM, "mlp: device allocation failed");
+  if (!m.loss_acc || !m.part || !m.partb || !m.db) return fail(UMWM_ERR_NOMEM, "mlp: device allocation failed");
   if (int rc = mlp_sync_bf16(m, nullptr)) return rc;
   UMWM_HIP_TRY(hipDeviceSynchronize());
   return 0;
@@ -687,7 +715,7 @@ int mlp_sync_bf16(Mlp& m, hipStream_t s) {
   return 0;
 }
 
-int mlp_forward(Mlp& m, int rows, hipStream_t s) {
+int mlp_forward(Mlp& m, int rows, hipStream_t s, const float* t, double* loss) {
   if (rows > m.cap_rows) return fail(UMWM_ERR_SIZE, "mlp: more rows than the buffers hold");
   const int nl = (int)m.L.size();
   const bf16* in = m.x;
@@ -699,30 +727,25 @@ int mlp_forward(Mlp& m, int rows, hipStream_t s) {
     g.M = rows; g.N = L.N; g.K = L.K;
     g.bias = L.b;
     g.ldc = L.N;
-    int rc;
+    int ep = EP_GELU;
     if (l + 1 < nl) {
       g.C = m.h[l]; g.Zout = m.z[l];
-      rc = gemm(A_MK, B_NK, EP_GELU, g, 1, s);
       in = m.h[l];
+    } else if (t) {
+      ep = EP_LOSS;
+      g.C = m.dy; g.target = t; g.loss = loss; g.nout = m.nout;
+      g.inv = 1.f / ((float)rows * (float)m.nout);
     } else {
+      ep = EP_F32;
       g.C = m.y;
-      rc = gemm(A_MK, B_NK, EP_F32, g, 1, s);
     }
-    if (rc) return rc;
+    if (int rc = gemm(A_MK, B_NK, ep, g, 1, s)) return rc;
   }
   return 0;
 }
 
-int mlp_loss(Mlp& m, const float* t, const float* wout, int rows, hipStream_t s) {
-  const int ld = m.L.back().N;
-  if (rows < 1) return 0;
-  hipLaunchKernelGGL(k_loss, dim3(rows), dim3(256), 0, s, (const float*)m.y, t, wout, rows,
-                     m.nout, ld, m.dy, m.loss_acc);
-  UMWM_HIP_TRY(hipGetLastError());
-  return 0;
-}
-
-int mlp_backward(Mlp& m, int rows, hipStream_t s) {
+int mlp_backward(Mlp& m, int rows, hipStream_t s, const AdamStep* adam) {
+  if (rows % 8) return fail(UMWM_ERR_ARGUMENT, "mlp: training rows must be a multiple of 8");
   const int nl = (int)m.L.size();
   const bf16* dz = m.dy;
   bf16* bufs[2] = {m.da, m.db};
@@ -730,29 +753,19 @@ int mlp_backward(Mlp& m, int rows, hipStream_t s) {
   for (int l = nl - 1; l >= 0; --l) {
     const MlpLayerDev& L = m.L[l];
     const bf16* a = l == 0 ? m.x : m.h[l - 1];
+    const int64_t nw = (int64_t)L.N * L.K;
     // weight gradient over the batch, split over rows so that the small
-    // output (N x K) still fills the GPU
-    const int tiles = ((L.N + BM - 1) / BM) * ((L.K + BN - 1) / BN);
-    int splits = std::max(1, std::min(rows / 256, (1024 + tiles - 1) / tiles));
-    splits = std::min(splits, 32);
+    // output (N x K) still fills the GPU twice
+    const int tiles = ((L.N + TT - 1) / TT) * ((L.K + TT - 1) / TT);
+    int splits = std::max(1, std::min(rows / 256, (512 + tiles - 1) / tiles));
+    splits = std::min<int>(std::min(splits, 32), (int)(m.part_elems / nw));
     GemmArgs g{};
     g.A = dz; g.lda = L.N;       // A(m = out, k = row) = dz[row][out]
     g.B = a; g.ldb = L.K;        // B(k = row, n = in) = a[row][in]
     g.M = L.N; g.N = L.K; g.K = rows;
     g.C = m.part; g.ldc = L.K;
-    if ((size_t)splits * L.N * L.K > m.part_elems) splits = (int)(m.part_elems / ((size_t)L.N * L.K));
-    // gemm() may lower the split count to whole chunks of 32 rows
-    int kchunk = (rows + splits - 1) / splits;
-    kchunk = (kchunk + BK - 1) / BK * BK;
-    const int used = (rows + kchunk - 1) / kchunk;
-    if (rows % 8) return fail(UMWM_ERR_ARGUMENT, "mlp: training rows must be a multiple of 8");
+    g.asum = m.partb;
     if (int rc = gemm(A_KM, B_KN, EP_PART, g, splits, s)) return rc;
-    const int64_t nw = (int64_t)L.N * L.K;
-    hipLaunchKernelGGL(k_reduce_parts, grid_for(nw), dim3(256), 0, s, (const float*)m.part, used,
-                       nw, L.gw);
-    hipLaunchKernelGGL(k_colsum, dim3((L.N + 31) / 32), dim3(256), 0, s, dz, rows, L.N,
-                       (int64_t)L.N, L.gb);
-    UMWM_HIP_TRY(hipGetLastError());
     if (l > 0) {
       // d a_{l-1} = dz W_l, times gelu'(z_{l-1})
       GemmArgs d{};
@@ -765,23 +778,25 @@ int mlp_backward(Mlp& m, int rows, hipStream_t s) {
       dz = bufs[pb];
       pb ^= 1;
     }
+    // after the product that reads the weights
+    const int chunk = gemm_chunk(rows, splits);
+    const LayerParts p{m.part, m.partb, (rows + chunk - 1) / chunk, nw, L.N};
+    if (adam)
+      hipLaunchKernelGGL(k_adam, grid_for(nw + L.N), dim3(256), 0, s, p, L, *adam);
+    else
+      hipLaunchKernelGGL(k_reduce_parts, grid_for(nw + L.N), dim3(256), 0, s, p, L.gw, L.gb);
+    UMWM_HIP_TRY(hipGetLastError());
   }
   return 0;
 }
 
-int mlp_adam(Mlp& m, float lr, float b1, float b2, float eps, float wd, hipStream_t s) {
+int mlp_train_step(Mlp& m, const float* t, int rows, float lr, double* loss, hipStream_t s) {
   m.step += 1;
-  const float c1 = 1.f / (1.f - std::pow(b1, (float)m.step));
-  const float c2 = 1.f / (1.f - std::pow(b2, (float)m.step));
-  for (auto& L : m.L) {
-    const int64_t nw = (int64_t)L.N * L.K;
-    hipLaunchKernelGGL(k_adam, grid_for(nw), dim3(256), 0, s, L.w, (const float*)L.gw, L.mw, L.vw,
-                       nw, lr, b1, b2, eps, wd, c1, c2);
-    hipLaunchKernelGGL(k_adam, grid_for(L.N), dim3(256), 0, s, L.b, (const float*)L.gb, L.mb, L.vb,
-                       (int64_t)L.N, lr, b1, b2, eps, 0.f, c1, c2);
-  }
-  UMWM_HIP_TRY(hipGetLastError());
-  return mlp_sync_bf16(m, s);
+  AdamStep h{lr, 0.9f, 0.999f, 1e-8f, 0.f, 0.f};
+  h.c1 = 1.f / (1.f - std::pow(h.b1, (float)m.step));
+  h.c2 = 1.f / (1.f - std::pow(h.b2, (float)m.step));
+  if (int rc = mlp_forward(m, rows, s, t, loss)) return rc;
+  return mlp_backward(m, rows, s, &h);
 }
 
 namespace {

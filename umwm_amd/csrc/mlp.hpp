@@ -25,12 +25,15 @@ using bf16 = __bf16;
 enum GemmLayout { A_MK = 0, A_KM = 1, B_NK = 0, B_KN = 1 };
 
 // Epilogues:
-//   EP_GELU      z = acc + bias[n]; Zout[m][n] = z (bf16, when given);
+//   EP_GELU      z = acc + bias[n]; Zout[m][n] = z (bf16, training);
 //                C[m][n] = gelu(z) (bf16)
-//   EP_F32       C[m][n] = acc + bias[n] (fp32; bias may be null)
+//   EP_F32       C[m][n] = acc + bias[n] (fp32)
+//   EP_LOSS      d = acc + bias[n] - target[m][n] for n < nout, else 0;
+//                loss += inv d^2, C[m][n] = 2 inv d (bf16)
 //   EP_BF16_BM   C[m][n] = acc + bias[m] (bf16): the transposed last layer
 //   EP_DGELU     C[m][n] = acc * gelu'(Zin[m][n]) (bf16)
-//   EP_PART      C[z][m][n] = acc (fp32 split-K partial, z = blockIdx.z)
+//   EP_PART      C[z][m][n] = acc (fp32 split-K partial z), asum[z][m] = the
+//                sum of A(m, k) over the split's k
 //   EP_SUR       C[m][n] = exp(min(osd[m] (acc + bias[m]) + omu[m], 30)) - 1
 //                (bf16): the surrogate's transposed last layer, its
 //                normalised output turned back into the spreading factor
@@ -38,7 +41,7 @@ enum GemmLayout { A_MK = 0, A_KM = 1, B_NK = 0, B_KN = 1 };
 //                arithmetic), whose bf16 rounding keeps 3 significant digits
 //                where dm^2 itself, close to 1, would keep 2
 enum GemmEpilogue { EP_GELU = 0, EP_F32 = 1, EP_BF16_BM = 2, EP_DGELU = 3, EP_PART = 4,
-                    EP_SUR = 5 };
+                    EP_SUR = 5, EP_LOSS = 6 };
 
 // The surrogate's first-layer operand taken straight from a domain's
 // spectrum: A(m, k) = (ln max(e[k lde + m], 1e-30) - mu[k]) is[k] for the
@@ -66,11 +69,18 @@ struct GemmArgs {
   bf16* Zout;
   int64_t lda, ldb, ldc, ldz;
   int M, N, K;
-  int kchunk;  // K range of one blockIdx.z (split-K)
+  int kchunk;  // K range of one split
+  float* asum;             // EP_PART
+  const float* target;     // EP_LOSS, leading dimension ldc
+  double* loss;            // EP_LOSS
+  int nout;                // EP_LOSS
+  float inv;               // EP_LOSS
   const float *omu, *osd;  // EP_SUR per-row output transform
   SpecOperand sa;          // A_SPEC operand (inference GEMM)
 };
 
+// Training GEMM: EP_GELU, EP_F32 and EP_LOSS with A_MK and B_NK, EP_DGELU with
+// A_MK and B_KN, EP_PART with A_KM and B_KN in `splits` ranges of k.
 int gemm(int alay, int blay, int ep, const GemmArgs& g, int splits, hipStream_t s);
 
 // Inference GEMM (forward only, B_NK, epilogue EP_GELU without Zout or
@@ -122,6 +132,7 @@ struct Mlp {
   float* y = nullptr;
   bf16 *dy = nullptr, *da = nullptr, *db = nullptr;
   float* part = nullptr;      // split-K partials of the weight gradients
+  float* partb = nullptr;     // and of the bias gradients
   size_t part_elems = 0;
   double* loss_acc = nullptr; // device loss accumulator
   int64_t step = 0;
@@ -132,16 +143,19 @@ struct Mlp {
 // Creates the network with widths dims[0..nl] (unpadded), He-uniform
 // weights from `seed`, zero biases, activation buffers for `rows` rows.
 int mlp_create(const std::vector<int>& dims, uint64_t seed, int rows, Mlp& m);
-// Forward on m.x (rows x K0 bf16 already written); training keeps z and h.
-int mlp_forward(Mlp& m, int rows, hipStream_t s);
-// Loss = mean over rows and the nout real outputs of w_o (y - t)^2 with
-// t fp32 [rows][N_last]; writes dy and accumulates the loss (device).
-int mlp_loss(Mlp& m, const float* t, const float* wout, int rows, hipStream_t s);
-// Backward from m.dy: gradients of every layer into gw, gb.
-int mlp_backward(Mlp& m, int rows, hipStream_t s);
-// Adam step on every layer (lr, betas, eps, decoupled weight decay), then
-// the bf16 weight copies.
-int mlp_adam(Mlp& m, float lr, float b1, float b2, float eps, float wd, hipStream_t s);
+// Forward on m.x (rows x K0 bf16 already written); keeps z and h.  Without t
+// the outputs go to m.y; with t (fp32 [rows][N_last]) the mean over rows and
+// the nout real outputs of (y - t)^2 is added to *loss (device) and its
+// gradient goes to m.dy.
+int mlp_forward(Mlp& m, int rows, hipStream_t s, const float* t = nullptr, double* loss = nullptr);
+// Backward from m.dy: gradients of every layer into gw, gb; or, with an Adam
+// step's constants, into the weights, their bf16 copies and the moments.
+struct AdamStep {
+  float lr, b1, b2, eps, c1, c2;
+};
+int mlp_backward(Mlp& m, int rows, hipStream_t s, const AdamStep* adam = nullptr);
+// One step: forward, loss (added to *loss), backward, Adam (0.9, 0.999, 1e-8).
+int mlp_train_step(Mlp& m, const float* t, int rows, float lr, double* loss, hipStream_t s);
 // Refreshes the bf16 copies from the master weights.
 int mlp_sync_bf16(Mlp& m, hipStream_t s);
 // Inference with the last layer transposed: out[o][ldo] (bf16) for `rows`

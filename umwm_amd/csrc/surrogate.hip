@@ -37,19 +37,10 @@ U* salloc(SurrogateImpl& S, size_t n) {
 
 inline dim3 g1(int64_t n, int t = 256) { return dim3((unsigned)((n + t - 1) / t)); }
 
-__global__ void k_fill_f32(float* p, int64_t n, float v) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
-}
 __global__ void k_fill_f64(double* p, int64_t n, double v) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
 }
-__global__ void k_fill_i32(int32_t* p, int64_t n, int32_t v) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
-}
-
 // One training sample per sea point: the raw inputs (ln e of every bin,
 // u10, v10, ln depth) and the raw targets ln dm^2, the directional
 // spreading factor (1 + mss_fac mss)^2 that sds_d12 just left in `dummy`
@@ -129,21 +120,21 @@ __device__ __forceinline__ uint64_t splitmix(uint64_t x) {
 }
 
 // Training or evaluation rows: row r of the batch is sample base + r
-// (evaluation, hashed == 0) or a hashed draw from [0, nrows) (training).
-__global__ void k_sur_gather(const float* __restrict__ feat, const float* __restrict__ targ,
-                             int rows, int nin, int nout, int K0, int N3, const float* fmu,
-                             const float* fis, const float* tmu, const float* tsd,
-                             bf16* __restrict__ x, float* __restrict__ tb, int64_t base,
-                             int hashed, uint64_t seed, int64_t nrows) {
-  const int r = blockIdx.y;
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= rows) return;
+// (evaluation, hashed == 0) or a hashed draw from [0, nrows) (training).  A
+// workgroup a row: the draw's 64-bit remainder, once per value before, had
+// cost half of the 20 us for 2048 rows of 1335 + 1332 values.
+__global__ __launch_bounds__(256) void k_sur_gather(
+    const float* __restrict__ feat, const float* __restrict__ targ, int nin, int nout, int K0,
+    int N3, const float* fmu, const float* fis, const float* tmu, const float* tsd,
+    bf16* __restrict__ x, float* __restrict__ tb, int64_t base, int hashed, uint64_t seed,
+    int64_t nrows) {
+  const int r = blockIdx.x;
   const int64_t row = hashed ? (int64_t)(splitmix(seed ^ (uint64_t)r * 0x632BE59BD9B4E019ull) %
                                          (uint64_t)nrows)
                              : base + r;
-  if (c < K0)
+  for (int c = threadIdx.x; c < K0; c += 256)
     x[(int64_t)r * K0 + c] = c < nin ? (bf16)((feat[row * nin + c] - fmu[c]) * fis[c]) : (bf16)0.f;
-  if (c < N3)
+  for (int c = threadIdx.x; c < N3; c += 256)
     tb[(int64_t)r * N3 + c] = c < nout ? (targ[row * nout + c] - tmu[c]) / tsd[c] : 0.f;
 }
 
@@ -168,13 +159,6 @@ __global__ void k_sur_point(DomainDev<T> d, int j0, int rows, int nb,
            dep <= range[3] * hi) ? 1 : 0;
 }
 
-__global__ void k_store_loss(double* acc, double* out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    *out = *acc;
-    *acc = 0;
-  }
-}
-
 __global__ void k_f32_to_bf16_pad(const float* __restrict__ a, int rows, int cols, int ld,
                                   bf16* __restrict__ x) {
   const int r = blockIdx.y, c = blockIdx.x * blockDim.x + threadIdx.x;
@@ -186,7 +170,6 @@ __global__ void k_f32_pad(const float* __restrict__ a, int rows, int cols, int l
   if (c < ld && r < rows) t[(int64_t)r * ld + c] = c < cols ? a[(int64_t)r * cols + c] : 0.f;
 }
 
-int pad8(int v) { return (v + 7) / 8 * 8; }
 
 }  // namespace
 
@@ -481,9 +464,8 @@ int umwm_hip_surrogate_gradients(umwm_surrogate* s, const float* x, const float*
     hipLaunchKernelGGL(k_f32_pad, dim3((N3 + 255) / 256, n), dim3(256), 0, S.stream,
                        (const float*)tt, n, S.nout, N3, tp);
     hipLaunchKernelGGL(k_fill_f64, dim3(1), dim3(64), 0, S.stream, S.net.loss_acc, (int64_t)1, 0.0);
-    rc = mlp_forward(S.net, n, S.stream);
+    rc = mlp_forward(S.net, n, S.stream, tp, S.net.loss_acc);
   }
-  if (!rc) rc = mlp_loss(S.net, tp, nullptr, n, S.stream);
   if (!rc) rc = mlp_backward(S.net, n, S.stream);
   if (!rc && hipStreamSynchronize(S.stream) != hipSuccess) rc = fail(UMWM_ERR_HIP, "surrogate_gradients");
   if (!rc && loss) (void)hipMemcpy(loss, S.net.loss_acc, sizeof(double), hipMemcpyDeviceToHost);
@@ -522,21 +504,13 @@ int umwm_hip_surrogate_train(umwm_surrogate* s, int32_t steps, double lr, int64_
   hipStream_t st = S.stream;
   const int K0 = S.net.L[0].K, N3 = S.net.L.back().N, B = S.batch;
   hipLaunchKernelGGL(k_fill_f64, g1(steps), dim3(256), 0, st, S.loss_hist, (int64_t)steps, 0.0);
-  hipLaunchKernelGGL(k_fill_f64, dim3(1), dim3(64), 0, st, S.net.loss_acc, (int64_t)1, 0.0);
   for (int k = 0; k < steps; ++k) {
     const uint64_t seed = S.seed * 0x9E3779B97F4A7C15ull + (uint64_t)S.net.step * 0xD1B54A32D192ED03ull;
-    hipLaunchKernelGGL(k_sur_gather, dim3((std::max(K0, N3) + 255) / 256, B), dim3(256), 0, st,
-                       (const float*)S.feat, (const float*)S.targ, B, S.nin, S.nout, K0, N3,
+    hipLaunchKernelGGL(k_sur_gather, dim3(B), dim3(256), 0, st,
+                       (const float*)S.feat, (const float*)S.targ, S.nin, S.nout, K0, N3,
                        (const float*)S.fmu, (const float*)S.fis, (const float*)S.tmu,
                        (const float*)S.tsd, S.net.x, S.tbatch, (int64_t)0, 1, seed, ntrain);
-    int rc = mlp_forward(S.net, B, st);
-    if (!rc) rc = mlp_loss(S.net, S.tbatch, nullptr, B, st);
-    if (!rc) {
-      hipLaunchKernelGGL(k_store_loss, dim3(1), dim3(64), 0, st, S.net.loss_acc, S.loss_hist + k);
-      rc = mlp_backward(S.net, B, st);
-    }
-    if (!rc) rc = mlp_adam(S.net, (float)lr, 0.9f, 0.999f, 1e-8f, 0.f, st);
-    if (rc) return rc;
+    if (int rc = mlp_train_step(S.net, S.tbatch, B, (float)lr, S.loss_hist + k, st)) return rc;
   }
   UMWM_HIP_TRY(hipStreamSynchronize(st));
   std::vector<double> h(steps);
@@ -580,14 +554,12 @@ int umwm_hip_surrogate_eval(umwm_surrogate* s, int64_t first, int64_t n, double*
   while (done + 8 <= n) {
     const int rows = (int)std::min<int64_t>(S.batch, (n - done) / 8 * 8);
     hipLaunchKernelGGL(k_fill_f64, dim3(1), dim3(64), 0, st, S.net.loss_acc, (int64_t)1, 0.0);
-    hipLaunchKernelGGL(k_sur_gather, dim3((std::max(K0, N3) + 255) / 256, rows), dim3(256), 0, st,
-                       (const float*)S.feat, (const float*)S.targ, rows, S.nin, S.nout, K0, N3,
+    hipLaunchKernelGGL(k_sur_gather, dim3(rows), dim3(256), 0, st,
+                       (const float*)S.feat, (const float*)S.targ, S.nin, S.nout, K0, N3,
                        (const float*)S.fmu, (const float*)S.fis, (const float*)S.tmu,
                        (const float*)S.tsd, S.net.x, S.tbatch, first + done, 0, (uint64_t)0,
                        S.count);
-    int rc = mlp_forward(S.net, rows, st);
-    if (!rc) rc = mlp_loss(S.net, S.tbatch, nullptr, rows, st);
-    if (rc) return rc;
+    if (int rc = mlp_forward(S.net, rows, st, S.tbatch, S.net.loss_acc)) return rc;
     double l = 0;
     UMWM_HIP_TRY(hipStreamSynchronize(st));
     UMWM_HIP_TRY(hipMemcpy(&l, S.net.loss_acc, sizeof(double), hipMemcpyDeviceToHost));
