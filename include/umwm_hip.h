@@ -313,7 +313,9 @@ int64_t umwm_hip_field_size(const umwm_domain* dom, const char* name);
 /* ---------------------------------------------------------------------- */
 /* Timing of the fused kernels (HIP events on the domain's stream)        */
 /* ---------------------------------------------------------------------- */
-/* Enables per-kernel event timing of the fused path (off by default). */
+/* Enables per-kernel event timing of the fused path (off by default).  A
+ * timed substep keeps the kernels apart: its sources are never integrated
+ * ahead of their rates. */
 int umwm_hip_set_timing(umwm_domain* dom, int enable);
 /* Accumulated milliseconds and launch counts of the four fused kernels
  * and of the surrogate's inference since the last reset: ms[0..4] =

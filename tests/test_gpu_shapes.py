@@ -73,3 +73,68 @@ def test_moments_after_set_equal_advection(grid, precision):
     finally:
         a.close()
         b.close()
+
+
+def wide(dx, precision, pm=36, currents=False):
+    wl = configs.tiny(3, 145, 140, 25, pm, winds=True, currents=currents, wspd=14.0)
+    wl.params.delx = wl.params.dely = dx
+    wl.params.dtg = 900.0
+    d = hip.Domain(wl.params, wl.grid_input(), wl.forcing_input(0), precision=precision)
+    d.init_jonswap(wl.jonswap)
+    d.stokes_drift(True)
+    d.forcinginput(wl.forcing_input(1))
+    return d
+
+
+# substeps whose sources are integrated ahead of their rates, where the
+# advective limit holds throughout (1 km), where the sources' time scales hold
+# (30 km) and where both do in turn, against the plain order of an explicit
+# tile of the same directions per wave: the same lengths, the same state to
+# rounding (one kernel compiled twice)
+@pytest.mark.parametrize("precision", [8, 4])
+@pytest.mark.parametrize("dx,pm,currents", [(1e3, 36, False), (6e3, 36, False), (9e3, 24, False),
+                                            (12e3, 28, False), (3e4, 36, False), (1e3, 36, True)])
+def test_sources_ahead_of_rates(dx, pm, currents, precision):
+    tol = 1e-12 if precision == 8 else 1e-5
+    a, b = wide(dx, precision, pm, currents), wide(dx, precision, pm, currents)
+    try:
+        D = 6 if pm == 24 else 9
+        b.set_tile(D, -(-pm // D), D, -(-pm // D), 2)
+        for k in range(12):
+            ra, rb = a.substep(), b.substep()
+            assert abs(ra[1] - rb[1]) <= tol * rb[1], (k, ra, rb)
+            assert abs(ra[0] - rb[0]) <= tol * rb[0], (k, ra, rb)
+        pts = a.get("physics_time_step")
+        assert np.allclose(pts, b.get("physics_time_step"), rtol=10 * tol, atol=0)
+        assert a.scalar("dts") <= float(pts.min()) * (1 + tol)
+        na, nb = a.run_dtg(), b.run_dtg()  # the rest of a window, and its short last substep
+        na, nb = a.run_dtg(), b.run_dtg()
+        assert na == nb and a.scalar("sumt") == b.scalar("sumt") == 900.0
+        for name in ("e", "ustar", "ht", "cd"):
+            x, y = a.get(name), b.get(name)
+            assert np.linalg.norm(x - y) <= 10 * tol * np.linalg.norm(y), name
+    finally:
+        a.close()
+        b.close()
+
+
+def test_sources_ahead_in_a_batch():
+    """Members that run ahead beside members that may not (currents) or cannot
+    (their time scales): each as by itself."""
+    spec = [(1e3, False), (1e3, True), (3e4, False)]
+    one = [wide(dx, 8, 36, c) for dx, c in spec]
+    many = [wide(dx, 8, 36, c) for dx, c in spec]
+    batch = hip.Batch(many)
+    try:
+        for _ in range(2):
+            batch.run_dtg()
+            for x in one:
+                x.run_dtg()
+        for x, y in zip(one, many):
+            for name in ("e", "ustar", "ht"):
+                u, v = x.get(name), y.get(name)
+                assert np.linalg.norm(u - v) <= 1e-12 * np.linalg.norm(v), name
+    finally:
+        batch.close()
+        for x in one + many:
+            x.close()

@@ -50,6 +50,10 @@ struct Scalars {
   // the rates kernel's running grid min of pts and max of the rotation
   // rate as order-preserving keys (0 = none yet; its last block clears them)
   unsigned long long pts_key, rot_key;
+  // the next substep's length is expected to be the advective limit, so that
+  // the sources may be integrated over it while their rates are found; and
+  // this substep was (k_stress clears it)
+  int32_t spec, done;
   // surrogate (FP32): this substep's sampled audit sums (error and weight)
   // and the domain's verdict on the previous substep's audit (0: the
   // network may serve, 1: every point takes the plain rates)

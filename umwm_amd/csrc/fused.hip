@@ -482,6 +482,10 @@ __device__ __forceinline__ Prefix prefix_at(const DomainDev<T>& d, const TabGen&
   return P;
 }
 
+// A substep's sources are integrated ahead of its rates after one whose time
+// scales were this much longer than the advective limit (see k_integrate).
+constexpr double kSpecMargin = 1.05;
+
 // ---------------------------------------------------------------------
 // k_rates
 // ---------------------------------------------------------------------
@@ -503,6 +507,7 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
   // with and without currents each follow the reference
   const bool rotation = rot_all || d.currents;
   Scalars* sc = d.sc;
+  if (sc->done) return;  // uniform over the launch: k_integrate has run ahead
   const int W = blockDim.x >> 6, lane = threadIdx.x & 63, w = wave_id();
   const int j = tk.i0 + lane;
   const bool active = sc->sumt < d.dtg;
@@ -962,6 +967,7 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
       sc->dtr = fmin(sc->dtr_temp, dts);
       sc->nsub = sc->nsub + 1;
       sc->last = sc->sumt >= d.dtg ? 1 : 0;
+      sc->spec = !d.currents && mn >= kSpecMargin * d.dtamin ? 1 : 0;
       if constexpr (SUR) {
         if (d.sur_r) {
           // the gate for the next substep: closed while the sampled error
@@ -982,14 +988,36 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
 // ---------------------------------------------------------------------
 // k_integrate
 // ---------------------------------------------------------------------
-template <typename T, int DMAX, bool FULL, bool SUR>
+// SPEC launches run before k_rates, over the substep length that is expected
+// (Scalars::spec: the advective limit, or what is left of the dtg), and keep
+// the largest |rate| of each point beside the integration.  If the point with
+// the shortest time scale allows that length, it is the substep's length
+// whatever the exact time scales are: the last workgroup then does k_rates'
+// bookkeeping and the substep's k_rates and plain k_integrate return at once.
+// Else they run as always and overwrite E*.  The rates share the
+// integration's wind input and dissipation, whose rounding differs from
+// k_rates' (1e-7 in FP32), so a length within 1e-5 of the limit is left to
+// k_rates; lengths are the same bits either way, the points' time scales
+// agree to that rounding.  k_rates + k_integrate, and this kernel (with FP64's
+// k_prefix) in their place, in us: 180,000 points x 37x36 FP32 258 + 454 ->
+// 479; 399,424 x 49x72 FP32 914 + 2,603 -> 2,916; 129,000 x 49x72 FP64 1,404 +
+// 3,536 -> 60 + 3,504; 42,000 x 37x36 FP64 199 + 466 -> 29 + 455.  The price of a wrong guess is this kernel's time, so one is made
+// only after a substep whose time scales were a twentieth above the limit
+// (kSpecMargin).  All waves of a point are in one workgroup here (one chunk,
+// gridDim.y = 1).
+template <typename T, int DMAX, bool FULL, bool SUR, bool SPEC>
 __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restrict__ doms,
                                                    const BlockTask* __restrict__ tasks, int ng,
                                                    int chunks) {
   const BlockTask tk = tasks[blockIdx.x];
   const DomainDev<T>& d = doms[tk.dom];
-  const Scalars* sc = d.sc;
-  if (!sc->active) return;  // uniform over the block
+  Scalars* const sc = d.sc;
+  // uniform over a domain's workgroups
+  if constexpr (SPEC) {
+    if (!sc->spec || d.currents || !(sc->sumt < d.dtg)) return;
+  } else {
+    if (!sc->active || sc->done) return;
+  }
   stage_fm64<T>();
   const int j = tk.i0 + (threadIdx.x & 63);
   const bool valid = j < d.im;
@@ -1004,8 +1032,12 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
   // X; the wave of the next chunk integrates those bins.
   const int oper = uniform_div(om + chunks - 1, chunks);
   const int o0 = chunk * oper, o1 = min(om, o0 + oper);
-  if (o0 >= o1) return;  // an idle slot; no barrier follows
-  const T dts = T(sc->dts);
+  if constexpr (!SPEC) {
+    if (o0 >= o1) return;  // an idle slot; no barrier follows
+  }
+  double dtd = sc->dts;
+  if constexpr (SPEC) dtd = fmin(d.dtamin, d.dtg - sc->sumt);
+  const T dts = T(dtd);
   const T dtx = dts * Tr<T>::kExpScale;  // dts in the exponential's base
   const uint32_t vj = (uint32_t)j * (uint32_t)sizeof(T);
   const uint32_t vr = (uint32_t)j * (uint32_t)(FT_N * sizeof(T));
@@ -1019,8 +1051,13 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
   [[maybe_unused]] const T* const pfxb = d.pfx;
   const T* const fr = d.f;
 
-  const PointState<T> s = point_stored(d, j);
+  PointState<T> s;
+  if constexpr (SPEC)
+    s = point_fresh(d, j, valid && slot == 0);
+  else
+    s = point_stored(d, j);
   const int oc = s.oc;
+  [[maybe_unused]] T rmax = 0;  // SPEC: the largest |rate| of this wave's bins
   [[maybe_unused]] const bool anyice = __any(valid && s.ice != T(0));
   const T sin_diss1 = T(d.sin_fac * d.fieldscale1), fs2 = T(d.fieldscale2);
   [[maybe_unused]] const T tpsf = T(d.twopisds_fac);
@@ -1168,6 +1205,9 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
       icx = Tr<T>::rcp(tc[FT_COTH]);
     }
     const T c0 = -dtx * crest;
+    // snl_arg, for sds as this kernel forms it
+    [[maybe_unused]] T csr = T(1) - (tc[FT_B1] + tc[FT_B2]), rq = 0;
+    if constexpr (SPEC && kDerive) csr *= tc[FT_COTH];
     // the spreading factor's upper bound, from the zeroth-moment prefix
     [[maybe_unused]] const T qhi = (T(1) + T(2) * mssf * pa0) * (T(1) + T(2) * mssf * pa0);
     // dm = q0 + qc cos 2th + qs sin 2th = (q0 - qc) + ct (2 qc ct + 2 qs st),
@@ -1231,6 +1271,15 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
           const T sds = dm * Tr<T>::ex_nn(fma(spow, Tr<T>::lg_nn(fabs(e)), Lk));
           X = sds * e;
           if constexpr (decltype(PROG)::value) {
+            if constexpr (SPEC) {
+              // FP64 has no registers left for a frequency's own maximum (31
+              // spilled, 541 against 455 us at 42,000 points); FP32 has, and
+              // saves the select per bin (2,916 against 3,039 us)
+              if constexpr (kDerive)
+                rq = fmax(rq, FULL || q < nd ? fabs(ss - fma(sds, csr, crest)) : T(0));
+              else
+                rmax = fmax(rmax, prog && (FULL || q < nd) ? fabs(ss - fma(sds, csr, crest)) : T(0));
+            }
             // E_s = e exp(dts (ssin - sds - sbf - sdt - sdv + sice)) + dts snl
             const T a = fma(-dtc, sds, fma(dtx, ss, c0));
             G = prog ? fma(-dsc, X, e * Tr<T>::ex(a)) : T(0);
@@ -1271,6 +1320,9 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
     } else if (anytail) {
       sweep(N{}, Y{}, N{}, N{});
     }
+    if constexpr (SPEC && kDerive) {
+      if (prog) rmax = fmax(rmax, rq);
+    }
     b2m2 = b2m1;
     b2m1 = tc[FT_B2];
     b1m1 = tc[FT_B1];
@@ -1291,6 +1343,66 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
       tg.advance(o, knext);
       if constexpr (kStored) pc = pn;
     }
+  }
+  if constexpr (SPEC) {
+    // the point's time scale, and the grid's as in k_rates
+    __shared__ double red[8][64];
+    const int W = blockDim.x >> 6, w = wave_id(), lane = threadIdx.x & 63;
+    red[w][lane] = (double)rmax;
+    __syncthreads();
+    if (w > 0) return;
+    double mx = 0;
+    for (int q = 0; q < W; ++q) mx = fmax(mx, red[q][lane]);
+    const double pts = d.explim / mx;
+    if (valid) pstore(d.pts, ldi, j, pts);
+    const double mn = wave_min(valid ? pts : (double)INFINITY);
+    if (lane > 0) return;
+    atomicMax(&sc->pts_key, ~okey(mn));
+    __builtin_amdgcn_s_waitcnt(0);  // complete before the arrival count
+    if (atomicAdd(&sc->counter, 1u) != (unsigned)d.nblocks - 1) return;
+    const double lim = okey_inv(~atomicExch(&sc->pts_key, 0ull));
+    const bool fits = lim * (1 - 1e-5) >= dtd;
+    if (fits) {
+      sc->dts = dtd;
+      sc->dta = dtd;
+      sc->sumt = sc->sumt + dtd;
+      sc->dtr = fmin(sc->dtr_temp, dtd);
+      sc->nsub = sc->nsub + 1;
+      sc->last = sc->sumt >= d.dtg ? 1 : 0;
+      sc->active = 1;
+    }
+    sc->spec = fits ? 1 : 0;
+    sc->done = fits ? 1 : 0;
+    sc->counter = 0;
+  }
+}
+
+// The prefix a SPEC launch reads where it is stored: k_rates, which leaves it
+// otherwise, has not run.  A thread a point; bound by the six FP64 planes a
+// frequency that it reads and writes.
+template <typename T>
+__global__ __launch_bounds__(64) void k_prefix(const DomainDev<T>* __restrict__ doms,
+                                               const BlockTask* __restrict__ tasks) {
+  const BlockTask tk = tasks[blockIdx.x];
+  const DomainDev<T>& d = doms[tk.dom];
+  const Scalars* sc = d.sc;
+  if (!sc->spec || d.currents || !(sc->sumt < d.dtg)) return;
+  const int j = tk.i0 + (int)threadIdx.x;
+  if (j >= d.im) return;
+  const size_t ldi = d.ldi;
+  const uint32_t vj = (uint32_t)j * (uint32_t)sizeof(T);
+  const uint32_t rb = (uint32_t)ldi * (uint32_t)sizeof(T);
+  const double hdth = 0.5 * d.dth;
+  const int om = d.om;
+  TabGen tg;
+  Prefix P;
+#pragma unroll 4
+  for (int o = 0; o < om; ++o) {
+    const rsrc_t pf = freq_rsrc(d.pfx, o, 3, ldi);
+    bst(pf, vj, T(hdth * P.a0));
+    bst(pf, vj, T(hdth * P.ac), rb);
+    bst(pf, vj, T(hdth * P.as), 2 * rb);
+    P.add(k3dk_at(d, tg, o, vj), load_mom(d.mom, ldi, o, j));
   }
 }
 
@@ -1654,6 +1766,7 @@ __global__ __launch_bounds__(64) void k_stress(const DomainDev<T>* __restrict__ 
   if (!d.sc->active) return;
   const int j = tk.i0 + (int)threadIdx.x;
   if (j >= d.im) return;
+  if (tk.local == 0 && threadIdx.x == 0) d.sc->done = 0;
   const size_t ldi = d.ldi, ldq = d.ldq;
   const int om = d.om;
   constexpr uint32_t E = sizeof(T);
@@ -1709,6 +1822,7 @@ struct Shape {
   int D2, ng2, c2, w2;
   bool paired;  // k_rates pairs opposite directions where it can
   bool split;
+  bool spec;    // k_integrate runs ahead of k_rates where the domains expect it
 };
 
 template <typename T, int D, bool SUR>
@@ -1743,9 +1857,23 @@ void launch_integrate(const DomainDev<T>* doms, const BlockTask* tasks, int ntas
   const int slots = h.ng2 * h.c2;
   const dim3 grid(ntasks, (slots + h.w2 - 1) / h.w2), block(64 * h.w2);
   if (h.ng2 * D == pm)
-    hipLaunchKernelGGL((k_integrate<T, D, true, SUR>), grid, block, 0, s, doms, tasks, h.ng2, h.c2);
+    hipLaunchKernelGGL((k_integrate<T, D, true, SUR, false>), grid, block, 0, s, doms, tasks, h.ng2, h.c2);
   else if constexpr (D != 2 && D != 4)
-    hipLaunchKernelGGL((k_integrate<T, D, false, SUR>), grid, block, 0, s, doms, tasks, h.ng2, h.c2);
+    hipLaunchKernelGGL((k_integrate<T, D, false, SUR, false>), grid, block, 0, s, doms, tasks, h.ng2, h.c2);
+}
+
+template <typename T>
+void launch_spec(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, const Shape& h,
+                 hipStream_t s) {
+  const dim3 grid(ntasks), block(64 * h.w2);
+  if constexpr (kStoredPrefix<T, false>)
+    hipLaunchKernelGGL((k_prefix<T>), grid, dim3(64), 0, s, doms, tasks);
+  if (h.D2 == 9)
+    hipLaunchKernelGGL((k_integrate<T, 9, true, false, true>), grid, block, 0, s, doms, tasks, h.ng2, 1);
+  else if (h.D2 == 6)
+    hipLaunchKernelGGL((k_integrate<T, 6, true, false, true>), grid, block, 0, s, doms, tasks, h.ng2, 1);
+  else
+    hipLaunchKernelGGL((k_integrate<T, 4, true, false, true>), grid, block, 0, s, doms, tasks, h.ng2, 1);
 }
 
 template <typename T, bool SUR>
@@ -1753,6 +1881,10 @@ int launch_kernels(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks,
                    int first, int rotation, const Shape& h, int nb, bool keep, hipStream_t s,
                    hipEvent_t* ev) {
   if (ev) (void)hipEventRecord(ev[0], s);
+  if constexpr (!SUR) {
+    // a timed substep keeps the kernels apart
+    if (h.spec && !first && !rotation && !ev) launch_spec<T>(doms, tasks, ntasks, h, s);
+  }
 #define UMWM_RATES(D_)                                                                       \
   case D_: launch_rates<T, D_, SUR>(doms, tasks, ntasks, pm, first, rotation, h, s); break;
   switch (h.D1) {
@@ -1854,7 +1986,7 @@ constexpr int kSweepWaves = 1536;
 constexpr int kAdvectWaves = 4096;
 
 Shape choose_shape(const Tile& t, int ntasks, int omax, bool sur) {
-  Shape h{t.D1, t.W1, 1, t.W1, t.D2, t.W2, 1, t.W2, true, false};
+  Shape h{t.D1, t.W1, 1, t.W1, t.D2, t.W2, 1, t.W2, true, false, false};
   const int pm = t.pmax;
   // the network's checks need all of a point's waves in one workgroup; wide
   // spectra keep the tile's own shape
@@ -1871,6 +2003,7 @@ Shape choose_shape(const Tile& t, int ntasks, int omax, bool sur) {
   h.w1 = h.w2 = waves_for(h.ng1 * h.c1);
   h.paired = false;  // one order of operations whatever D
   h.split = ntasks * omax < kAdvectWaves;
+  h.spec = h.c2 == 1 && h.w2 == h.ng2;
   return h;
 }
 
