@@ -567,15 +567,12 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_stress_atm(DomainDev<T> d) {
   s.tomx = v[4];
   s.tomy = v[5];
   s.wspd = d.wspd[j];
-  s.wdir = d.wdir[j];
-  s.uc = d.uc[j];
-  s.vc = d.vc[j];
-  s.us1 = d.us1[j];
-  s.vs1 = d.vs1[j];
   s.rhoa = d.rhoa[j];
   s.rhow = d.rhow[j];
   s.kom = d.k[(size_t)(om - 1) * ldi + j];
-  store_stress(d, j, stress_atm_point(s, d.dthg, d.z, d.nu_air, d.kappa));
+  const SkinWind skin = skin_wind(s.wspd, d.wdir[j], d.uc[j], d.vc[j], d.us1[j], d.vs1[j], d.z,
+                                  d.nu_air, d.kappa);
+  store_stress(d, j, stress_atm_point(s, skin, d.dthg));
 }
 
 // ---------------------------------------------------------------------

@@ -147,7 +147,7 @@ struct StressIn {
   double sx, sy;      // sum_o taux_util(o) * kdk(o)
   double dx, dy;      // same over o >= oc
   double tomx, tomy;  // taux_util(om), tauy_util(om)
-  double wspd, wdir, uc, vc, us1, vs1, rhoa, rhow, kom;
+  double wspd, rhoa, rhow, kom;
 };
 
 struct StressOut {
@@ -155,8 +155,24 @@ struct StressOut {
   double taux_diag, tauy_diag, tailatmx, tailatmy, cd, ustar;
 };
 
-__device__ inline StressOut stress_atm_point(const StressIn& s, double dthg, double z,
-                                             double nu_air, double kappa) {
+// The wind relative to the surface and its skin friction velocity, of the
+// point alone: the longest chain of the stress (six logarithms in turn).
+struct SkinWind {
+  double wspdrel, wdirrel, u;
+};
+__device__ inline SkinWind skin_wind(double wspd, double wdir, double uc, double vc, double us1,
+                                     double vs1, double z, double nu_air, double kappa) {
+  // wind_relative with the surface Stokes drift (:240-243, :333-344)
+  const double urel = wspd * cos(wdir) - (uc + us1);
+  const double vrel = wspd * sin(wdir) - (vc + vs1);
+  SkinWind k;
+  k.wspdrel = sqrt(urel * urel + vrel * vrel);
+  k.wdirrel = atan2(vrel, urel);
+  k.u = friction_velocity_skin(k.wspdrel, z, nu_air, kappa);
+  return k;
+}
+
+__device__ inline StressOut stress_atm_point(const StressIn& s, const SkinWind& k, double dthg) {
   StressOut r;
   const double tail = stress_tail(s.wspd, s.kom);
   r.tailatmx = s.tomx * s.kom * tail * s.rhow * dthg;
@@ -165,15 +181,10 @@ __device__ inline StressOut stress_atm_point(const StressIn& s, double dthg, dou
   r.tauy_form = s.sy * s.rhow * dthg + r.tailatmy;
   r.taux_diag = s.dx * s.rhow * dthg;
   r.tauy_diag = s.dy * s.rhow * dthg;
-  // wind_relative with the surface Stokes drift (:240-243, :333-344)
-  const double urel = s.wspd * cos(s.wdir) - (s.uc + s.us1);
-  const double vrel = s.wspd * sin(s.wdir) - (s.vc + s.vs1);
-  const double wspdrel = sqrt(urel * urel + vrel * vrel);
-  const double wdirrel = atan2(vrel, urel);
+  const double wspdrel = k.wspdrel, wdirrel = k.wdirrel, u = k.u;
   const double w2 = s.wspd * s.wspd;
   const double cd_form =
       sqrt(r.taux_form * r.taux_form + r.tauy_form * r.tauy_form) / (s.rhoa * w2);
-  const double u = friction_velocity_skin(wspdrel, z, nu_air, kappa);
   double cd_skin = (u * u) / w2;
   cd_skin = cd_skin * (1 + 2 * cd_skin / (cd_skin + cd_form + 2.2250738585072014e-308)) / 3;
   if (cd_skin > 1e-2) cd_skin = 1e-2;
