@@ -571,10 +571,9 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
     const rsrc_t rz = make_rsrc(eb, 0u);
     // PAIR launches (FULL with an even DMAX) pair each direction p with p + pm/2
     // (theta + pi): cos and sin change sign while cos 2theta and sin 2theta
-    // do not, so a pair shares its direction record, the mss factor and one
-    // update of the moments.  Wave w then holds pairs w DMAX/2 + h in slots
-    // h and h + DMAX/2, which also halves the direction records the loop
-    // keeps in scalar registers.
+    // do not, so a pair shares its direction record and the mss factor.  Wave
+    // w then holds pairs w DMAX/2 + h in slots h and h + DMAX/2, which also
+    // halves the direction records the loop keeps in scalar registers.
     static_assert(!PAIR || (FULL && DMAX % 2 == 0), "paired sweeps are mask-free and even");
     constexpr int H = DMAX / 2;
     const int ph = grp * H, half = pm / 2;
