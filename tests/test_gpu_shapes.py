@@ -138,3 +138,28 @@ def test_sources_ahead_in_a_batch():
         batch.close()
         for x in one + many:
             x.close()
+
+
+@pytest.mark.parametrize("precision", [8, 4])
+@pytest.mark.parametrize("om,pm", [(6, 16), (7, 4), (5, 36), (7, 28)])
+def test_few_frequencies(om, pm, precision):
+    """One chunk of two directions a wave on a small grid: a shape whose sources
+    are not integrated ahead, over substeps that the advective limit holds."""
+    wl = configs.tiny(4, 16, 13, om, pm, wspd=14.0)
+    wl.params.delx = wl.params.dely = 300.0
+    a, b = (hip.Domain(wl.params, wl.grid_input(), wl.forcing_input(0), precision=precision)
+            for _ in range(2))
+    try:
+        D = 6 if pm % 6 == 0 else 9
+        b.set_tile(D, -(-pm // D), D, -(-pm // D), 2)
+        for d in (a, b):
+            d.init_jonswap(wl.jonswap)
+            d.stokes_drift(True)
+            d.substeps(12)
+        tol = 1e-12 if precision == 8 else 1e-5
+        for name in ("e", "es", "ustar"):
+            x, y = a.get(name), b.get(name)
+            assert np.linalg.norm(x - y) <= tol * np.linalg.norm(y), name
+    finally:
+        a.close()
+        b.close()

@@ -2011,7 +2011,7 @@ Shape choose_shape(const Tile& t, int ntasks, int omax, bool sur) {
   h.w1 = h.w2 = waves_for(h.ng1 * h.c1);
   h.paired = false;  // one order of operations whatever D
   h.split = ntasks * omax < kAdvectWaves;
-  h.spec = h.c2 == 1 && h.w2 == h.ng2;
+  h.spec = h.D2 >= 4 && h.c2 == 1 && h.w2 == h.ng2;  // launch_spec has D = 4, 6 and 9
   return h;
 }
 
