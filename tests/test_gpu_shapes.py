@@ -89,8 +89,7 @@ def wide(dx, precision, pm=36, currents=False):
 # substeps whose sources are integrated ahead of their rates, where the
 # advective limit holds throughout (1 km), where the sources' time scales hold
 # (30 km) and where both do in turn, against the plain order of an explicit
-# tile of the same directions per wave: the same lengths, the same state to
-# rounding (one kernel compiled twice)
+# tile: the same lengths, the same state to rounding
 @pytest.mark.parametrize("precision", [8, 4])
 @pytest.mark.parametrize("dx,pm,currents", [(1e3, 36, False), (6e3, 36, False), (9e3, 24, False),
                                             (12e3, 28, False), (3e4, 36, False), (1e3, 36, True)])
@@ -99,7 +98,7 @@ def test_sources_ahead_of_rates(dx, pm, currents, precision):
     a, b = wide(dx, precision, pm, currents), wide(dx, precision, pm, currents)
     try:
         D = 6 if pm == 24 else 9
-        b.set_tile(D, -(-pm // D), D, -(-pm // D), 2)
+        b.set_tile(D, -(-pm // D), 18, -(-pm // 18), 2)  # 18 directions: never ahead
         for k in range(12):
             ra, rb = a.substep(), b.substep()
             assert abs(ra[1] - rb[1]) <= tol * rb[1], (k, ra, rb)
@@ -111,6 +110,22 @@ def test_sources_ahead_of_rates(dx, pm, currents, precision):
         na, nb = a.run_dtg(), b.run_dtg()
         assert na == nb and a.scalar("sumt") == b.scalar("sumt") == 900.0
         for name in ("e", "ustar", "ht", "cd"):
+            x, y = a.get(name), b.get(name)
+            assert np.linalg.norm(x - y) <= 10 * tol * np.linalg.norm(y), name
+    finally:
+        a.close()
+        b.close()
+
+
+@pytest.mark.parametrize("precision", [8, 4])
+def test_sources_ahead_with_a_given_tile(precision):
+    tol = 1e-12 if precision == 8 else 1e-5
+    a, b = wide(1e3, precision), wide(1e3, precision)
+    try:
+        a.set_tile(18, 2, 9, 4, 2)
+        b.set_tile(18, 2, 18, 2, 2)
+        assert a.run_dtg() == b.run_dtg()
+        for name in ("e", "ustar", "physics_time_step"):
             x, y = a.get(name), b.get(name)
             assert np.linalg.norm(x - y) <= 10 * tol * np.linalg.norm(y), name
     finally:
