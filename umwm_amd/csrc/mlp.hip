@@ -66,16 +66,65 @@ struct Tile64 {
   }
 };
 
+// The bias gradient beside the products over the batch: the sums over k of
+// A(m, k), which lies as [k][m].  A workgroup takes 32 m: 8 groups of its
+// threads add every 8th k each, one after the other, then the 8 sums are added
+// in order.  A chain of K / 8 additions whose loads are what it waits for, so
+// they go out 32 at a time.
+constexpr int kSumCols = 32, kSumRows = 8;
+
+// workgroups of the sums, a whole number on each XCD
+__host__ __device__ inline int bias_blocks(int M) {
+  return ((M + kSumCols - 1) / kSumCols + 7) / 8 * 8;
+}
+
+__device__ __forceinline__ void bias_sum(const GemmArgs& g, float* part) {
+  const int c = (int)threadIdx.x % kSumCols, rg = (int)threadIdx.x / kSumCols;
+  const int m = (int)blockIdx.x * kSumCols + c;
+  float s = 0.f;
+  if (m < g.M) {
+    const bf16* a = g.A + m;
+    int k = rg;
+    for (; k + 31 * kSumRows < g.K; k += 32 * kSumRows) {
+      bf16 v[32];
+#pragma unroll
+      for (int i = 0; i < 32; ++i) v[i] = a[(int64_t)(k + i * kSumRows) * g.lda];
+#pragma unroll
+      for (int i = 0; i < 32; ++i) s += (float)v[i];
+    }
+    for (; k < g.K; k += kSumRows) s += (float)a[(int64_t)k * g.lda];
+  }
+  part[rg * kSumCols + c] = s;
+  __syncthreads();
+  if (rg == 0 && m < g.M) {
+    float t = 0.f;
+#pragma unroll
+    for (int q = 0; q < kSumRows; ++q) t += part[q * kSumCols + c];
+    g.asum[m] = t;
+  }
+}
+
 template <int AL, int BL, int EP>
 __global__ __launch_bounds__(256, 2) void k_gemm(GemmArgs g, int ntm, int ntn, int nz) {
   using TA = Tile64<AL == A_KM>;
   using TB = Tile64<BL == B_KN>;
   __shared__ __attribute__((aligned(16))) bf16 As[2][TT * TA::LD];
   __shared__ __attribute__((aligned(16))) bf16 Bs[2][TT * TB::LD];
+  int b = (int)blockIdx.x, nb = (int)gridDim.x;
+  if constexpr (EP == EP_PART) {
+    // the first workgroups sum the bias gradient beside the products
+    const int sums = bias_blocks(g.M);
+    if (b < sums) {
+      bias_sum(g, reinterpret_cast<float*>(As));
+      return;
+    }
+    b -= sums;
+    nb -= sums;
+  }
   // blocks sharing rows of A and of the K range run on one XCD (workgroups go
   // round-robin over the 8), whose L2 then holds them
-  const int per = (int)(gridDim.x / 8);
-  const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  const int per = nb / 8;
+  const int t = b % 8 * per + b / 8;
   if (t >= ntm * ntn * nz) return;
   const int tz = t / (ntm * ntn), tm = t / ntn % ntm, tn = t % ntn;
   const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
@@ -115,19 +164,12 @@ __global__ __launch_bounds__(256, 2) void k_gemm(GemmArgs g, int ntm, int ntn, i
       S.b[c] = __builtin_bit_cast(bf16x8, bld16<float>(rB, k0 + kbv[c] < ke ? ob[c] : kOut));
     }
   };
-  // EP_PART, first column of blocks: the sums over k of A's rows, the bias
-  // gradient of the products over the batch
-  [[maybe_unused]] float csum[8] = {};
-  const bool sums = EP == EP_PART && AL == A_KM && tn == 0 && g.asum;
   auto sstore = [&](const Stage& S, int buf) {
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const int q = tid + c * 256, r = q >> 3, x = (q & 7) * 8;
       *(bf16x8*)&As[buf][r * TA::LD + x] = S.a[c];
       *(bf16x8*)&Bs[buf][r * TB::LD + x] = S.b[c];
-      if (sums)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) csum[i] += (float)S.a[c][i];
     }
   };
   f32x16 acc;
@@ -156,19 +198,6 @@ __global__ __launch_bounds__(256, 2) void k_gemm(GemmArgs g, int ntm, int ntn, i
     gload(st[0], k0 + 4 * TT);
     mfma(1);  // all zero past an odd number of tiles
     __syncthreads();
-  }
-  if constexpr (EP == EP_PART) {
-    if (sums) {  // 32 rows of threads per group of 8 columns, in order
-      float* red = reinterpret_cast<float*>(As);  // [32][64]
-#pragma unroll
-      for (int i = 0; i < 8; ++i) red[(tid >> 3) * TT + (tid & 7) * 8 + i] = csum[i];
-      __syncthreads();
-      if (tid < TT && m0 + tid < g.M) {
-        float s = 0.f;
-        for (int r = 0; r < 32; ++r) s += red[r * TT + tid];
-        g.asum[(int64_t)tz * g.M + m0 + tid] = s;
-      }
-    }
   }
   // epilogue
   [[maybe_unused]] double loss = 0;
@@ -497,21 +526,19 @@ __global__ __launch_bounds__(256, 2) void k_gemm_inf(GemmArgs g, int ntm, int nt
     }
 }
 
-// A layer's weight and bias gradients from the partials of the products over
-// the batch, added in order (the result does not depend on scheduling): the
-// first n elements are the weights, the next nbias the biases.
+// A layer's weight gradient from the partials of the products over the batch,
+// added in order (the result does not depend on scheduling), and its bias
+// gradient: the first n elements are the weights, the next nbias the biases.
 struct LayerParts {
-  const float *pw, *pb;  // [splits][n], [splits][nbias]
+  const float *pw, *pb;  // [splits][n], [nbias]
   int splits;
   int64_t n;
   int nbias;
 };
 __device__ __forceinline__ float part_sum(const LayerParts& a, int64_t i) {
-  const bool wt = i < a.n;
-  const float* p = wt ? a.pw + i : a.pb + (i - a.n);
-  const int64_t step = wt ? a.n : a.nbias;
+  if (i >= a.n) return a.pb[i - a.n];
   float s = 0.f;
-  for (int k = 0; k < a.splits; ++k) s += p[k * step];
+  for (int k = 0; k < a.splits; ++k) s += a.pw[k * a.n + i];
   return s;
 }
 
@@ -551,10 +578,10 @@ __global__ void k_to_bf16(const float* __restrict__ a, bf16* __restrict__ b, int
 
 inline dim3 grid_for(int64_t n, int t = 256) { return dim3((unsigned)((n + t - 1) / t)); }
 
-// K range of one split: whole K tiles
+// K range of one split, in whole steps of 32 (K tiles end where it ends)
 inline int gemm_chunk(int K, int splits) {
   const int k = (K + std::max(1, splits) - 1) / std::max(1, splits);
-  return (k + TT - 1) / TT * TT;
+  return (k + 31) / 32 * 32;
 }
 
 }  // namespace
@@ -575,7 +602,7 @@ int gemm(int alay, int blay, int ep, const GemmArgs& g0, int splits, hipStream_t
   const int ntm = (g.M + TT - 1) / TT, ntn = (g.N + TT - 1) / TT;
   const int64_t nt = (int64_t)ntm * ntn * nz;
   if (nt > (1ll << 30)) return fail(UMWM_ERR_SIZE, "gemm: too many tiles");
-  const dim3 grid((unsigned)((nt + 7) / 8 * 8));
+  const dim3 grid((unsigned)((nt + 7) / 8 * 8 + (ep == EP_PART ? bias_blocks(g.M) : 0)));
 #define UMWM_GEMM(AL_, BL_, EP_)                                                            \
   if (alay == AL_ && blay == BL_ && ep == EP_) {                                            \
     hipLaunchKernelGGL((k_gemm<AL_, BL_, EP_>), grid, dim3(256), 0, s, g, ntm, ntn, nz);    \
@@ -694,11 +721,11 @@ int mlp_create(const std::vector<int>& dims, uint64_t seed, int rows, Mlp& m) {
   m.dy = dalloc<bf16>(m, (size_t)rows * m.L.back().N);
   m.da = dalloc<bf16>(m, (size_t)rows * wmax);
   m.db = dalloc<bf16>(m, (size_t)rows * wmax);
-  // split-K partials: at most 32 splits of the largest weight matrix and of
-  // the longest bias
+  // split-K partials: at most 32 splits of the largest weight matrix; and the
+  // longest bias gradient
   m.part_elems = part * 32;
   m.part = dalloc<float>(m, m.part_elems);
-  m.partb = dalloc<float>(m, (size_t)wmax * 32);
+  m.partb = dalloc<float>(m, (size_t)wmax);
   m.loss_acc = dalloc<double>(m, 1);
   if (!m.loss_acc || !m.part || !m.partb || !m.db) return fail(UMWM_ERR_NOMEM, "mlp: device allocation failed");
   if (int rc = mlp_sync_bf16(m, nullptr)) return rc;
@@ -755,9 +782,12 @@ int mlp_backward(Mlp& m, int rows, hipStream_t s, const AdamStep* adam) {
     const bf16* a = l == 0 ? m.x : m.h[l - 1];
     const int64_t nw = (int64_t)L.N * L.K;
     // weight gradient over the batch, split over rows so that the small
-    // output (N x K) still fills the GPU twice
-    const int tiles = ((L.N + TT - 1) / TT) * ((L.K + TT - 1) / TT);
-    int splits = std::max(1, std::min(rows / 256, (512 + tiles - 1) / tiles));
+    // output (N x K) still fills the GPU.  The splits set the order of the
+    // sums and with it the last bits of the gradients, which Adam's normalised
+    // step turns into differences of 6e-4 in the weights after sixteen steps:
+    // the rule counts blocks of 128 x 128 whatever the GEMM's own are.
+    const int tiles = ((L.N + 127) / 128) * ((L.K + 127) / 128);
+    int splits = std::max(1, std::min(rows / 256, (1024 + tiles - 1) / tiles));
     splits = std::min<int>(std::min(splits, 32), (int)(m.part_elems / nw));
     GemmArgs g{};
     g.A = dz; g.lda = L.N;       // A(m = out, k = row) = dz[row][out]

@@ -32,8 +32,8 @@ enum GemmLayout { A_MK = 0, A_KM = 1, B_NK = 0, B_KN = 1 };
 //                loss += inv d^2, C[m][n] = 2 inv d (bf16)
 //   EP_BF16_BM   C[m][n] = acc + bias[m] (bf16): the transposed last layer
 //   EP_DGELU     C[m][n] = acc * gelu'(Zin[m][n]) (bf16)
-//   EP_PART      C[z][m][n] = acc (fp32 split-K partial z), asum[z][m] = the
-//                sum of A(m, k) over the split's k
+//   EP_PART      C[z][m][n] = acc (fp32 split-K partial z), asum[m] = the sum
+//                of A(m, k) over all k
 //   EP_SUR       C[m][n] = exp(min(osd[m] (acc + bias[m]) + omu[m], 30)) - 1
 //                (bf16): the surrogate's transposed last layer, its
 //                normalised output turned back into the spreading factor
@@ -132,7 +132,7 @@ struct Mlp {
   float* y = nullptr;
   bf16 *dy = nullptr, *da = nullptr, *db = nullptr;
   float* part = nullptr;      // split-K partials of the weight gradients
-  float* partb = nullptr;     // and of the bias gradients
+  float* partb = nullptr;     // a layer's bias gradient
   size_t part_elems = 0;
   double* loss_acc = nullptr; // device loss accumulator
   int64_t step = 0;
