@@ -54,3 +54,35 @@ def test_operators_by_rows(grid, ice, oracle_lib):
                 d.end_first()
     finally:
         d.close()
+
+
+@pytest.mark.parametrize("pm", [24, 28, 36, 72])
+def test_wind_square_to_a_direction(pm, oracle_lib):
+    """Winds along the axes, the diagonals and the directions themselves, some
+    at a right angle to a bin, where the sign of cos(wdir - th) chooses between
+    dissipation coefficients a hundredfold apart: each bin as the oracle has
+    it."""
+    # the wind input is a few products of values good to a few ulp (4e-15);
+    # cancellation against the phase speed costs up to 1e-3 of that
+    tol = 1e-11
+    wl = configs.tiny(seed=5, mm=26, nm=24, om=25, pm=pm, land=False, winds=True)
+    o, d = make_pair(wl)
+    try:
+        th = (np.arange(pm) + 1 - 0.5 * (pm + 1)) * (2 * np.pi / pm)
+        diag = [np.arctan2(a, b) for a in (-1, 0, 1) for b in (-1, 0, 1) if a or b]
+        wdir = np.resize(np.concatenate([diag, th, np.arange(-36, 37) * np.pi / 36]),
+                         d.get("wdir").size)
+        for m in (o, d):
+            m.forcinginterpolate()
+        d.set("wdir", wdir)
+        o.raw("wdir")[1:] = wdir
+        assert np.array_equal(d.get("wdir"), o.get("wdir"))
+        d.sin_d12()
+        o.sin_d12()
+        x, y = d.get("ssin"), o.get("ssin")
+        big = np.abs(y) > 1e-6 * np.max(np.abs(y), axis=(1, 2), keepdims=True)
+        assert np.max(np.abs(x - y)[big] / np.abs(y[big])) <= tol
+        assert relerr(x, y) <= tol
+    finally:
+        d.close()
+        o.close()

@@ -113,7 +113,10 @@ __device__ inline SinPoint<T> sin_point(const DomainDev<T>& d, int j) {
 
 // One thread per (frequency, point), over its directions: the point's inputs
 // and tables are read once.  In FP64 cos(wdir - th) comes from the angle-sum
-// identity, one cosine and sine instead of a cosine per bin.
+// identity, one cosine and sine instead of a cosine per bin, except near right
+// angles: its sign chooses between dissipation coefficients a hundredfold
+// apart, and the identity's rounding (1e-16) may give 0 or the other sign
+// where the wind stands square to a bin.
 template <typename T>
 __global__ void k_sin_bins(DomainDev<T> d) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
@@ -131,10 +134,12 @@ __global__ void k_sin_bins(DomainDev<T> d) {
   for (int p = 0; p < d.pm; ++p) {
     const T ct = d.cth[p], st = d.sth[p];
     T cwt;
-    if constexpr (sizeof(T) == 8)
+    if constexpr (sizeof(T) == 8) {
       cwt = fma(cw, ct, sw * st);
-    else
+      if (fabs(cwt) < 1e-12) cwt = cos(wdir - d.th[p]);
+    } else {
       cwt = cos(wdir - d.th[p]);
+    }
     d.ssin[((size_t)o * d.pm + p) * d.ldi + j] =
         ssin_bin(s, logl2, cwt, cp0, ct, st, fkovg, T(d.sin_fac), T(d.fieldscale1),
                  T(d.fieldscale2), o);
