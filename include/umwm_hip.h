@@ -299,7 +299,9 @@ int umwm_hip_write_restart(umwm_domain* dom, const char* path);
 int umwm_hip_read_restart(umwm_domain* dom, const char* path);
 
 /* Scalars: sumt dts dta dtr dtamin cfllim cgmax mindelx dlnf dth bf1 bf2
- * first nsub.  Settable: sumt dts dtr_temp first, and keep_sources: set to 1
+ * first nsub, and since the domain's creation the substeps whose sources were
+ * integrated ahead of their rates (substeps_ahead) and those where that was
+ * tried and their time scales did not allow it (substeps_missed).  Settable: sumt dts dtr_temp first, and keep_sources: set to 1
  * (it cannot be unset) before the substep that reaches dtg, it makes the
  * fused path save that substep's E^n and incoming ustar (one more spectrum
  * of device memory), so that stress("ocn") at output time can rebuild the

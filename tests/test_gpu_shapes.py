@@ -178,3 +178,53 @@ def test_few_frequencies(om, pm, precision):
     finally:
         a.close()
         b.close()
+
+
+@pytest.mark.parametrize("precision", [8, 4])
+def test_lengths_kept_or_left_to_the_rates(precision):
+    """The third substep's time scales against the advective limit it was
+    guessed to take: below it (the guess is taken back), within the hundredth
+    that the sources' rounding is given (left to the rates) and above it (kept).
+    The guesses are counted, and the lengths are those of the plain order, bit
+    for bit.  With currents no guess is made."""
+    tol = 1e-12 if precision == 8 else 1e-5
+
+    def start(explim=None, currents=False):
+        wl = configs.tiny(3, 145, 140, 25, 36, winds=True, currents=currents, wspd=14.0)
+        wl.params.delx = wl.params.dely = 1e3
+        wl.params.dtg = 900.0
+        if explim:
+            wl.params.explim = explim
+        d = hip.Domain(wl.params, wl.grid_input(), wl.forcing_input(0), precision=precision)
+        d.init_jonswap(wl.jonswap)
+        d.stokes_drift(True)
+        d.forcinginput(wl.forcing_input(1))
+        return d, wl.params.explim
+
+    d, explim = start()
+    d.substeps(3)
+    # the limit holds throughout, so that the state does not depend on explim
+    limit = float(d.get("physics_time_step").min()) / d.scalar("dtamin")
+    assert limit > 2 and d.scalar("dts") == d.scalar("dtamin")
+    d.close()
+    for ratio, ahead, missed in ((0.97, 1, 1), (1.005, 1, 1), (1.5, 2, 0)):
+        a, b = (start(explim * ratio / limit)[0] for _ in range(2))
+        try:
+            b.set_tile(9, 4, 18, 2, 4)  # never ahead
+            for k in range(3):
+                assert a.substep() == b.substep(), (ratio, k)
+                assert a.scalar("dts") == b.scalar("dts")
+            assert (a.scalar("dts") == a.scalar("dtamin")) == (ratio > 1)
+            assert a.scalar("substeps_ahead") == ahead, ratio
+            assert a.scalar("substeps_missed") == missed, ratio
+            assert b.scalar("substeps_ahead") == b.scalar("substeps_missed") == 0
+            for name in ("e", "ustar", "physics_time_step", "wspd", "shelt", "oc"):
+                x, y = a.get(name), b.get(name)
+                assert np.linalg.norm(x - y) <= tol * np.linalg.norm(y), (ratio, name)
+        finally:
+            a.close()
+            b.close()
+    d, _ = start(currents=True)
+    d.substeps(4)
+    assert d.scalar("substeps_ahead") == d.scalar("substeps_missed") == 0
+    d.close()

@@ -1740,6 +1740,8 @@ int umwm_hip_get_scalar(umwm_domain* dom, const char* name, double* v) {
     if (n == "maxrot") { *v = s.maxrot; return 0; }
     if (n == "nsub") { *v = s.nsub; return 0; }
     if (n == "zerocurrents") { *v = s.anycur ? 0 : 1; return 0; }
+    if (n == "substeps_ahead") { *v = s.ahead; return 0; }
+    if (n == "substeps_missed") { *v = s.missed; return 0; }
     return fail(UMWM_ERR_UNKNOWN_FIELD, "unknown scalar: " + n);
   });
 }

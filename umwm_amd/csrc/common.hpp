@@ -54,6 +54,9 @@ struct Scalars {
   // the sources may be integrated over it while their rates are found; and
   // this substep was (k_stress clears it)
   int32_t spec, done;
+  // substeps whose sources were integrated ahead of their rates, and guesses
+  // of a length that the rates did not bear out
+  int32_t ahead, missed;
   // surrogate (FP32): this substep's sampled audit sums (error and weight)
   // and the domain's verdict on the previous substep's audit (0: the
   // network may serve, 1: every point takes the plain rates)

@@ -483,8 +483,9 @@ __device__ __forceinline__ Prefix prefix_at(const DomainDev<T>& d, const TabGen&
 }
 
 // A substep's sources are integrated ahead of its rates after one whose time
-// scales were this much longer than the advective limit (see k_integrate).
-constexpr double kSpecMargin = 1.05;
+// scales were this much longer than the advective limit (see k_integrate); the
+// length stands where they turn out longer than it by kSpecSlack.
+constexpr double kSpecMargin = 1.05, kSpecSlack = 1.01;
 
 // ---------------------------------------------------------------------
 // k_rates
@@ -994,16 +995,19 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
 // whatever the exact time scales are: the last workgroup then does k_rates'
 // bookkeeping and the substep's k_rates and plain k_integrate return at once.
 // Else they run as always and overwrite E*.  The rates share the
-// integration's wind input and dissipation, whose rounding differs from
-// k_rates' (1e-7 in FP32), so a length within 1e-5 of the limit is left to
-// k_rates; lengths are the same bits either way, the points' time scales
-// agree to that rounding.  k_rates + k_integrate, and this kernel (with FP64's
-// k_prefix) in their place, in us: 180,000 points x 37x36 FP32 258 + 454 ->
-// 479; 399,424 x 49x72 FP32 914 + 2,603 -> 2,916; 129,000 x 49x72 FP64 1,404 +
-// 3,536 -> 60 + 3,504; 42,000 x 37x36 FP64 199 + 466 -> 29 + 455.  The price of a wrong guess is this kernel's time, so one is made
-// only after a substep whose time scales were a twentieth above the limit
-// (kSpecMargin).  All waves of a point are in one workgroup here (one chunk,
-// gridDim.y = 1).
+// integration's wind input and dissipation, which k_rates groups otherwise: in
+// FP32 its dissipation differs by up to 6e-6 (the rounding of an exponent of
+// several tens; 1e-5 at sds_power = 4), and a rate is a difference in which
+// both may cancel.  So a length within kSpecSlack of the time scales is left to
+// k_rates: the two would have to cancel a thousandfold in a point's largest
+// rate before a length differed.  Lengths are the same bits then, the points'
+// time scales agree to that rounding.  k_rates + k_integrate, and this kernel
+// (with FP64's k_prefix) in their place, in us: 180,000 points x 37x36 FP32
+// 258 + 454 -> 479; 399,424 x 49x72 FP32 914 + 2,603 -> 2,916; 129,000 x 49x72
+// FP64 1,404 + 3,536 -> 60 + 3,504; 42,000 x 37x36 FP64 199 + 466 -> 29 + 455.
+// The price of a wrong guess is this kernel's time, so one is made only after a
+// substep whose time scales were a twentieth above the limit (kSpecMargin).
+// All waves of a point are in one workgroup here (one chunk, gridDim.y = 1).
 template <typename T, int DMAX, bool FULL, bool SUR, bool SPEC>
 __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restrict__ doms,
                                                    const BlockTask* __restrict__ tasks, int ng,
@@ -1360,7 +1364,7 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
     __builtin_amdgcn_s_waitcnt(0);  // complete before the arrival count
     if (atomicAdd(&sc->counter, 1u) != (unsigned)d.nblocks - 1) return;
     const double lim = okey_inv(~atomicExch(&sc->pts_key, 0ull));
-    const bool fits = lim * (1 - 1e-5) >= dtd;
+    const bool fits = lim >= kSpecSlack * dtd;
     if (fits) {
       sc->dts = dtd;
       sc->dta = dtd;
@@ -1372,6 +1376,7 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
     }
     sc->spec = fits ? 1 : 0;
     sc->done = fits ? 1 : 0;
+    if (fits) sc->ahead += 1; else sc->missed += 1;
     sc->counter = 0;
   }
 }
