@@ -129,3 +129,38 @@ def test_batch_forcing_currents_keep_equal_alone(prec, use_graph):
         b.close()
         for d in batch_doms + alone:
             d.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", [4, 8])
+@pytest.mark.parametrize("n,dx", [(3, 1e4), (7, 1e3)])
+def test_batch_past_the_launch_shapes_equals_alone(n, dx, prec):
+    """Default tiles choose their launch shape by the size of the whole launch:
+    members that by themselves are split over frequency chunks and direction
+    segments and together are not (three), or together run their sources ahead
+    of their rates (seven).  Every member equals itself run alone, bit for bit."""
+    def make(k):
+        wl = configs.tiny(40 + k, 64, 48, 25, 36, land=False, winds=True, wspd=9.0 + k)
+        wl.params.delx = wl.params.dely = dx
+        wl.params.dtg = 600.0
+        d = hip.Domain(wl.params, wl.grid_input(), wl.forcing_input(0), precision=prec)
+        d.init_jonswap(wl.jonswap)
+        d.stokes_drift(True)
+        d.forcinginput(wl.forcing_input(1))
+        return d
+
+    doms, alone = [make(k) for k in range(n)], [make(k) for k in range(n)]
+    b = hip.Batch(doms)
+    try:
+        for _ in range(2):
+            assert b.run_dtg() == [d.run_dtg() for d in alone]
+            for k, (x, y) in enumerate(zip(doms, alone)):
+                for name in ("e", "ustar", "taux_form", "hs_ice", "ht"):
+                    assert np.array_equal(x.get(name), y.get(name)), (k, name)
+                assert x.scalar("dts") == y.scalar("dts")
+        assert all(d.scalar("substeps_ahead") == 0 for d in alone)
+        assert any(d.scalar("substeps_ahead") > 0 for d in doms) == (n == 7)
+    finally:
+        b.close()
+        for d in doms + alone:
+            d.close()

@@ -1431,11 +1431,12 @@ struct AdvLoads {
 
 // Sums over the directions in the order of the moments (see Mom): `add`
 // takes directions in sequence, `group` ends a group.  t: e, e cos 2th,
-// e sin 2th and the stress partials; kSeq (FP32 where a wave takes every
-// direction) keeps the stress partials and the wave height as one running
-// FP32 sum each.
-template <typename T, bool kSeq>
+// e sin 2th and in FP64 the stress partials; FP32 keeps the stress partials
+// and the wave height as one running sum over all directions each.
+template <typename T>
 struct DirSums {
+  static constexpr bool kSeq = sizeof(T) == 4;
+  static constexpr int kGrouped = kSeq ? 3 : 5;
   T q[5], hs;
   double t[5];
   __device__ __forceinline__ void clear() {
@@ -1457,7 +1458,7 @@ struct DirSums {
   }
   __device__ __forceinline__ void group() {
 #pragma unroll
-    for (int i = 0; i < (kSeq ? 3 : 5); ++i) {
+    for (int i = 0; i < kGrouped; ++i) {
       t[i] += (double)q[i];
       q[i] = 0;
     }
@@ -1490,7 +1491,7 @@ __global__ __launch_bounds__(64) void k_moments(const DomainDev<T>* __restrict__
   const uint32_t vj = (uint32_t)j * (uint32_t)sizeof(T), rb = (uint32_t)ldi * (uint32_t)sizeof(T);
   const rsrc_t pe = freq_rsrc(d.e, o, pm, ldi);
   const int ng = dir_groups(pm), glen = uniform_div(pm + ng - 1, ng);
-  DirSums<T, true> S;
+  DirSums<T> S;
   S.clear();
   int gend = glen;
   for (int p = 0; p < pm; p += 4) {
@@ -1515,8 +1516,10 @@ __global__ __launch_bounds__(64) void k_moments(const DomainDev<T>* __restrict__
 // SPLIT: one workgroup per (frequency, 64 sea points), a wave per direction
 // group, for launches that would otherwise leave most of the GPU idle.
 // Else fw = blockDim / 64 frequencies per workgroup, a wave taking all
-// directions of one.  Both give the same moments bit for bit, and in FP64 the
-// same stress partials.
+// directions of one.  Both add in the same order, so that a domain's results
+// do not depend on what else is in the launch: the waves' groups are joined in
+// turn, and the running sums of FP32 are taken by one wave from the directions'
+// terms, which the others leave in LDS.
 template <typename T, int NB, bool SPLIT>
 __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_advect(
     const DomainDev<T>* __restrict__ doms, const BlockTask* __restrict__ tasks, int ng) {
@@ -1574,9 +1577,15 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_advect(
   const int plo = SPLIT ? wid * glen : 0, phi = SPLIT ? min(pm, plo + glen) : pm;
   // the moments of the new spectrum and the stress_vector_integral sums
   // over the directions of this frequency
-  constexpr bool kSeq = sizeof(T) == 4 && !SPLIT;
-  DirSums<T, kSeq> S;
+  constexpr bool kSeq = DirSums<T>::kSeq;
+  constexpr int NG = DirSums<T>::kGrouped;
+  DirSums<T> S;
   S.clear();
+  // SPLIT: the groups' sums, [ng][NG][64], and in FP32 the terms of the running
+  // sums, [pm][2][64] (advect_lds)
+  extern __shared__ double smem[];
+  [[maybe_unused]] const int lane = (int)threadIdx.x & 63;
+  [[maybe_unused]] T* const terms = reinterpret_cast<T*>(smem + ng * NG * 64);
   int gend = plo + glen;
   auto stress_acc = [&](int p, T v) {
     T ct, st, c2, s2;
@@ -1585,6 +1594,10 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_advect(
     T ss = sin_m(sf, sin_y(sf, ct, st), m);
     if (!prog) ss = fmax(ss, T(0));
     S.add(v, v * ss, ct, st, c2, s2);
+    if constexpr (SPLIT && kSeq) {
+      terms[2 * p * 64 + lane] = v;
+      terms[(2 * p + 1) * 64 + lane] = v * ss;
+    }
     if (p + 1 == gend) {  // wave-uniform
       S.group();
       gend += glen;
@@ -1709,15 +1722,26 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_advect(
   }
   S.group();  // the last group, where it is short
   if constexpr (SPLIT) {
-    __shared__ double red[8][5][64];
-    const int lane = (int)threadIdx.x & 63;
+    double* const red = smem + lane;
 #pragma unroll
-    for (int i = 0; i < 5; ++i) red[wid][i][lane] = S.t[i];
+    for (int i = 0; i < NG; ++i) red[(wid * NG + i) * 64] = S.t[i];
     __syncthreads();
     if (wid != 0) return;
     for (int q = 1; q < ng; ++q)
 #pragma unroll
-      for (int i = 0; i < 5; ++i) S.t[i] += red[q][i][lane];
+      for (int i = 0; i < NG; ++i) S.t[i] += red[(q * NG + i) * 64];
+    if constexpr (kSeq) {
+      S.q[3] = S.q[4] = S.hs = 0;
+#pragma unroll 4
+      for (int p = 0; p < pm; ++p) {
+        T ct, st, c2, s2;
+        cld4(dir4, p, ct, st, c2, s2);
+        const T wv = terms[(2 * p + 1) * 64 + lane];
+        S.q[3] = fma(wv, ct, S.q[3]);
+        S.q[4] = fma(wv, st, S.q[4]);
+        S.hs += terms[2 * p * 64 + lane];
+      }
+    }
   }
   if (valid) {
     const T icp = T(1) / cp_prev;
@@ -1729,7 +1753,6 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_advect(
     } else {
       tx = T(S.t[3]);
       ty = T(S.t[4]);
-      if constexpr (sizeof(T) == 4) hs = T(S.t[0]) * bld<T>(row_rsrc(d.kdk, o, ldi), vj);
     }
     store_mom(d, o, j, S.t[0], S.t[1], S.t[2]);
     const rsrc_t sp = freq_rsrc(d.sp, o, kPartials<T>, ldi);
@@ -1889,6 +1912,14 @@ void launch_spec(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, c
     hipLaunchKernelGGL((k_integrate<T, 4, true, false, true>), grid, block, 0, s, doms, tasks, h.ng2, 1);
 }
 
+// LDS of k_advect's split: at most 48 KB (FP32, 72 directions)
+template <typename T>
+size_t advect_lds(int ng, int pm) {
+  size_t n = (size_t)ng * DirSums<T>::kGrouped * 64 * sizeof(double);
+  if (DirSums<T>::kSeq) n += (size_t)pm * 2 * 64 * sizeof(T);
+  return n;
+}
+
 template <typename T, bool SUR>
 int launch_kernels(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, int omax, int pm,
                    int first, int rotation, const Shape& h, int nb, bool keep, hipStream_t s,
@@ -1943,10 +1974,11 @@ int launch_kernels(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks,
   const int ng = dir_groups(pm);
   if (h.split && ng <= 8) {
     const dim3 ga(ntasks, omax), block(64 * ng);
+    const size_t sh = advect_lds<T>(ng, pm);
     if (nb == 4)
-      hipLaunchKernelGGL((k_advect<T, 4, true>), ga, block, 0, s, doms, tasks, ng);
+      hipLaunchKernelGGL((k_advect<T, 4, true>), ga, block, sh, s, doms, tasks, ng);
     else
-      hipLaunchKernelGGL((k_advect<T, 2, true>), ga, block, 0, s, doms, tasks, ng);
+      hipLaunchKernelGGL((k_advect<T, 2, true>), ga, block, sh, s, doms, tasks, ng);
   } else {
     // one wave per (64 points, frequency), FW frequencies per workgroup (2
     // measured 1-2 % faster than 4 or 8 on 720x360)
