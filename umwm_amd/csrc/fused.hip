@@ -619,7 +619,10 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
         sok = valid ? pload(d.sur_ok, ldi, j) : 0;
         aud = d.sur_audit_stride > 0 && ((tk.local + nsub0) % d.sur_audit_stride) == 0;
         gate = sc->sur_closed == 0;
-        do_sur = __any(sok != 0) && (gate || aud);
+        // in a scalar register: the sweep's range follows from it, and with it
+        // in a vector one every buffer access became a loop over the lanes'
+        // descriptors (1,179 -> 877 us at 127,587 points x 49x72)
+        do_sur = __builtin_amdgcn_readfirstlane(__any(sok != 0) && (gate || aud)) != 0;
       }
     }
     T rmax = 0;
@@ -657,13 +660,17 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
         }
       }
     }
+    // (stores of lanes past the end are dropped rather than branched around:
+    // a divergent branch here moves what it shares with the loads of the
+    // moments, their descriptors, to vector registers)
     auto store_prefix = [&](int o, T pa0, T pac, T pas) {
       if constexpr (kStoredPrefix<T, SUR>) {
-        if (valid && grp == 0) {
+        if (grp == 0) {
           const rsrc_t pf = freq_rsrc(pfxb, o, 3, ldi);
-          bst(pf, vj, pa0);
-          bst(pf, vj, pac, rb);
-          bst(pf, vj, pas, 2 * rb);
+          const uint32_t v = valid ? vj : kDropOffset;
+          bst(pf, v, pa0);
+          bst(pf, v, pac, rb);
+          bst(pf, v, pas, 2 * rb);
         }
       }
     };
@@ -826,7 +833,8 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
       // the prefix of the diagnostic tail's bins, for k_integrate
       if (grp == 0) {
 #pragma unroll 4
-        for (int o = max(o0, omain); o < o1; ++o) {
+        for (int t = max(o0, omain); t < o1; ++t) {
+          const int o = __builtin_amdgcn_readfirstlane(t);  // see uniform_div
           store_prefix(o, T(hdth * P.a0), T(hdth * P.ac), T(hdth * P.as));
           P.add(k3dk_at(d, tg, o, vj), load_mom(momb, ldi, o, j));
         }
