@@ -96,3 +96,17 @@ def lane_loops(path, symbol):
 def test_scalar_descriptors(sweeps, kernel):
     path, table = sweeps
     assert lane_loops(path, table[kernel][0]) == 0
+
+
+# registers of a wave on a SIMD's 512, in steps of 8
+WAVES = {"k_rates<float, 9, true, false, true>": 3, "k_rates<float, 9, false, false, true>": 3,
+         "k_rates<float, 9, true, false, false>": 4, "k_rates<float, 36, true, true, false>": 3,
+         "k_integrate<float, 9, true, true, false>": 3, "k_integrate<float, 12, true, false, false>": 3,
+         "k_integrate<float, 9, true, false, true>": 3, "k_rates<double, 9, true, false, false>": 2}
+
+
+@pytest.mark.parametrize("kernel", WAVES)
+def test_waves_per_simd(sweeps, kernel):
+    _, table = sweeps
+    vgprs = (table[kernel][1] + 7) // 8 * 8
+    assert 512 // vgprs >= WAVES[kernel], vgprs

@@ -494,8 +494,17 @@ constexpr double kSpecMargin = 1.05, kSpecSlack = 1.01;
 // p0 + DMAX - 1 of direction group slot % ng and the frequencies of chunk
 // slot / ng; slots past ng * chunks are idle.  SUR launches keep all of a
 // point's waves in one workgroup (one chunk, gridDim.y = 1).
+// The moments of a frequency enter the prefix at the end of its iteration.
+// Carried from the one before, they and the next ones' cost six registers more
+// than loaded at its start, which the narrow FP32 sweeps have (9 directions:
+// 289 against 303 us at 179,813 points x 37x36); the others then keep a wave a
+// SIMD, some with the bound of kWaves: 36 directions in pairs 222 -> 190 us
+// there, 280 -> 206 at 93,870 x 49x72, the surrogate's 9 876 -> 862 at 127,587.
+template <typename T, int DMAX, bool PAIR, bool SUR>
+constexpr int kWaves = sizeof(T) == 4 && ((SUR && DMAX == 9) || (!SUR && PAIR && DMAX == 36)) ? 3 : 2;
+
 template <typename T, int DMAX, bool FULL, bool PAIR, bool SUR>
-__global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ doms,
+__global__ __launch_bounds__(512, (kWaves<T, DMAX, PAIR, SUR>)) void k_rates(const DomainDev<T>* __restrict__ doms,
                                                const BlockTask* __restrict__ tasks, int first,
                                                int rot_all, int ng, int chunks) {
   extern __shared__ double smem[];
@@ -645,9 +654,9 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
     // rather than holding DMAX more scalar registers
     [[maybe_unused]] uint32_t rc[DMAX];
     FreqTab<T> tc;
-    Mom<double> mo = load_mom(momb, ldi, o0, j);
-    [[maybe_unused]] double k3 = 0;
-    if constexpr (!kDerive) k3 = k3dk_at(d, tg, o0, vj);
+    constexpr bool kAhead = sizeof(T) == 4 && !SUR && DMAX <= 9;  // see kWaves
+    Mom<double> mo;
+    if constexpr (kAhead) mo = load_mom(momb, ldi, o0, j);
     {
       const rsrc_t ep = freq_rsrc(eb, o0, pm, ldi);
 #pragma unroll
@@ -689,9 +698,9 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
           for (int q = 0; q < DMAX; ++q) rn[q] = bld_u16(FULL || q < nd ? rp : rz, vj2 + dirp(q) * rb2);
         }
       }
-      const Mom<double> mn = load_mom(momb, ldi, on, j);
-      [[maybe_unused]] double k3n = 0;
-      if constexpr (!kDerive) k3n = k3dk_at(d, tg, on, vj);
+      const Mom<double> mn = load_mom(momb, ldi, kAhead ? on : o, j);
+      T k3 = 0;
+      if constexpr (!kDerive) k3 = bld<T>(row_rsrc(d.k3dk, o, ldi), vj);
       float knext = 0.f;
       if constexpr (kDerive) {
         knext = tg.load_k(o + 4);
@@ -816,9 +825,8 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
           }
         }
       }
-      P.add(k3, mo);
+      P.add(k3, kAhead ? mo : mn);
       mo = mn;
-      if constexpr (!kDerive) k3 = k3n;
 #pragma unroll
       for (int q = 0; q < DMAX; ++q) ec[q] = en[q];
       if constexpr (SUR) {
@@ -1016,8 +1024,10 @@ __global__ __launch_bounds__(512) void k_rates(const DomainDev<T>* __restrict__ 
 // The price of a wrong guess is this kernel's time, so one is made only after a
 // substep whose time scales were a twentieth above the limit (kSpecMargin).
 // All waves of a point are in one workgroup here (one chunk, gridDim.y = 1).
+// Twelve directions in FP32 load the moments late and are bounded to three
+// waves a SIMD as in k_rates: 519 -> 461 us at 179,813 points x 37x36.
 template <typename T, int DMAX, bool FULL, bool SUR, bool SPEC>
-__global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restrict__ doms,
+__global__ __launch_bounds__(512, (sizeof(T) == 4 && !SUR && DMAX == 12 ? 3 : 2)) void k_integrate(const DomainDev<T>* __restrict__ doms,
                                                    const BlockTask* __restrict__ tasks, int ng,
                                                    int chunks) {
   const BlockTask tk = tasks[blockIdx.x];
@@ -1144,10 +1154,11 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
   // the moments it is summed from
   [[maybe_unused]] Mom<T> pc{};
   [[maybe_unused]] Prefix P;
+  [[maybe_unused]] constexpr bool kAhead = DMAX != 12;  // see kWaves
   [[maybe_unused]] Mom<double> mo{};
   if constexpr (!kStored) {
     P = prefix_at(d, tg, o0, j, vj);
-    mo = load_mom(momb, ldi, o0, j);
+    if constexpr (kAhead) mo = load_mom(momb, ldi, o0, j);
   } else if constexpr (kDerive) {
     pc = load_mom(pfxb, ldi, o0, j);
   }
@@ -1174,7 +1185,7 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
       if constexpr (kStored)
         pn = load_mom(pfxb, ldi, on, j);
       else
-        mn = load_mom(momb, ldi, on, j);
+        mn = load_mom(momb, ldi, kAhead ? on : o, j);
       tg.table(o, tc);
     } else {
       load_tab<kSweepSlots>(ftab, ldi, o, vr, tc);
@@ -1347,7 +1358,7 @@ __global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restric
     }
     if constexpr (!kStored) {
       const double k3 = k * k * tc[FT_KDK];  // k^3 dk
-      P.add(k3, mo);
+      P.add(k3, kAhead ? mo : mn);
       mo = mn;
     }
     if constexpr (kDerive) {
