@@ -228,3 +228,30 @@ def test_lengths_kept_or_left_to_the_rates(precision):
     d.substeps(4)
     assert d.scalar("substeps_ahead") == d.scalar("substeps_missed") == 0
     d.close()
+
+
+@pytest.mark.parametrize("grid", [(270, 250, 7, 28), (270, 250, 6, 32), (190, 180, 7, 68),
+                                  (250, 225, 6, 44)])
+def test_nine_directions_with_idle_slots(grid):
+    """FP32 grids large enough for waves of nine directions that do not divide
+    pm, which run their sources ahead too: the bits of the plain order."""
+    mm, nm, om, pm = grid
+    wl = configs.tiny(4, mm, nm, om, pm, land=False, winds=True, wspd=14.0)
+    wl.params.delx = wl.params.dely = 500.0
+    a, b = (hip.Domain(wl.params, wl.grid_input(), wl.forcing_input(0), precision=4)
+            for _ in range(2))
+    try:
+        assert (a.im + 63) // 64 * -(-pm // 9) >= 4096
+        b.set_tile(9, -(-pm // 9), 9, -(-pm // 9), 4)  # never ahead
+        for d in (a, b):
+            d.init_jonswap(wl.jonswap)
+            d.stokes_drift(True)
+            d.forcinginput(wl.forcing_input(1))
+        for _ in range(6):
+            assert a.substep() == b.substep()
+        assert a.scalar("substeps_ahead") > 0 and b.scalar("substeps_ahead") == 0
+        for name in ("e", "es", "ustar"):
+            assert np.array_equal(a.get(name), b.get(name)), name
+    finally:
+        a.close()
+        b.close()

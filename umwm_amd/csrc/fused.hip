@@ -1918,12 +1918,15 @@ void launch_integrate(const DomainDev<T>* doms, const BlockTask* tasks, int ntas
 }
 
 template <typename T>
-void launch_spec(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, const Shape& h,
-                 hipStream_t s) {
+void launch_spec(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, int pm,
+                 const Shape& h, hipStream_t s) {
   const dim3 grid(ntasks), block(64 * h.w2);
   if constexpr (kStoredPrefix<T, false>)
     hipLaunchKernelGGL((k_prefix<T>), grid, dim3(64), 0, s, doms, tasks);
-  if (h.D2 == 9)
+  if (h.ng2 * h.D2 != pm) {  // FP32 waves of nine, see choose_shape
+    if constexpr (sizeof(T) == 4)
+      hipLaunchKernelGGL((k_integrate<T, 9, false, false, true>), grid, block, 0, s, doms, tasks, h.ng2, 1);
+  } else if (h.D2 == 9)
     hipLaunchKernelGGL((k_integrate<T, 9, true, false, true>), grid, block, 0, s, doms, tasks, h.ng2, 1);
   else if (h.D2 == 6)
     hipLaunchKernelGGL((k_integrate<T, 6, true, false, true>), grid, block, 0, s, doms, tasks, h.ng2, 1);
@@ -1946,7 +1949,7 @@ int launch_kernels(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks,
   if (ev) (void)hipEventRecord(ev[0], s);
   if constexpr (!SUR) {
     // a timed substep keeps the kernels apart
-    if (h.spec && !first && !rotation && !ev) launch_spec<T>(doms, tasks, ntasks, h, s);
+    if (h.spec && !first && !rotation && !ev) launch_spec<T>(doms, tasks, ntasks, pm, h, s);
   }
 #define UMWM_RATES(D_)                                                                       \
   case D_: launch_rates<T, D_, SUR>(doms, tasks, ntasks, pm, first, rotation, h, s); break;
@@ -2042,14 +2045,24 @@ int waves_for(int slots) {
 //   2,809 points  FP64 284 -> 75   FP32 104 -> 41
 //   11,449 points FP64 303 -> 188  FP32 108 -> 78
 // D divides pm: masked slots cost as much as full ones (pm = 48 at 13,924
-// points, D = 6 against 9: FP64 633 -> 310 us, FP32 125 -> 98).
+// points, D = 6 against 9: FP64 633 -> 310 us, FP32 125 -> 98).  Where only
+// four would, an FP32 grid whose waves of nine fill the GPU at the four a SIMD
+// holds takes nine, the last wave with idle slots: a frequency's tables weigh
+// more on a narrow wave than those slots do.  Substeps of 79,921 points in us,
+// D = 4 -> 9: 37x28 590 -> 558, 37x40 916 -> 879, 37x44 900 -> 911, 37x56
+// 1,110 -> 1,050, 37x68 1,317 -> 1,160; 179,813 points x 37x28 1,308 -> 1,231.
+// At 38,936 points the count of waves decides (37x28 339 and 312, 37x44 472 and
+// 513, 37x64 601 and 626, 37x68 680 and 643).  FP64, whose directions weigh
+// more, keeps four: 867 us against 914 at 38,936 points x 37x28, 1,557 against
+// 1,549 at 79,921.
 // k_advect's split pays while its waves (one per frequency and point block)
 // leave the GPU short of work: 2,809 points FP64 29.7 -> 25.7, FP32 25.6 ->
 // 19.2 us; 11,449 points 84.9 -> 92.9 and 39.4 -> 49.1 us.
 constexpr int kSweepWaves = 1536;
 constexpr int kAdvectWaves = 4096;
+constexpr int kFullWaves = 4096;
 
-Shape choose_shape(const Tile& t, int ntasks, int omax, bool sur) {
+Shape choose_shape(const Tile& t, int ntasks, int omax, bool sur, bool fp32) {
   Shape h{t.D1, t.W1, 1, t.W1, t.D2, t.W2, 1, t.W2, true, false, false};
   const int pm = t.pmax;
   // the network's checks need all of a point's waves in one workgroup; wide
@@ -2067,8 +2080,9 @@ Shape choose_shape(const Tile& t, int ntasks, int omax, bool sur) {
   };
   int D = pm % 9 == 0 ? 9 : pm % 6 == 0 ? 6 : 4;
   if (ntasks * (pm / D) * chunks(D) < kSweepWaves / 2) D = 2;
+  if (D == 4 && fp32 && ntasks * ((pm + 8) / 9) >= kFullWaves) D = 9;
   h.D1 = h.D2 = D;
-  h.ng1 = h.ng2 = pm / D;
+  h.ng1 = h.ng2 = (pm + D - 1) / D;
   h.c1 = h.c2 = chunks(D);
   h.w1 = h.w2 = waves_for(h.ng1 * h.c1);
   h.paired = false;  // one order of operations whatever D
@@ -2113,7 +2127,7 @@ int launch_fused(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, i
       tile.W2 *= 2;
     }
   }
-  const Shape h = choose_shape(tile, ntasks, omax, sur);
+  const Shape h = choose_shape(tile, ntasks, omax, sur, sizeof(T) == 4);
   if constexpr (std::is_same_v<T, float>) {
     if (sur)
       return launch_kernels<T, true>(doms, tasks, ntasks, omax, tile.pmax, first, rotation, h,
