@@ -331,7 +331,12 @@ int umwm_hip_synchronize(umwm_domain* dom);
  * rates with D1 directions per thread (6, 9, 18 or 36) and W1 waves,
  * integrate with D2 (3, 6, 9, 12 or 18) and W2 waves (W in 1..8,
  * D*W >= pm), and advect prefetching NB directions ahead (2 or 4).
- * Used by the autotuner (umwm_amd/autotune.py). */
+ * A new domain has the default tile, D1 = 9 (else 18 or 36) and D2 = 9 (else
+ * 12 or 18), the first that at most 8 waves cover, and NB = 2.  While that one
+ * is set, also when it is set again, it stands for a launch shape by the size of
+ * the grid: where pm <= 72 the sweeps' directions a wave and their split over
+ * frequencies then follow from it, not from these values.  Any other tile is
+ * launched as it is.  Used by the autotuner (umwm_amd/autotune.py). */
 int umwm_hip_set_tile(umwm_domain* dom, const int32_t tile[5]);
 int umwm_hip_get_tile(const umwm_domain* dom, int32_t tile[5]);
 
@@ -356,7 +361,8 @@ int umwm_hip_batch_run_dtg(umwm_batch* b, int use_graph, int32_t* nsub);
  * receives member k's substeps taken this dtg (array of n members, may be
  * NULL). */
 int umwm_hip_batch_substeps(umwm_batch* b, int32_t n, int use_graph, int32_t* nsub);
-/* Tile shape of the batch's fused launches (layout of umwm_hip_set_tile). */
+/* Tile of the batch's fused launches (layout and default as in
+ * umwm_hip_set_tile, for the largest pm of the batch). */
 int umwm_hip_batch_tile(const umwm_batch* b, int32_t out[5]);
 /* Sets the batch's tile shape (same rules as umwm_hip_set_tile over the
  * largest pm of the batch).  Members are launched in groups of equal pm;

@@ -139,3 +139,10 @@ def test_tile_candidates():
     assert autotune.candidates(36, (6, 9, 18, 36)) == [(6, 6), (9, 4), (18, 2), (36, 1)]
     assert autotune.candidates(72, (6, 9)) == [(9, 8)]
     assert all(w <= 8 for _, w in autotune.candidates(24, autotune.INTEGRATE_D))
+
+
+def test_default_tile():
+    assert autotune.default_tile(36) == (9, 4, 9, 4, 2)
+    assert autotune.default_tile(72) == (9, 8, 9, 8, 2)
+    assert autotune.default_tile(76) == (18, 5, 12, 7, 2)
+    assert autotune.default_tile(120) == (18, 7, 18, 7, 2)

@@ -5,7 +5,7 @@ moments formed after a spectrum is set against those the advection leaves."""
 import numpy as np
 import pytest
 
-from umwm_amd import configs, hip
+from umwm_amd import autotune, configs, hip
 
 pytestmark = pytest.mark.gpu
 
@@ -255,3 +255,71 @@ def test_nine_directions_with_idle_slots(grid):
     finally:
         a.close()
         b.close()
+
+
+@pytest.mark.parametrize("precision", [8, 4])
+@pytest.mark.parametrize("grid", GRIDS)
+def test_default_shape_equals_given_tile(grid, precision):
+    """As test_default_shape_equals_explicit_tile, under a tile that is not the
+    default and is therefore launched as it is given: the same bits."""
+    pm = grid[3]
+    a, b = fresh(grid, precision), fresh(grid, precision)
+    try:
+        D = 9 if pm <= 72 else 18
+        b.set_tile(D, -(-pm // D), D, -(-pm // D), 4)
+        assert b.tile()[4] == 4
+        for n in (1, 3):
+            assert a.substeps(n) == b.substeps(n)
+        for name in ("e", "ustar"):
+            assert np.array_equal(a.get(name), b.get(name)), name
+    finally:
+        a.close()
+        b.close()
+
+
+def test_the_default_tile_stands_for_the_choice():
+    """Setting the tile that was read, or the default after another, leaves the
+    launch shape to the grid, seen by the sources that run ahead with four
+    directions a wave; a batch likewise."""
+    doms = [wide(1e3, 8, 28) for _ in range(2)]
+    d = doms[0]
+    batch = hip.Batch(doms[1:])
+    try:
+        d.substeps(2)
+        batch.substeps(2)
+
+        def ahead(m, step):
+            n = m.scalar("substeps_ahead")
+            step(2)
+            return m.scalar("substeps_ahead") - n
+
+        assert d.tile() == autotune.default_tile(28) == (9, 4, 9, 4, 2)
+        assert ahead(d, d.substeps) == 2
+        d.set_tile(*d.tile())
+        assert ahead(d, d.substeps) == 2
+        d.set_tile(9, 4, 9, 4, 4)
+        assert d.tile() == (9, 4, 9, 4, 4) and ahead(d, d.substeps) == 0
+        d.set_tile(*autotune.default_tile(28))
+        assert ahead(d, d.substeps) == 2
+        m = doms[1]
+        assert ahead(m, batch.substeps) == 2
+        batch.set_tile(9, 4, 18, 2, 2)
+        assert ahead(m, batch.substeps) == 0
+        batch.set_tile(*autotune.default_tile(28))
+        assert ahead(m, batch.substeps) == 2
+    finally:
+        batch.close()
+        for x in doms:
+            x.close()
+
+
+def test_autotune_keeps_the_default_where_it_is_faster():
+    """On a small grid the shape split over frequency chunks takes half the
+    time of any tile, whose kernels the tuner times one by one."""
+    d = fresh((64, 48, 37, 36), 8)
+    try:
+        d.substeps(3)
+        choice, table = autotune.autotune(d, steps=3)
+        assert choice == d.tile() == autotune.default_tile(36) and len(table) == 4
+    finally:
+        d.close()

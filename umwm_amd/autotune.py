@@ -2,15 +2,20 @@
 
 k_rates and k_integrate give each thread D consecutive directions of one
 sea point and W = ceil(pm / D) waves per workgroup; k_advect keeps NB
-directions of gathers in flight per wave.  Larger D means fewer
-cross-wave exchanges and more work per thread but more registers; larger
-NB means more loads in flight but fewer resident waves.  The best shape
-depends on pm, the precision and the grid size, so it is measured: each
-candidate runs a few live substeps with HIP-event timing and the fastest
-shape per kernel is kept.  Candidates only change the order of
-directional sums, so the model state advances normally while tuning.
+directions of gathers in flight per wave.  Larger D means that a
+frequency's tables are formed for more directions at once but more
+registers; larger NB means more loads in flight but fewer resident waves.
+The best shape depends on pm, the precision and the grid size, so it is
+measured: each candidate runs a few live substeps with HIP-event timing
+and the fastest shape per kernel is kept.  Whole substeps then decide
+between that tile and the default one, which splits the sweeps of small
+grids over frequency and integrates the sources ahead of their rates where
+it can, neither of which the kernels' own times show.  Candidates only
+change the order of directional sums, so the model state advances normally
+while tuning.
 """
 import math
+import time
 
 RATES_D = (6, 9, 18, 36)
 INTEGRATE_D = (3, 6, 9, 12, 18)
@@ -24,6 +29,26 @@ def candidates(pm, ds):
         if 1 <= W <= 8:
             out.append((D, W))
     return out
+
+
+def default_tile(pm):
+    """The tile of a new domain, which stands for a launch shape by the size
+    of its grid (umwm_hip_set_tile)."""
+    def first(ds):
+        return next((D, math.ceil(pm / D)) for D in ds if math.ceil(pm / D) <= 8)
+    return first((9, 18, 36)) + first((9, 12, 18, 36)) + (2,)
+
+
+def substep_time(dom, tile, steps):
+    """Seconds of a live substep under `tile`, back to back; None where the
+    time of the forcing window ran out meanwhile (what is left does nothing)."""
+    dom.set_tile(*tile)
+    dom.substeps(1)  # captures the launch
+    n0 = dom.scalar("nsub")
+    t0 = time.perf_counter()
+    dom.substeps(steps)
+    t = (time.perf_counter() - t0) / steps
+    return t if dom.scalar("nsub") == n0 + steps else None
 
 
 def autotune(dom, steps=3, verbose=None):
@@ -54,7 +79,17 @@ def autotune(dom, steps=3, verbose=None):
     best1 = min(c1, key=lambda a: min(t[0] for x, _, _, t in table if x == a))
     best2 = min(c2, key=lambda b: min(t[1] for _, y, _, t in table if y == b))
     best3 = min(ADVECT_NB, key=lambda nb: min(t[2] for _, _, z, t in table if z == nb))
-    choice = (best1[0], best1[1], best2[0], best2[1], best3)
+    choice, default = (best1[0], best1[1], best2[0], best2[1], best3), default_tile(pm)
+    if choice != default:
+        # in turn, the faster of two passes each; the default unless the other
+        # is shown to be faster
+        t = [(substep_time(dom, choice, steps), substep_time(dom, default, steps))
+             for _ in range(2)]
+        t = [(a, b) for a, b in t if a and b]
+        if not t or min(b for _, b in t) <= min(a for a, _ in t):
+            choice = default
+        if verbose:
+            verbose(f"autotune: substeps {t} s, {choice}")
     dom.set_tile(*choice)
     return choice, table
 

@@ -155,6 +155,13 @@ Tile choose_tile(int pm) {
   return t;
 }
 
+// Whether a caller's tile is the default for pm, whose launch shape the
+// sweeps choose by the grid (Tile::chosen).
+bool is_default(const Tile& t, int pm) {
+  const Tile c = choose_tile(pm);
+  return t.D1 == c.D1 && t.W1 == c.W1 && t.D2 == c.D2 && t.W2 == c.W2 && t.NB == c.NB;
+}
+
 bool tile_ok(const Tile& t, int pm) {
   const bool d1 = t.D1 == 6 || t.D1 == 9 || t.D1 == 18 || t.D1 == 36;
   const bool d2 = t.D2 == 3 || t.D2 == 6 || t.D2 == 9 || t.D2 == 12 || t.D2 == 18;
@@ -1796,7 +1803,7 @@ int umwm_hip_set_tile(umwm_domain* dom, const int32_t tile[5]) {
     if (!tile_ok(t, D.S.pm))
       return fail(UMWM_ERR_ARGUMENT, "tile needs D1 in {6,9,18,36}, D2 in {3,6,9,12,18}, "
                                      "W in 1..8, D*W >= pm, NB in {2,4}");
-    t.chosen = true;
+    t.chosen = !is_default(t, D.S.pm);
     D.tile = t;
     return 0;
   });
@@ -2143,14 +2150,14 @@ int umwm_hip_batch_set_tile(umwm_batch* b, const int32_t tile[5]) {
     for (auto* D : B->doms) pmmax = std::max(pmmax, D->S.pm);
     Tile t = tile_from(tile, pmmax);
     if (!tile_ok(t, pmmax)) return fail(UMWM_ERR_ARGUMENT, "tile does not cover pm");
-    t.chosen = true;
+    t.chosen = !is_default(t, pmmax);
     B->tile = t;
     for (auto& g : B->groups) {
       Tile gt = t;  // same D and NB, waves for this class's pm
       gt.W1 = (g.pm + t.D1 - 1) / t.D1;
       gt.W2 = (g.pm + t.D2 - 1) / t.D2;
       gt.pmax = g.pm;
-      g.tile = tile_ok(gt, g.pm) ? gt : choose_tile(g.pm);
+      g.tile = t.chosen && tile_ok(gt, g.pm) ? gt : choose_tile(g.pm);
     }
     if (B->exec) {  // the captured graph holds the old launch shape
       (void)hipGraphExecDestroy(B->exec);

@@ -23,8 +23,8 @@ struct Tile {
   // pm of the domains launched together (a batch launches each pm class
   // on its own); W D = pmax selects the sweeps' mask-free variants
   int pmax = 36;
-  // set by the caller: the sweeps run as set (else choose_shape in fused.hip
-  // may split them further where the grid is small)
+  // another than the default was set: the sweeps run as set (else choose_shape
+  // in fused.hip shapes them by the size of the grid)
   bool chosen = false;
 };
 
