@@ -1,9 +1,12 @@
 """Spectra and Stokes profiles on their way to and from the host: what is set
 is what is read, over the sizes where the staged transfers change."""
+import ctypes as C
+import os
+
 import numpy as np
 import pytest
 
-from umwm_amd import configs, hip
+from umwm_amd import build, configs, hip
 
 pytestmark = pytest.mark.gpu
 
@@ -61,3 +64,31 @@ def test_stokes_rows(grid):
         assert np.all(np.abs(us[1:] * vs[:1] - vs[1:] * us[:1]) <= 0.2 * speed[1:] * speed[:1])
     finally:
         d.close()
+
+
+def free_bytes():
+    hiprt = C.CDLL(os.path.join(build.ROCM, "lib", "libamdhip64.so"))
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hiprt.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.parametrize("precision", [8, 4])
+def test_transfers_allocate_nothing(precision):
+    """What get and set need on the device comes with the domain: a program
+    that reads and sets fields between substeps_noalloc calls allocates none."""
+    def transfers(d):
+        e = d.get("e")
+        d.set("e", e)
+        d.get("us")
+
+    d = domain(14, 13, 37, 36, precision)
+    transfers(d)  # the runtime's own first use
+    big = domain(83, 71, 31, 44, precision)
+    try:
+        before = free_bytes()
+        transfers(big)
+        assert free_bytes() == before
+    finally:
+        d.close()
+        big.close()

@@ -242,6 +242,27 @@ int launch_end(DomainImpl<T>& D, bool stokes, bool diag) {
   return launch_integrals<T>(D.d, D.tasks, D.ntasks, D.end_d, D.h.lm, stokes, diag, D.stream);
 }
 
+// Staging for D's spectra on their way to and from the host: all points if
+// they fit, else whole groups of 64, and fewer where the device has no room for
+// that.  Allocated with the domain, so that get and set allocate nothing.
+constexpr size_t kStageBytes = 32u << 20;
+
+template <typename T>
+int alloc_stage(DomainImpl<T>& D) {
+  const size_t bins = (size_t)D.h.om * D.h.pm;
+  size_t pts = std::max<size_t>(kStageBytes / (bins * sizeof(double)) / 64 * 64, 64);
+  pts = std::max<size_t>(std::min<size_t>(pts, D.h.im), 1);
+  for (; pts; pts /= 2) {
+    D.stage = D.arena.template alloc<double>(pts * bins);
+    if (D.stage) {
+      D.stage_pts = (int)pts;
+      return 0;
+    }
+    (void)hipGetLastError();
+  }
+  return fail(UMWM_ERR_NOMEM, "device allocation for a spectrum's transfer failed");
+}
+
 template <typename T>
 int create_impl(const umwm_params& P, const umwm_grid_input* g, const umwm_forcing_input* f0,
                 DomainImpl<T>*& out) {
@@ -572,6 +593,7 @@ int create_impl(const umwm_params& P, const umwm_grid_input* g, const umwm_forci
   }
   UMWM_HIP_TRY(hipMemcpyAsync(D->d, &h, sizeof(DomainDev<T>), hipMemcpyHostToDevice, s));
   D->tile = choose_tile(pm);
+  if ((rc = alloc_stage(*D))) { delete D; return rc; }
   for (auto& e : D->ev) UMWM_HIP_TRY(hipEventCreate(&e));
   UMWM_HIP_TRY(hipStreamSynchronize(s));
   // stokes_drift('init') on the cold-start spectrum, as umwm_initialize does
@@ -932,27 +954,6 @@ int64_t field_size(const DomainImpl<T>& D, FieldKind k) {
   return 0;
 }
 
-// Staging for D's spectra: all points if they fit, else whole groups of 64,
-// and fewer where the device has no room for that.
-constexpr size_t kStageBytes = 32u << 20;
-
-template <typename T>
-int ensure_stage(DomainImpl<T>& D) {
-  if (D.stage) return 0;
-  const size_t point = (size_t)D.h.om * D.h.pm * sizeof(double);
-  size_t pts = std::max<size_t>(kStageBytes / point / 64 * 64, 64);
-  pts = std::min<size_t>(pts, D.h.im);
-  for (; pts; pts /= 2) {
-    D.stage = D.arena.template alloc<double>(pts * (size_t)D.h.om * D.h.pm);
-    if (D.stage) {
-      D.stage_pts = (int)pts;
-      return 0;
-    }
-    (void)hipGetLastError();
-  }
-  return fail(UMWM_ERR_NOMEM, "device allocation for a spectrum's transfer failed");
-}
-
 template <typename T>
 int get_field_impl(DomainImpl<T>& D, const std::string& name, double* buf, int64_t n) {
   FieldRef r;
@@ -967,7 +968,6 @@ int get_field_impl(DomainImpl<T>& D, const std::string& name, double* buf, int64
   switch (r.kind) {
     case F_SPEC: {
       // device [o][p][ldi] -> reference (om,pm,im) column-major
-      if (int rc = ensure_stage(D)) return rc;
       const size_t np = (size_t)h.om * h.pm;
       for (int j0 = 0; j0 < h.im; j0 += D.stage_pts) {
         const int nj = std::min(D.stage_pts, h.im - j0);
@@ -1005,7 +1005,6 @@ int get_field_impl(DomainImpl<T>& D, const std::string& name, double* buf, int64
       // staging holds: a copy of its own for each had cost the bus's latency
       // a level, 0.49 ms for 42 levels of 171 points, now
       // 0.03
-      if (int rc = ensure_stage(D)) return rc;
       const size_t room = (size_t)D.stage_pts * h.om * h.pm, row = im * sizeof(double);
       const size_t lm = std::max(h.lm, 1), nl = std::max<size_t>(std::min(lm, room / im), 1);
       for (size_t l = 0; l < lm; l += nl) {
@@ -1050,7 +1049,6 @@ int set_field_impl(DomainImpl<T>& D, const std::string& name, const double* buf,
   std::lock_guard<std::mutex> turn(D.stage_mutex);
   switch (r.kind) {
     case F_SPEC: {
-      if (int rc = ensure_stage(D)) return rc;
       const size_t np = (size_t)h.om * h.pm;
       for (int j0 = 0; j0 < h.im; j0 += D.stage_pts) {
         const int nj = std::min(D.stage_pts, h.im - j0);

@@ -102,8 +102,7 @@ struct DomainImpl : DomainBase {
   bool use_graph = true;
   EndDev end{};              // diag and Stokes outputs
   EndDev* end_d = nullptr;   // device copy (array of one)
-  // staging for spectra on their way to and from the host: allocated at the
-  // first such transfer, at most kStageBytes, of stage_pts points
+  // staging for spectra on their way to and from the host, of stage_pts points
   double* stage = nullptr;
   int stage_pts = 0;
   std::mutex stage_mutex;  // threads may read one domain's fields at once
