@@ -34,7 +34,8 @@
 // prefetches the next frequency's spectrum (and, in FP32, its tables) while
 // computing the current one.  Launches whose waves all hold exactly DMAX
 // directions take a variant without per-slot masks, and k_rates one that
-// pairs each direction with its opposite (caller-chosen tiles).
+// pairs each direction with its opposite (given tiles, the surrogate and spectra
+// wider than 72 directions).
 //
 // snl(o) = bf1r(o) X(o+1) + bf2r(o) X(o+2) - snl_fac X(o), X = sds e
 // (src/umwm_source_functions.F90:165-171) is folded into the integration
@@ -53,7 +54,7 @@
 // computed once per thread, directions reached with a scalar offset.  The
 // FP32 sweeps derive their (frequency, point) tables from k and the depth
 // (TabGen); FP64 reads an 8-value record per lane (four 16-byte loads).
-// The directional moments with the x stress partial are a 4-value record.
+// The directional moments and the stress partials are planes.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -379,10 +380,11 @@ struct Tr<double> {
     return fm64::log_t(x, sFm64 + fm64::kExpTabLen, sFm64 + fm64::kExpTabLen + fm64::kLogTabLen);
   }
   __device__ static __forceinline__ double ex(double x) { return fm64::exp_t(x, sFm64); }
-  // k_rates' forms: its logarithms are of |e|, k and cf (finite, >= 0) and a
-  // NaN spectral value reaches its rate through e itself, so the special
-  // cases reduce to log 0 = -inf (0.9 ms less per hurricane member-substep;
-  // in k_integrate the same change added spills and cost 2.7 ms)
+  // The forms of the dissipation: its logarithms are of |e|, k and cf (finite,
+  // >= 0) and a NaN spectral value reaches its rate or its X through e itself,
+  // so the special cases reduce to log 0 = -inf (k_rates 0.9 ms less per
+  // hurricane member-substep).  The integration's exponential and the
+  // diagnostic tail keep them
   __device__ static __forceinline__ double lg_nn(double x) {
     return fm64::log_t<false>(x, sFm64 + fm64::kExpTabLen,
                               sFm64 + fm64::kExpTabLen + fm64::kLogTabLen);
@@ -452,8 +454,8 @@ struct Prefix {
 
 // Whether k_rates leaves the prefix for k_integrate or k_integrate sums it
 // again: in FP64 that spilled (155 -> 350 us at 2,852 points) and in the
-// surrogate's variant it cost a tenth (968 -> 1,064 us at 129,000 points x
-// 49x72); in plain FP32 the store costs k_rates more than k_integrate saves
+// surrogate's variant it cost a tenth (865 -> 959 us at 127,587 points x
+// 49x72, k_rates 593 -> 574); in plain FP32 the store costs k_rates more than k_integrate saves
 // (256 + 427 against 301 + 415 us at 179,776 points).
 template <typename T, bool SUR>
 constexpr bool kStoredPrefix = sizeof(T) == 8 || SUR;
@@ -508,16 +510,16 @@ __global__ __launch_bounds__(512, (kWaves<T, DMAX, PAIR, SUR>)) void k_rates(con
                                                const BlockTask* __restrict__ tasks, int first,
                                                int rot_all, int ng, int chunks) {
   extern __shared__ double smem[];
-  stage_fm64<T>();
   const BlockTask tk = tasks[blockIdx.x];
   const DomainDev<T>& d = doms[tk.dom];
+  Scalars* sc = d.sc;
+  if (sc->done) return;  // uniform over a domain's workgroups: k_integrate has run ahead
+  stage_fm64<T>();
   // rotation tendency on the first substep of the launch (rot_all) and on
   // every substep of a domain with currents (src/umwm_advection.F90:117,
   // currents .or. first): the choice is per domain, so that batch members
   // with and without currents each follow the reference
   const bool rotation = rot_all || d.currents;
-  Scalars* sc = d.sc;
-  if (sc->done) return;  // uniform over the launch: k_integrate has run ahead
   const int W = blockDim.x >> 6, lane = threadIdx.x & 63, w = wave_id();
   const int j = tk.i0 + lane;
   const bool active = sc->sumt < d.dtg;
@@ -1484,8 +1486,7 @@ struct DirSums {
   }
 };
 
-// Stores the moments of (o, j), and the stress partials and (FP32) the
-// frequency's share of the wave height, e dk, as planes of sp.
+// Stores the moments of (o, j).
 template <typename T>
 __device__ __forceinline__ void store_mom(const DomainDev<T>& d, int o, int j, double m0, double mc,
                                           double ms) {
@@ -1890,7 +1891,7 @@ void launch_rates(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, 
   // a launch whose waves all hold D directions takes a variant with no
   // per-slot masks
   if (h.ng1 * D == pm) {
-    if constexpr (D % 2 == 0) {
+    if constexpr (D % 2 == 0 && D > 4) {  // 2 and 4 are choose_shape's, unpaired
       if (h.paired) {
         hipLaunchKernelGGL((k_rates<T, D, true, true, SUR>), grid, block, sh, s, doms, tasks, first,
                            rotation, h.ng1, h.c1);
