@@ -1486,23 +1486,15 @@ struct DirSums {
   }
 };
 
-// Stores the moments of (o, j).  FP32 grids too large for the split stream
-// them past the L2s as they do the spectrum: left there, k_rates paid for their
-// write-back (277 -> 255 us at 179,813 points x 37x36, k_advect 695 -> 699).
-template <bool STREAM, typename T>
+// Stores the moments of (o, j).
+template <typename T>
 __device__ __forceinline__ void store_mom(const DomainDev<T>& d, int o, int j, double m0, double mc,
                                           double ms) {
   const rsrc_t r = row_rsrc(d.mom, (size_t)o, 3 * (size_t)d.ldi);
   const uint32_t v = (uint32_t)j * 8u, pl = (uint32_t)d.ldi * 8u;
-  if constexpr (STREAM) {
-    bst_stream(r, v, m0);
-    bst_stream(r, v, mc, pl);
-    bst_stream(r, v, ms, 2 * pl);
-  } else {
-    bst(r, v, m0);
-    bst(r, v, mc, pl);
-    bst(r, v, ms, 2 * pl);
-  }
+  bst(r, v, m0);
+  bst(r, v, mc, pl);
+  bst(r, v, ms, 2 * pl);
 }
 
 // The moments of the current spectrum, after anything but k_advect wrote it;
@@ -1538,7 +1530,7 @@ __global__ __launch_bounds__(64) void k_moments(const DomainDev<T>* __restrict__
     }
   }
   S.group();
-  if (j < d.im) store_mom<false>(d, o, j, S.t[0], S.t[1], S.t[2]);
+  if (j < d.im) store_mom(d, o, j, S.t[0], S.t[1], S.t[2]);
 }
 
 // SPLIT: one workgroup per (frequency, 64 sea points), a wave per direction
@@ -1782,7 +1774,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_advect(
       tx = T(S.t[3]);
       ty = T(S.t[4]);
     }
-    store_mom<sizeof(T) == 4 && !SPLIT>(d, o, j, S.t[0], S.t[1], S.t[2]);
+    store_mom(d, o, j, S.t[0], S.t[1], S.t[2]);
     const rsrc_t sp = freq_rsrc(d.sp, o, kPartials<T>, ldi);
     bst(sp, vj, tx * icp);
     bst(sp, vj, ty * icp, rb);
