@@ -43,7 +43,7 @@ constexpr int BK = 32;  // K tile of the inference GEMM
 // its way into LDS took a 2-byte store per value.
 //
 // One training step of 2048 rows through 1335-512-512-512-1332 took 790 us
-// (GEMMs 430 of them), now 175 us of kernels (138).
+// (GEMMs 430 of them), now 179 us of kernels (138).
 constexpr int TT = 64;             // block of C and K tile
 constexpr int LMK = TT + 8, LKM = TT + 32;
 
