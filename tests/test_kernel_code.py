@@ -86,10 +86,10 @@ def lane_loops(path, symbol):
 
 
 @pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no llvm-objdump")
-@pytest.mark.parametrize("kernel", ["k_rates<float, 9, true, false, true>",
-                                    "k_rates<float, 18, true, true, true>",
-                                    "k_rates<float, 9, true, false, false>",
-                                    "k_rates<double, 9, true, false, false>",
+@pytest.mark.parametrize("kernel", ["k_rates<float, 9, true, false, true, true>",
+                                    "k_rates<float, 18, true, true, true, true>",
+                                    "k_rates<float, 9, true, false, false, false>",
+                                    "k_rates<double, 9, true, false, false, true>",
                                     "k_integrate<float, 9, true, true, false>",
                                     "k_integrate<float, 9, true, false, true>",
                                     "k_integrate<double, 9, true, false, false>"])
@@ -99,10 +99,10 @@ def test_scalar_descriptors(sweeps, kernel):
 
 
 # registers of a wave on a SIMD's 512, in steps of 8
-WAVES = {"k_rates<float, 9, true, false, true>": 3, "k_rates<float, 9, false, false, true>": 3,
-         "k_rates<float, 9, true, false, false>": 4, "k_rates<float, 36, true, true, false>": 3,
+WAVES = {"k_rates<float, 9, true, false, true, true>": 3, "k_rates<float, 9, false, false, true, true>": 3,
+         "k_rates<float, 9, true, false, false, false>": 4, "k_rates<float, 36, true, true, false, false>": 3,
          "k_integrate<float, 9, true, true, false>": 3, "k_integrate<float, 12, true, false, false>": 3,
-         "k_integrate<float, 9, true, false, true>": 3, "k_rates<double, 9, true, false, false>": 2}
+         "k_integrate<float, 9, true, false, true>": 3, "k_rates<double, 9, true, false, false, true>": 2}
 
 
 @pytest.mark.parametrize("kernel", WAVES)

@@ -452,13 +452,19 @@ struct Prefix {
   }
 };
 
-// Whether k_rates leaves the prefix for k_integrate or k_integrate sums it
-// again: in FP64 that spilled (155 -> 350 us at 2,852 points) and in the
-// surrogate's variant it cost a tenth (865 -> 959 us at 127,587 points x
-// 49x72, k_rates 593 -> 574); in plain FP32 the store costs k_rates more than k_integrate saves
-// (256 + 427 against 301 + 415 us at 179,776 points).
+// Whether k_rates leaves the prefix for k_integrate or k_integrate, with D
+// directions a wave, sums it again: in FP64 that spilled (155 -> 350 us at 2,852
+// points), in the surrogate's variant it cost a tenth (865 -> 959 us at 127,587
+// points x 49x72, k_rates 593 -> 574), and FP32 waves of twelve lost a wave per
+// SIMD to it (426 -> 519 us at 179,813 points x 37x36, 636 -> 786 at 93,870 x
+// 49x72, k_rates 219 -> 189 and 270 -> 242).  In plain FP32 with other widths
+// the store costs k_rates more than k_integrate saves (nine: 256 + 427 against
+// 301 + 415 us at 179,776 points; eighteen: 206 + 601 against 243 + 576 at
+// 93,870 x 49x72).
 template <typename T, bool SUR>
-constexpr bool kStoredPrefix = sizeof(T) == 8 || SUR;
+constexpr bool stored_prefix(int D) {
+  return sizeof(T) == 8 || SUR || D == 12;
+}
 
 // k^3 dk of (o, j): FP64 reads the table, FP32 forms it from k as the sweeps
 // do (TabGen).
@@ -505,7 +511,7 @@ constexpr double kSpecMargin = 1.05, kSpecSlack = 1.01;
 template <typename T, int DMAX, bool PAIR, bool SUR>
 constexpr int kWaves = sizeof(T) == 4 && ((SUR && DMAX == 9) || (!SUR && PAIR && DMAX == 36)) ? 3 : 2;
 
-template <typename T, int DMAX, bool FULL, bool PAIR, bool SUR>
+template <typename T, int DMAX, bool FULL, bool PAIR, bool SUR, bool STORE>
 __global__ __launch_bounds__(512, (kWaves<T, DMAX, PAIR, SUR>)) void k_rates(const DomainDev<T>* __restrict__ doms,
                                                const BlockTask* __restrict__ tasks, int first,
                                                int rot_all, int ng, int chunks) {
@@ -675,7 +681,7 @@ __global__ __launch_bounds__(512, (kWaves<T, DMAX, PAIR, SUR>)) void k_rates(con
     // a divergent branch here moves what it shares with the loads of the
     // moments, their descriptors, to vector registers)
     auto store_prefix = [&](int o, T pa0, T pac, T pas) {
-      if constexpr (kStoredPrefix<T, SUR>) {
+      if constexpr (STORE) {
         if (grp == 0) {
           const rsrc_t pf = freq_rsrc(pfxb, o, 3, ldi);
           const uint32_t v = valid ? vj : kDropOffset;
@@ -839,7 +845,7 @@ __global__ __launch_bounds__(512, (kWaves<T, DMAX, PAIR, SUR>)) void k_rates(con
       }
       if constexpr (kDerive) tg.advance(o, knext);
     }
-    if constexpr (kStoredPrefix<T, SUR>) {
+    if constexpr (STORE) {
       // the prefix of the diagnostic tail's bins, for k_integrate
       if (grp == 0) {
 #pragma unroll 4
@@ -1026,10 +1032,8 @@ __global__ __launch_bounds__(512, (kWaves<T, DMAX, PAIR, SUR>)) void k_rates(con
 // The price of a wrong guess is this kernel's time, so one is made only after a
 // substep whose time scales were a twentieth above the limit (kSpecMargin).
 // All waves of a point are in one workgroup here (one chunk, gridDim.y = 1).
-// Twelve directions in FP32 load the moments late and are bounded to three
-// waves a SIMD as in k_rates: 519 -> 461 us at 179,813 points x 37x36.
 template <typename T, int DMAX, bool FULL, bool SUR, bool SPEC>
-__global__ __launch_bounds__(512, (sizeof(T) == 4 && !SUR && DMAX == 12 ? 3 : 2)) void k_integrate(const DomainDev<T>* __restrict__ doms,
+__global__ __launch_bounds__(512) void k_integrate(const DomainDev<T>* __restrict__ doms,
                                                    const BlockTask* __restrict__ tasks, int ng,
                                                    int chunks) {
   const BlockTask tk = tasks[blockIdx.x];
@@ -1069,7 +1073,7 @@ __global__ __launch_bounds__(512, (sizeof(T) == 4 && !SUR && DMAX == 12 ? 3 : 2)
   const T* const eb = d.e;
   T* const esb = d.es;
   const T* const ftab = d.ftab;
-  constexpr bool kStored = kStoredPrefix<T, SUR>, kRegDirs = sizeof(T) == 4;
+  constexpr bool kStored = stored_prefix<T, SUR>(DMAX), kRegDirs = sizeof(T) == 4;
   [[maybe_unused]] const double* const momb = d.mom;
   [[maybe_unused]] const T* const pfxb = d.pfx;
   const T* const fr = d.f;
@@ -1156,11 +1160,10 @@ __global__ __launch_bounds__(512, (sizeof(T) == 4 && !SUR && DMAX == 12 ? 3 : 2)
   // the moments it is summed from
   [[maybe_unused]] Mom<T> pc{};
   [[maybe_unused]] Prefix P;
-  [[maybe_unused]] constexpr bool kAhead = DMAX != 12;  // see kWaves
   [[maybe_unused]] Mom<double> mo{};
   if constexpr (!kStored) {
     P = prefix_at(d, tg, o0, j, vj);
-    if constexpr (kAhead) mo = load_mom(momb, ldi, o0, j);
+    mo = load_mom(momb, ldi, o0, j);
   } else if constexpr (kDerive) {
     pc = load_mom(pfxb, ldi, o0, j);
   }
@@ -1187,7 +1190,7 @@ __global__ __launch_bounds__(512, (sizeof(T) == 4 && !SUR && DMAX == 12 ? 3 : 2)
       if constexpr (kStored)
         pn = load_mom(pfxb, ldi, on, j);
       else
-        mn = load_mom(momb, ldi, kAhead ? on : o, j);
+        mn = load_mom(momb, ldi, on, j);
       tg.table(o, tc);
     } else {
       load_tab<kSweepSlots>(ftab, ldi, o, vr, tc);
@@ -1360,7 +1363,7 @@ __global__ __launch_bounds__(512, (sizeof(T) == 4 && !SUR && DMAX == 12 ? 3 : 2)
     }
     if constexpr (!kStored) {
       const double k3 = k * k * tc[FT_KDK];  // k^3 dk
-      P.add(k3, kAhead ? mo : mn);
+      P.add(k3, mo);
       mo = mn;
     }
     if constexpr (kDerive) {
@@ -1881,29 +1884,32 @@ struct Shape {
   bool spec;    // k_integrate runs ahead of k_rates where the domains expect it
 };
 
-template <typename T, int D, bool SUR>
+template <typename T, int D, bool SUR, bool STORE>
 void launch_rates(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, int pm, int first,
                   int rotation, const Shape& h, hipStream_t s) {
-  const int slots = h.ng1 * h.c1;
-  const dim3 grid(ntasks, (slots + h.w1 - 1) / h.w1), block(64 * h.w1);
-  // the cross-wave maximum, and the surrogate's four cross-wave sums
-  const size_t sh = (size_t)(SUR ? 4 : 1) * h.w1 * 64 * sizeof(double);
-  // a launch whose waves all hold D directions takes a variant with no
-  // per-slot masks
-  if (h.ng1 * D == pm) {
-    if constexpr (D % 2 == 0 && D > 4) {  // 2 and 4 are choose_shape's, unpaired
-      if (h.paired) {
-        hipLaunchKernelGGL((k_rates<T, D, true, true, SUR>), grid, block, sh, s, doms, tasks, first,
-                           rotation, h.ng1, h.c1);
-        return;
+  // choose_shape's waves of 2 and 4 have a k_integrate as narrow
+  if constexpr (sizeof(T) == 8 || D > 4 || !STORE) {
+    const int slots = h.ng1 * h.c1;
+    const dim3 grid(ntasks, (slots + h.w1 - 1) / h.w1), block(64 * h.w1);
+    // the cross-wave maximum, and the surrogate's four cross-wave sums
+    const size_t sh = (size_t)(SUR ? 4 : 1) * h.w1 * 64 * sizeof(double);
+    // a launch whose waves all hold D directions takes a variant with no
+    // per-slot masks
+    if (h.ng1 * D == pm) {
+      if constexpr (D % 2 == 0 && D > 4) {  // 2 and 4 are unpaired
+        if (h.paired) {
+          hipLaunchKernelGGL((k_rates<T, D, true, true, SUR, STORE>), grid, block, sh, s, doms, tasks,
+                             first, rotation, h.ng1, h.c1);
+          return;
+        }
       }
+      if constexpr (!(SUR && D % 2 == 0))
+        hipLaunchKernelGGL((k_rates<T, D, true, false, SUR, STORE>), grid, block, sh, s, doms, tasks,
+                           first, rotation, h.ng1, h.c1);
+    } else if constexpr (D > 4) {
+      hipLaunchKernelGGL((k_rates<T, D, false, false, SUR, STORE>), grid, block, sh, s, doms, tasks,
+                         first, rotation, h.ng1, h.c1);
     }
-    if constexpr (!(SUR && D % 2 == 0))
-      hipLaunchKernelGGL((k_rates<T, D, true, false, SUR>), grid, block, sh, s, doms, tasks, first,
-                         rotation, h.ng1, h.c1);
-  } else if constexpr (D > 4) {
-    hipLaunchKernelGGL((k_rates<T, D, false, false, SUR>), grid, block, sh, s, doms, tasks, first,
-                       rotation, h.ng1, h.c1);
   }
 }
 
@@ -1922,7 +1928,7 @@ template <typename T>
 void launch_spec(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks, int pm,
                  const Shape& h, hipStream_t s) {
   const dim3 grid(ntasks), block(64 * h.w2);
-  if constexpr (kStoredPrefix<T, false>)
+  if constexpr (stored_prefix<T, false>(9))
     hipLaunchKernelGGL((k_prefix<T>), grid, dim3(64), 0, s, doms, tasks);
   if (h.ng2 * h.D2 != pm) {  // FP32 waves of nine, see choose_shape
     if constexpr (sizeof(T) == 4)
@@ -1953,7 +1959,12 @@ int launch_kernels(const DomainDev<T>* doms, const BlockTask* tasks, int ntasks,
     if (h.spec && !first && !rotation && !ev) launch_spec<T>(doms, tasks, ntasks, pm, h, s);
   }
 #define UMWM_RATES(D_)                                                                       \
-  case D_: launch_rates<T, D_, SUR>(doms, tasks, ntasks, pm, first, rotation, h, s); break;
+  case D_:                                                                                   \
+    if (stored_prefix<T, SUR>(h.D2))                                                         \
+      launch_rates<T, D_, SUR, true>(doms, tasks, ntasks, pm, first, rotation, h, s);        \
+    else if constexpr (!stored_prefix<T, SUR>(0))                                            \
+      launch_rates<T, D_, SUR, false>(doms, tasks, ntasks, pm, first, rotation, h, s);       \
+    break;
   switch (h.D1) {
     UMWM_RATES(6)
     UMWM_RATES(9)
