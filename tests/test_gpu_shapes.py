@@ -323,3 +323,29 @@ def test_autotune_keeps_the_default_where_it_is_faster():
         assert choice == d.tile() == autotune.default_tile(36) and len(table) == 4
     finally:
         d.close()
+
+
+@pytest.mark.parametrize("grid", [(270, 250, 6, 36), (190, 180, 7, 72)])
+def test_rates_of_eighteen_directions(grid):
+    """FP32 grids large enough for k_rates to take eighteen directions a wave,
+    where the sources set the substep: the bits of nine."""
+    mm, nm, om, pm = grid
+    wl = configs.tiny(4, mm, nm, om, pm, land=False, winds=True, wspd=18.0)
+    wl.params.delx = wl.params.dely = 2e5
+    a, b = (hip.Domain(wl.params, wl.grid_input(), wl.forcing_input(0), precision=4)
+            for _ in range(2))
+    try:
+        assert (a.im + 63) // 64 * (pm // 9) >= 4096
+        b.set_tile(9, pm // 9, 18, pm // 18, 2)
+        for d in (a, b):
+            d.init_jonswap(wl.jonswap)
+            d.stokes_drift(True)
+            d.forcinginput(wl.forcing_input(1))
+        for _ in range(4):
+            assert a.substep() == b.substep()
+        assert 0 < a.scalar("dts") < a.scalar("dtamin") and a.scalar("substeps_ahead") == 0
+        for name in ("physics_time_step", "e", "ustar"):
+            assert np.array_equal(a.get(name), b.get(name)), name
+    finally:
+        a.close()
+        b.close()

@@ -2066,7 +2066,10 @@ int waves_for(int slots) {
 // At 38,936 points the count of waves decides (37x28 339 and 312, 37x44 472 and
 // 513, 37x64 601 and 626, 37x68 680 and 643).  FP64, whose directions weigh
 // more, keeps four: 867 us against 914 at 38,936 points x 37x28, 1,557 against
-// 1,549 at 79,921.
+// 1,549 at 79,921.  On FP32 grids as large k_rates alone takes eighteen where
+// they divide pm: substeps whose sources limit them 1,433 -> 1,399 us at
+// 179,813 points x 37x36 (k_rates 283 -> 250), 1,751 -> 1,746 at 93,870 x 49x72;
+// no gain at 38,844 (55 -> 58 of 333).
 // k_advect's split pays while its waves (one per frequency and point block)
 // leave the GPU short of work: 2,809 points FP64 29.7 -> 25.7, FP32 25.6 ->
 // 19.2 us; 11,449 points 84.9 -> 92.9 and 39.4 -> 49.1 us.
@@ -2098,6 +2101,10 @@ Shape choose_shape(const Tile& t, int ntasks, int omax, bool sur, bool fp32) {
   h.c1 = h.c2 = chunks(D);
   h.w1 = h.w2 = waves_for(h.ng1 * h.c1);
   h.paired = false;  // one order of operations whatever D
+  if (fp32 && pm % 18 == 0 && h.c1 == 1 && ntasks * (pm / 9) >= kFullWaves) {
+    h.D1 = 18;
+    h.ng1 = h.w1 = pm / 18;
+  }
   h.split = ntasks * omax < kAdvectWaves;
   h.spec = h.D2 >= 4 && h.c2 == 1 && h.w2 == h.ng2;  // launch_spec has D = 4, 6 and 9
   return h;
