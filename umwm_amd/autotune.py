@@ -79,18 +79,25 @@ def autotune(dom, steps=3, verbose=None):
     best1 = min(c1, key=lambda a: min(t[0] for x, _, _, t in table if x == a))
     best2 = min(c2, key=lambda b: min(t[1] for _, y, _, t in table if y == b))
     best3 = min(ADVECT_NB, key=lambda nb: min(t[2] for _, _, z, t in table if z == nb))
-    choice, default = (best1[0], best1[1], best2[0], best2[1], best3), default_tile(pm)
-    if choice != default:
-        # in turn, the faster of two passes each; the default where it is
-        # clearly faster, or nothing could be timed (two that run their sources
-        # ahead differ only in the kernels that then do not run)
-        t = [(substep_time(dom, choice, steps), substep_time(dom, default, steps))
-             for _ in range(2)]
-        t = [(a, b) for a, b in t if a and b]
-        if not t or min(b for _, b in t) < 0.97 * min(a for a, _ in t):
-            choice = default
+    # whole substeps of the kernels' choice, of the same with the default's
+    # k_integrate, and of the default: in turn, the faster of two passes each.
+    # A later one has to be clearly faster: two that run their sources ahead
+    # differ only in kernels that then do not run.  The default where nothing
+    # could be timed.
+    default = default_tile(pm)
+    tiles = list(dict.fromkeys([best1 + best2 + (best3,), best1 + default[2:4] + (best3,), default]))
+    times = [[substep_time(dom, x, steps) for x in tiles] for _ in range(2)]
+    if all(t for row in times for t in row):
+        best = [min(row[k] for row in times) for k in range(len(tiles))]
+        k = 0
+        for q in range(1, len(tiles)):
+            if best[q] < 0.97 * best[k]:
+                k = q
+        choice = tiles[k]
         if verbose:
-            verbose(f"autotune: substeps {t} s, {choice}")
+            verbose(f"autotune: substeps {dict(zip(tiles, best))} s, {choice}")
+    else:
+        choice = default
     dom.set_tile(*choice)
     return choice, table
 
